@@ -359,8 +359,12 @@ int  qss_unpack_layer_record(qss_ctx *c, const double *src, size_t n);
  * least 256).  Where ny and nz are multiples of 128 (at most 1024) the
  * twiddles run inside the two GEMMs; elsewhere in twiddle kernels between
  * them.  Contexts start FACTORED where the twiddles run inside the GEMMs
- * (measured faster at 256^2, 384^2 and 512^2) and DENSE otherwise.  Results
- * agree to rounding.  Setting a method drops a captured graph.              */
+ * (measured faster at 256^2, 384^2 and 512^2) and DENSE otherwise.  FP64
+ * contexts whose axes allow it run O(N log N) line transforms instead of
+ * either GEMM form until a method is set here or a tile shape is forced
+ * (qss_set_gemm_variant); qss_transform_method names the GEMM form all the
+ * while.  Results agree to rounding.  Setting a method drops a captured
+ * graph.                                                                     */
 #define QSS_TRANSFORM_DENSE    0
 #define QSS_TRANSFORM_FACTORED 1
 int  qss_set_transform_method(qss_ctx *c, int method);

@@ -27,13 +27,16 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}",
           "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
           "-Wno-unused-command-line-argument"]
 NO_CONTRACT = {"particles.hip", "push_tile.hip", "beam.hip", "spectral.hip", "adjoint.hip",
-               "driver.hip"}
+               "driver.hip", "line.hip"}
 # MFMA accumulators in VGPRs: with AGPR accumulators the compiler copies
 # every loop-carried accumulator AGPR->VGPR->AGPR at the K-loop back-edge,
 # draining the MFMA pipeline once per iteration
 MFMA_VGPR = {"gemm.hip", "fact_fused.hip"}
+# literals stay where they are used: hoisted out of the pass loops of every
+# radix they would fill the scalar registers and spill
+NO_MACHINE_LICM = {"line.hip"}
 SOURCES = ["gemm.hip", "spectral.hip", "beam.hip", "particles.hip", "push_tile.hip",
-           "adjoint.hip", "driver.hip", "noalloc.hip", "fact.hip", "fact_fused.hip", "qss_api.cpp",
+           "adjoint.hip", "driver.hip", "noalloc.hip", "line.hip", "fact.hip", "fact_fused.hip", "qss_api.cpp",
            "h5file.cpp", "save.cpp"]
 
 
@@ -44,6 +47,8 @@ def _compile(src: str) -> str:
         flags.append("-ffp-contract=off")
     if src in MFMA_VGPR:
         flags += ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
+    if src in NO_MACHINE_LICM:
+        flags += ["-mllvm", "-disable-machine-licm"]
     if src.endswith(".cpp"):
         flags = ["-x", "hip"] + flags
     cmd = [HIPCC] + flags + ["-c", os.path.join(CSRC, src), "-o", obj]

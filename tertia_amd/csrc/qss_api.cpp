@@ -254,6 +254,90 @@ int transform_fact(qss_ctx *c, int n, const int *kz, const int *ky, const double
   return QSS_OK;
 }
 
+// ---- line transforms (line.hip) ----------------------------------------------
+// flops of a transform along one axis of every plane, as a fast transform's
+// 2.5 n log2 n per line (the dense table's 2 n^2 where that is what runs)
+double line_flops(const LineAxis &ax, double cells) {
+  return cells * (ax.np ? 2.5 * std::log2((double)ax.n) : 2.0 * ax.n);
+}
+
+bool use_lines(const qss_ctx *c) { return c->line_use && c->gemm_force < 0; }
+
+// transforms along z with the corrector's epilogue; store[b] = 0: the result
+// is not kept, only its push field
+int line_cols(qss_ctx *c, int n, const int *kz, const double *const *in, double *const *out,
+              double alpha, const int *resid = nullptr, const int *push = nullptr,
+              const double *const *pplane = nullptr, double beta = 0.0, bool one_wake = false,
+              const int *store = nullptr) {
+  ColArgs a{};
+  a.ax = c->line[1];
+  a.ny = c->ny; a.nbatch = n; a.nw = one_wake ? 1 : c->nw;
+  a.nc = c->ncell;
+  a.alpha = alpha; a.beta = beta;
+  a.F = c->F; a.w_f = c->ncell * kPushComp; a.rslots = c->d_resid;
+  for (int b = 0; b < n; ++b) {
+    a.in[b] = in[b]; a.out[b] = out[b]; a.kz[b] = kz[b];
+    a.P[b] = pplane ? pplane[b] : nullptr;
+    a.resid[b] = resid ? resid[b] : -1;
+    a.push[b] = push ? push[b] : -1;
+    a.store[b] = store ? store[b] : 1;
+  }
+  Timed t(c, KC_GEMM, true);
+  HIPCHECK(launch_line_cols(a, c->stream, t.e0, t.e1));
+  if (c->timing) c->gemm_flops += line_flops(a.ax, (double)c->ncell * n * a.nw);
+  return QSS_OK;
+}
+
+// transform_batch: y pass in -> tmp, z pass tmp -> out
+int transform_line(qss_ctx *c, int n, const int *kz, const int *ky, const double *const *in,
+                   double *const *out, double alpha, const int *resid, const int *push,
+                   const double *const *pplane, double beta, bool one_wake) {
+  if (!resid && !push && beta == 0.0 && line_plane_ok(c->line[0], c->line[1])) {
+    SmallPlaneArgs a{};
+    a.y = c->line[0]; a.z = c->line[1];
+    a.nbatch = n; a.nw = one_wake ? 1 : c->nw; a.nc = c->ncell; a.alpha = alpha;
+    for (int b = 0; b < n; ++b) {
+      a.in[b] = in[b]; a.out[b] = out[b]; a.ky[b] = ky[b]; a.kz[b] = kz[b];
+    }
+    Timed t(c, KC_GEMM, true);
+    HIPCHECK(launch_line_plane(a, c->stream, t.e0, t.e1));
+    if (c->timing)
+      c->gemm_flops += line_flops(a.y, (double)c->ncell * n * a.nw) +
+                       line_flops(a.z, (double)c->ncell * n * a.nw);
+    return QSS_OK;
+  }
+  RowArgs r{};
+  r.ax = c->line[0];
+  r.nz = c->nz; r.nbatch = n; r.nw = one_wake ? 1 : c->nw;
+  r.nc = c->ncell;
+  for (int b = 0; b < n; ++b) { r.in[b] = in[b]; r.out[b] = c->tmp[b]; r.ky[b] = ky[b]; }
+  {
+    Timed t(c, KC_GEMM, true);
+    HIPCHECK(launch_line_rows(r, c->stream, t.e0, t.e1));
+  }
+  if (c->timing) c->gemm_flops += line_flops(r.ax, (double)c->ncell * n * r.nw);
+  return line_cols(c, n, kz, c->tmp, out, alpha, resid, push, pplane, beta, one_wake);
+}
+
+// one row kernel: forward along y of the nin z-transformed sources in tmp, the
+// per-mode map, inverse along y of its results back into tmp
+int line_modes(qss_ctx *c, bool guess, bool all, bool fin, bool psi, bool clear_resid) {
+  ModeArgs a{};
+  a.ax = c->line[0];
+  a.nz = c->nz; a.nw = c->nw; a.nc = c->ncell;
+  for (int b = 0; b < (guess ? 2 : 3); ++b) a.in[b] = c->tmp[b];
+  // a work-group reads and writes its own row of the planes alone, and has
+  // read it whole before it writes
+  for (int b = 0; b < (psi ? 8 : 6); ++b) a.out[b] = c->tmp[b];
+  for (int s = 0; s < SP_N; ++s) a.S[s] = c->S[s];
+  a.ly = c->p.ly; a.lz = c->p.lz; a.hx = c->hxs; a.dens = c->p.dens;
+  a.all = all; a.fin = fin; a.psi = psi;
+  a.rslots = clear_resid ? c->d_resid : nullptr;
+  Timed t(c, KC_SPEC, true);
+  HIPCHECK(launch_line_modes(a, guess, c->stream, t.e0, t.e1));
+  return QSS_OK;
+}
+
 // out_b = alpha * T_kz[b] . in_b . T_ky[b]: y-pass into tmp, then z-pass
 // reuse: the split-bf16 operands may come from the producer of the inputs
 // (c->xs_src records which planes xs holds); false for caller-owned planes
@@ -265,6 +349,8 @@ int transform_batch(qss_ctx *c, int n, const int *kz, const int *ky,
     qss_set_error("transform batch size");
     return QSS_E_ARG;
   }
+  if (use_lines(c) && c->line_plain)
+    return transform_line(c, n, kz, ky, in, out, alpha, resid, push, pplane, beta, one_wake);
   if (c->fact_use && !c->npc && !c->mixed)
     return transform_fact(c, n, kz, ky, in, out, alpha, resid, push, pplane, beta, one_wake);
   GemmArgs g{};
@@ -348,7 +434,20 @@ int do_beam(qss_ctx *c, int slice, int isplit) {
   return QSS_OK;
 }
 
-int do_guess(qss_ctx *c, int first) {
+int line_fields(qss_ctx *c, bool psi, bool resid, bool keep_e, bool keep_b, bool fin);
+
+// kinds of Ex, Ey, Ez, Bx, By, Bz, rho, psi along z (y)
+constexpr int kOutKz[8] = {QSS_KIND_C, QSS_KIND_C, QSS_KIND_S, QSS_KIND_S, QSS_KIND_S, QSS_KIND_C,
+                           QSS_KIND_C, QSS_KIND_C};
+constexpr int kOutKy[8] = {QSS_KIND_C, QSS_KIND_S, QSS_KIND_C, QSS_KIND_S, QSS_KIND_C, QSS_KIND_S,
+                           QSS_KIND_C, QSS_KIND_C};
+
+// in_step: inside a layer step only what a later pass of the step reads is
+// written: the spectra that the final pass rewrites, and the C planes of E and
+// B that only the push field is made from, are left out.
+// keep_e: C-layer E kept all the same (the next Iterate is the final one,
+// whose residual compares with it)
+int do_guess(qss_ctx *c, int first, bool in_step = false, bool keep_e = true) {
   if (first) {
     // The reference zeroes every spectrum at the first layer (:479-494) but
     // then re-transforms the P layer, so only the beam spectrum (which
@@ -362,6 +461,18 @@ int do_guess(qss_ctx *c, int first) {
   // beam P spectrum = previous beam spectrum (:637-646): swap buffers
   std::swap(c->S[SP_RHOBP], c->S[SP_RHOB]);
   std::swap(c->S[SP_JXBP], c->S[SP_JXB]);
+  if (use_lines(c)) {
+    // the spectra of the finished layer become the P spectra by trading places
+    // (the other transforms' Guess kernel copies them)
+    const int now[7] = {SP_RHO, SP_JX, SP_JY, SP_JZ, SP_EX, SP_EY, SP_EZ};
+    const int prev[7] = {SP_RHOP, SP_JXP, SP_JYP, SP_JZP, SP_EXP, SP_EYP, SP_EZP};
+    for (int q = 0; q < 7; ++q) std::swap(c->S[now[q]], c->S[prev[q]]);
+    const int kz[2] = {QSS_KIND_C, QSS_KIND_C};
+    const double *in[2] = {c->C[QSS_RHOBEAM], c->C[QSS_JXBEAM]};
+    CHECK(line_cols(c, 2, kz, in, c->tmp, 1.0));
+    CHECK(line_modes(c, true, !in_step, false, false, false));
+    return line_fields(c, false, false, !in_step || keep_e, !in_step, false);
+  }
   {
     const int kz[2] = {QSS_KIND_C, QSS_KIND_C}, ky[2] = {QSS_KIND_C, QSS_KIND_C};
     const double *in[2] = {c->C[QSS_RHOBEAM], c->C[QSS_JXBEAM]};
@@ -425,7 +536,40 @@ int do_push_deposit(qss_ctx *c, int full) {
   return QSS_OK;
 }
 
-int do_iterate(qss_ctx *c, int final_pass, double *res_dev) {
+// the inverse transforms along z that end a Guess or an Iterate: C-layer E, B
+// (kept or not), the push field unless it is the layer's final pass, rho and
+// psi with it
+int line_fields(qss_ctx *c, bool psi, bool resid, bool keep_e, bool keep_b, bool fin) {
+  double *out[8] = {c->C[QSS_EX], c->C[QSS_EY], c->C[QSS_EZ], c->C[QSS_BX],
+                    c->C[QSS_BY], c->C[QSS_BZ], c->C[QSS_RHO], c->C[QSS_PSI]};
+  const double *pp[8] = {c->P[QSS_EX], c->P[QSS_EY], c->P[QSS_EZ], c->P[QSS_BX],
+                         c->P[QSS_BY], c->P[QSS_BZ], nullptr, nullptr};
+  int rc[8], push[8], store[8];
+  for (int b = 0; b < 8; ++b) {
+    rc[b] = resid && b < 3 ? b : -1;
+    push[b] = !fin && b < 6 ? b : -1;   // after the final pass the next Guess rebuilds it
+    store[b] = b < 3 ? keep_e : b < 6 ? keep_b : 1;
+  }
+  return line_cols(c, psi ? 8 : 6, kOutKz, c->tmp, out, 1.0 / (4.0 * c->ny * c->nz), rc, push, pp,
+                   0.0, false, store);
+}
+
+// in_step, keep_e: as do_guess
+int do_iterate(qss_ctx *c, int final_pass, double *res_dev, bool in_step = false,
+               bool keep_e = true) {
+  if (use_lines(c)) {
+    const bool lean = in_step && !final_pass, psi = final_pass && !c->skip_rho_psi;
+    const int kz[3] = {QSS_KIND_C, QSS_KIND_C, QSS_KIND_S};
+    const double *in[3] = {c->C[QSS_JX], c->C[QSS_JY], c->C[QSS_JZ]};
+    CHECK(line_cols(c, 3, kz, in, c->tmp, 1.0));
+    CHECK(line_modes(c, false, !lean, final_pass, psi, !lean));
+    CHECK(line_fields(c, psi, !lean, !lean || keep_e, !lean, final_pass));
+    if (res_dev) {
+      Timed t(c, KC_SPEC);
+      HIPCHECK(launch_residual_final(c, res_dev));
+    }
+    return QSS_OK;
+  }
   {
     const int kz[3] = {QSS_KIND_C, QSS_KIND_C, QSS_KIND_S};
     const int ky[3] = {QSS_KIND_C, QSS_KIND_S, QSS_KIND_C};
@@ -563,15 +707,15 @@ int do_layer_step(qss_ctx *c, int slice, int isplit, double *res_dev, char *tape
   c->deposit_rho = false;
   CHECK(do_beam(c, slice, isplit));
   field_of(0);
-  CHECK(do_guess(c, slice == 0));
+  CHECK(do_guess(c, slice == 0, true, c->p.n_iter == 0));
   for (int it = 0; it < c->p.n_iter; ++it) {
     CHECK(do_push_deposit(c, 0));
     field_of(it + 1);
-    CHECK(do_iterate(c, 0, nullptr));
+    CHECK(do_iterate(c, 0, nullptr, true, it == c->p.n_iter - 1));
   }
   CHECK(do_push_deposit(c, 1));
   c->F = F0;   // the final corrector's push field is not replayed
-  CHECK(do_iterate(c, 1, res_dev));
+  CHECK(do_iterate(c, 1, res_dev, true));
   swap_c_p(c);
   return QSS_OK;
 }
@@ -1160,6 +1304,29 @@ int qss_create(const qss_params *p, int device, uint32_t history_mask, qss_ctx *
       c->fact_use = true;
     }
   }
+  // line transforms (line.hip)
+  c->line_plain = c->line_use = p->precision == QSS_PREC_FP64;
+  for (int i = 0; i < 2 && c->line_use; ++i) {
+    LineAxis &ax = c->line[i];
+    const bool fast = line_chain(i == 0 ? c->ny : c->nz, &ax);
+    ax.Tc = c->d_T[2 * i];
+    ax.Ts = c->d_T[2 * i + 1];
+    if (!fast) {
+      c->line_plain = false;
+      c->line_use = ax.n <= (i == 0 ? kLineDenseY : kLineDenseZ);
+      continue;
+    }
+    if (!line_fixed(ax) && ax.n < kLineLooseMin) c->line_plain = false;
+    std::vector<double> tw;
+    line_table(ax, tw);
+    if ((r = dalloc(&c->d_linetw[i], tw.size())) != QSS_OK) return fail(r);
+    ax.tw = c->d_linetw[i];
+    if (hipMemcpy(c->d_linetw[i], tw.data(), tw.size() * 8, hipMemcpyHostToDevice) !=
+        hipSuccess) {
+      qss_set_error("line transform table upload failed");
+      return fail(QSS_E_HIP);
+    }
+  }
   if ((r = dalloc(&c->F, ncw * kPushComp)) != QSS_OK) return fail(r);
   if (c->mixed && (r = dalloc(&c->Ff, ncw * kPushComp)) != QSS_OK) return fail(r);
   if (nw > 1) {
@@ -1266,6 +1433,7 @@ int qss_destroy(qss_ctx *c) {
   dfree(c->d_G[0]); dfree(c->d_G[1]); dfree(c->d_tw[0]); dfree(c->d_tw[1]);
   dfree(c->d_Gf[0]); dfree(c->d_Gf[1]); dfree(c->d_twf[0]); dfree(c->d_twf[1]);
   dfree(c->d_Gfd[0]); dfree(c->d_Gfd[1]);
+  dfree(c->d_linetw[0]); dfree(c->d_linetw[1]);
   dfree(c->F); dfree(c->Ff); dfree(c->d_bins); dfree(c->d_wbunch);
   for (auto &p : c->Ts) dfree(p);
   for (auto &p : c->xs) dfree(p);
@@ -1808,6 +1976,7 @@ int qss_set_transform_method(qss_ctx *c, int method) {
     return QSS_E_ARG;
   }
   graph_free(c);   // a captured graph holds the other method's launches
+  c->line_plain = c->line_use = false;   // a GEMM method was asked for
   c->fact_use = method == QSS_TRANSFORM_FACTORED;
   return QSS_OK;
 }

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "../../include/qss.h"
+#include "line_plan.h"
 
 // spectral state ids (fft_of_* arrays, movefieldshydrolinlayersplit.cpp:267-313)
 enum {
@@ -137,6 +138,77 @@ void fact_fused_matrix(int n, int pass, std::vector<double> &g);
 void fact_fused_twiddles(int n, std::vector<double> &tw);
 
 // ---------------------------------------------------------------------------
+// line transforms (tertia_amd/csrc/line.hip): the FP64 default.  An axis has a
+// fast form (a chain of passes of small radix) or the dense table applied line
+// by line (np = 0).  Transforms by themselves take lines where both axes are
+// fast and of a compile-time length or at least kLineLooseMin (3 planes of 200 x
+// 312 1.14 times the GEMMs' speed, 4 of 100 x 100 0.90); a layer step's Guess and Iterate, whose row kernel does the work of five
+// launches, also with a dense axis: along y up to 128 (a 121 x 97 sweep 1.07 times
+// the GEMMs' speed, 74 x 122 1.12, 129 x 129 0.86), along z up to 256 (64 x 161
+// 1.17)
+// ---------------------------------------------------------------------------
+constexpr int kLineDenseY = 128, kLineDenseZ = 256, kLineLooseMin = 192;
+// transforms along z of nbatch planes: out = alpha T_z in (+ beta out), with
+// the corrector epilogue
+struct ColArgs {
+  LineAxis ax;                       // z
+  int ny, nbatch, nw;
+  long nc;                           // wake stride of every plane
+  const double *in[kGemmMaxBatch];
+  double *out[kGemmMaxBatch];
+  const double *P[kGemmMaxBatch];    // P-layer planes (push field)
+  int kz[kGemmMaxBatch], resid[kGemmMaxBatch], push[kGemmMaxBatch];
+  int store[kGemmMaxBatch];          // 0: the result goes to the push field only
+  double alpha, beta;
+  double *F;
+  long w_f;
+  unsigned long long *rslots;
+};
+// transforms along y: out = in T_y
+struct RowArgs {
+  LineAxis ax;                       // y
+  int nz, nbatch, nw;
+  long nc;
+  const double *in[kGemmMaxBatch];
+  double *out[kGemmMaxBatch];
+  int ky[kGemmMaxBatch];
+};
+// both transforms of small planes: out = alpha T_z in T_y
+struct SmallPlaneArgs {
+  LineAxis y, z;
+  int nbatch, nw;
+  long nc;
+  const double *in[kGemmMaxBatch];
+  double *out[kGemmMaxBatch];
+  int ky[kGemmMaxBatch], kz[kGemmMaxBatch];
+  double alpha;
+};
+// rows of the z-transformed sources (beam rho, Jx or Jx, Jy, Jz): forward along
+// y, the Guess or Iterate map, inverse along y of Ex..Bz (rho, psi)
+struct ModeArgs {
+  LineAxis ax;                       // y
+  int nz, nw;
+  long nc;
+  const double *in[3];
+  double *out[kGemmMaxBatch];
+  double *S[SP_N];
+  double ly, lz, hx, dens;
+  bool all;                          // write every spectrum, not only what the next pass reads
+  bool fin;                          // Iterate: the final pass (psi's spectrum)
+  bool psi;                          // Iterate: rho and psi transformed too (8 outputs)
+  unsigned long long *rslots;        // Iterate: residual slots to clear (or null)
+};
+hipError_t launch_line_cols(const ColArgs &a, hipStream_t s, hipEvent_t ev0 = nullptr,
+                            hipEvent_t ev1 = nullptr);
+hipError_t launch_line_rows(const RowArgs &a, hipStream_t s, hipEvent_t ev0 = nullptr,
+                            hipEvent_t ev1 = nullptr);
+bool line_plane_ok(const LineAxis &y, const LineAxis &z);
+hipError_t launch_line_plane(const SmallPlaneArgs &a, hipStream_t s, hipEvent_t ev0 = nullptr,
+                             hipEvent_t ev1 = nullptr);
+hipError_t launch_line_modes(const ModeArgs &a, bool guess, hipStream_t s,
+                             hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+
+// ---------------------------------------------------------------------------
 // adjoint sweep (tertia_amd/csrc/adjoint.hip, qss_sweep_vjp)
 // ---------------------------------------------------------------------------
 struct AdjTileArgs {
@@ -237,6 +309,11 @@ struct qss_ctx {
   double2 *d_tw[2] = {};
   double *tmp2[kGemmMaxBatch] = {};
   int fact_var[2][kGemmMaxBatch + 1] = {};
+  // line transforms (line.hip), in use until a GEMM method or tile shape is
+  // asked for
+  bool line_plain = false, line_use = false;   // transforms by themselves; layer steps
+  LineAxis line[2];                  // y, z
+  double *d_linetw[2] = {};
   double *F = nullptr;               // push field
   float *Ff = nullptr;               // push field, fp32 (mixed modes)
   bool mixed = false;                // precision != QSS_PREC_FP64

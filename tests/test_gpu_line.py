@@ -1,0 +1,57 @@
+"""GPU: the line-transform kernels (line.hip) at the edges of their shapes: lengths
+compiled in (two and three passes), loose chains with and without a radix above 8,
+the dense table (odd lengths, prime factors above 13) on either axis, partial
+strips of columns, and planes small enough for one work-group.
+
+Transforms against the oracle at the transform tests' bound (1e-13 of the largest
+result); sweeps, which run the fused Guess and Iterate rows, against the oracle at
+the small sweeps' bound (rel-L2 1e-10)."""
+import numpy as np
+import pytest
+
+from tests.helpers import max_rel
+from tertia_amd.params import QSS_SHAPE_NGP_REF, small
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nz,ny", [(32, 40), (64, 48), (80, 96), (192, 160), (512, 320), (200, 312),
+                                   (242, 208), (484, 250), (512, 512)])
+def test_line_transform_vs_oracle(oracle_mod, nz, ny):
+    from tertia_amd.mesh import Mesh
+    m = Mesh(small(ny=ny, nz=nz, nslices=1), history=())
+    try:
+        x = np.random.default_rng(ny + 1000 * nz).standard_normal((nz, ny))
+        for kz in (0, 1):
+            for ky in (0, 1):
+                ref = oracle_mod.transform2d(x, kz, ky, use_fft=False, nthreads=4)
+                assert max_rel(m.transform2d(x, kz, ky, 0.25), 0.25 * ref) < 1e-13, (kz, ky)
+    finally:
+        m.close()
+
+
+@pytest.mark.parametrize("ny,nz,kw", [
+    (32, 32, {}), (48, 80, {}), (192, 64, {"n_iter": 0}), (320, 160, {}),   # compiled lengths
+    (36, 100, {}), (52, 66, {"n_iter": 1}),                                # loose chains
+    (33, 48, {}), (48, 35, {}), (121, 97, {"shape": QSS_SHAPE_NGP_REF}), (34, 74, {}),   # dense
+    (128, 256, {}), (17, 19, {})])
+def test_sweep_on_line_grids_vs_oracle(oracle_mod, ny, nz, kw):
+    from tertia_amd.mesh import Mesh
+    p = small(ny=ny, nz=nz, nslices=12, **kw)
+    fields = ("Ex", "Ey", "Ez", "By", "Psi")
+    m = Mesh(p, history=fields)
+    o = oracle_mod.Oracle(p, use_fft=False, nthreads=8, history=fields)
+    try:
+        rg = m.MoveAllSplitLayers()
+        st, ro = o.sweep()
+        assert st == 0
+        assert np.abs(rg - ro).max() < 1e-9
+        for f in fields:
+            G = np.stack([m.history(f, s) for s in range(p.nslices)])
+            R = np.stack([o.history(f, s) for s in range(p.nslices)])
+            e = float(np.linalg.norm(G - R) / np.linalg.norm(R))
+            print(ny, nz, f, "%.1e" % e, flush=True)
+            assert e <= 1e-10, (f, e)
+    finally:
+        m.close()
+        o.close()
