@@ -32,9 +32,9 @@ NO_CONTRACT = {"particles.hip", "push_tile.hip", "beam.hip", "spectral.hip", "ad
 # every loop-carried accumulator AGPR->VGPR->AGPR at the K-loop back-edge,
 # draining the MFMA pipeline once per iteration
 MFMA_VGPR = {"gemm.hip", "fact_fused.hip"}
-# literals stay where they are used: hoisted out of the pass loops of every
-# radix they would fill the scalar registers and spill
-NO_MACHINE_LICM = {"line.hip"}
+# literals stay where they are used: hoisted out of the loops (the line kernels'
+# passes of every radix, the push's chunks) they would fill the registers and spill
+NO_MACHINE_LICM = {"line.hip", "push_tile.hip"}
 SOURCES = ["gemm.hip", "spectral.hip", "beam.hip", "particles.hip", "push_tile.hip",
            "adjoint.hip", "driver.hip", "noalloc.hip", "line.hip", "fact.hip", "fact_fused.hip", "qss_api.cpp",
            "h5file.cpp", "save.cpp"]

@@ -9,12 +9,14 @@
 //      never leave the CU;
 //   2. each thread pushes one particle per chunk of 256 (same arithmetic as
 //      the reference, -ffp-contract=off);
-//   3. every deposit event (one per sub-step, :1391-1466) is keyed by its
-//      window cell; the chunk's keys are bitonic-sorted in LDS (register
-//      shuffles inside a wave, LDS across waves) and every window node sums
-//      the events of its four CIC corner cells in sorted order — a segmented
-//      reduction with no atomics (DepositCurrentsInCellSplit :1547-1655 /
-//      MoveInCell movepart_layer_CIC.cpp:449-496);
+//   3. every deposit event (one per sub-step, :1391-1466) enters the list of its
+//      window cell; the lane that owns the cell orders the list by event index and
+//      sums the events over the cell's four nodes in registers, and the four
+//      corners go to the window's node sums in LDS in four turns
+//      (DepositCurrentsInCellSplit :1547-1655 / MoveInCell
+//      movepart_layer_CIC.cpp:449-496).  A round with a crowded cell, and the
+//      float form, sort the chunk's events by cell and index instead, every node
+//      summing the runs of its four corner cells;
 //   4. the 21x21 node window (tile + 2-cell halo + 1) goes to HBM and
 //      k_combine adds the windows overlapping each node in a fixed order,
 //      which is the periodic ghost fold of ExchangeCurrentsSplit (:1685-1711).
@@ -29,6 +31,8 @@
 // summation order, is a pure function of the input.
 
 #include <hip/hip_ext.h>
+
+#include <type_traits>
 
 #include "qss_internal.h"
 #include "split_bf16.h"
@@ -56,11 +60,16 @@ struct TileArgs {
   int ntj, ntk, ny, nz;
   const double *F;
   const float *Ff;        // fp32 push field (mixed modes)
-  double hx, hy, hz, weight;
+  // products of uniform values, made on the host: there is no scalar FP64 unit, so
+  // in the kernel each would sit in a vector register pair for its whole run
+  double kick;            // charge over mass (-1) times half the slice step
+  double mweight;         // -weight: the deposit factor of an electron
   double hxy, hxz;        // hx / hy, hx / hz
+  double nyd, nzd;        // ny, nz
+  double lo[2], hi[2];    // -2 ny, -2 nz; 3 ny, 3 nz: positions past these are errors
   double bext[3];         // uniform external B (movepart_splitlayer.cpp:1271-1273)
-  int shape, full;
-  double *win;            // ntiles x NWIN x 4
+  int shape;
+  double *win;            // per tile and part 4 components (rho last) of NWIN nodes
   // full step staging (indexed by the old slot)
   double *sy, *sz, *spx, *spy, *spz;
   int32_t *scell, *sdest;  // sdest = direction | rank << 4
@@ -104,66 +113,291 @@ __host__ __device__ inline TileArgs wake_view(const TileArgs &a0, int w) {
 
 using qss_tile::sort256;
 
+template <typename T>
+struct alignas(2 * sizeof(T)) pair_t {
+  T x, y;
+};
+template <typename FT>
+__device__ inline const FT *field_of(const TileArgs &a) {
+  if constexpr (sizeof(FT) == 8) return a.F;
+  else return a.Ff;
+}
+
+// 1 / sqrt(1 + p^2).  In double: the hardware's estimate (about 2^-24) and two
+// Newton steps on g = x y, h = y / 2 (Goldschmidt's coupled form), then a last
+// correction, 13 operations with an error under an ulp, where the square root and
+// the division it replaces are 29 with two roundings.
+__device__ inline float inv_gamma(float px, float py, float pz) {
+  return 1.0f / sqrt(1.0f + px * px + py * py + pz * pz);
+}
+__device__ inline double inv_gamma(double px, double py, double pz) {
+  const double x = 1.0 + px * px + py * py + pz * pz;
+  double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  y = __builtin_fma(h, __builtin_fma(-h, g, 0.5), h);   // half of 1/sqrt(x)
+  y = y + y;
+  return __builtin_fma(0.5 * y, __builtin_fma(-(x * y), y, 1.0), y);
+}
+
+// threadIdx.x through a register the compiler cannot see into, where the masks and
+// addresses it gives should be remade in each round: kept over the chunk loop they
+// spill what the loop needs
+__device__ inline int thread_index() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+// ---- deposit of one round (at most one event per thread) ----------------------
+// By cells: 256 particles of 4 per cell make lists of about 4, and each event is
+// read once, where the sort of 256 keys (36 exchange stages, six of them through LDS
+// with two barriers each) and the four reads of each event by its nodes took a third
+// of a chunk's time.  Pushes of a 512^2 plane, 4 per cell: 44.5 us (full: 54.7) with
+// the sort, 34.4 (42.7) by cells, all else as it is here.
+// kCell: events of a cell that its owner lane sums directly: the bytes of one 8-byte
+// list, and past 8 the longest list sets the pace of its wave.
+constexpr int kCell = 8;
+
+template <int N>
+__device__ inline void sort_network(int *v) {
+  const auto cx = [&](int i, int j) {
+    const int a = v[i], b = v[j];
+    v[i] = min(a, b);
+    v[j] = max(a, b);
+  };
+  if constexpr (N == 4) {
+    cx(0, 1); cx(2, 3); cx(0, 2); cx(1, 3); cx(1, 2);
+  } else {   // 19 exchanges for 8
+    static_assert(N == 8, "networks for 4 and 8");
+    cx(0, 2); cx(1, 3); cx(4, 6); cx(5, 7); cx(0, 4); cx(1, 5); cx(2, 6); cx(3, 7);
+    cx(0, 1); cx(2, 3); cx(4, 5); cx(6, 7); cx(2, 4); cx(3, 5); cx(1, 4); cx(3, 6);
+    cx(1, 2); cx(3, 4); cx(5, 6);
+  }
+}
+
+// Sums of one cell's events over its four nodes, in the order of the events'
+// indices: the order in which they reached the list does not matter.
+template <int N, int NQ>
+__device__ inline void cell_sums(uint2 bytes, int n, const double *ev_y, const double *ev_z,
+                                 const double (*ev_w)[NT], bool cic, double (*s)[NQ]) {
+  int e[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    e[i] = i < n ? (int)((i < 4 ? bytes.x >> 8 * i : bytes.y >> 8 * (i - 4)) & 255) : NT + i;
+  sort_network<N>(e);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if (i >= n) break;
+    const int ei = e[i];
+    double w[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) w[q] = ev_w[q][ei];
+    // NGP: all of it in corner 0
+    const double yp = cic ? ev_y[ei] : 0., zp = cic ? ev_z[ei] : 0.;
+    const double yc = 1. - yp, zc = 1. - zp;
+    const double c[4] = {yc * zc, yp * zc, yc * zp, yp * zp};
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) s[k][q] = __builtin_fma(c[k], w[q], s[k][q]);
+  }
+}
+
+// A lane sums the events of the window cell it owns in this half (cells 0 .. NT - 1
+// or the rest) over the four corners in registers, each event read once, and the
+// four corners are added to the node sums one after the other, a barrier
+// between: in one corner's turn no two cells share a node.  Cells are dealt to
+// the waves in turn, since a chunk's events lie in few neighbouring rows.
+// Leaves the counts at zero.
+template <int NQ>
+__device__ inline void deposit_cells(int half, int *cnt, const uint2 *list, const double *ev_y,
+                                     const double *ev_z, const double (*ev_w)[NT],
+                                     double (*wacc)[NWIN], bool cic) {
+  const int t = thread_index();
+  const int cell = 4 * (t & 63) + (t >> 6) + NT * half;
+  double s[4][NQ];
+  const int n = cell < NWIN ? cnt[cell] : 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) s[k][q] = 0.0;
+  if (n) {
+    cnt[cell] = 0;
+    const uint2 bytes = list[cell];
+    if (n <= 4) cell_sums<4, NQ>(bytes, n, ev_y, ev_z, ev_w, cic, s);
+    else cell_sums<8, NQ>(bytes, n, ev_y, ev_z, ev_w, cic, s);
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (k > 0 && !cic) break;
+    if (n) {
+      const int node = cell + (k & 1) + (k >> 1) * W;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) wacc[q][node] += s[k][q];
+    }
+    __syncthreads();
+  }
+}
+
+// A round with more than kCell events in some cell: the events sorted by cell and
+// index, every node summing the runs of its four corner cells.
+template <int NQ>
+__device__ inline void deposit_sorted(int cellw, int *keys, int *sorted, short *cstart,
+                                            short *cend, double *ev_y, double *ev_z,
+                                            double (*ev_w)[NT], double (*wacc)[NWIN], bool cic) {
+  const int t = thread_index();
+  for (int i = t; i < NWIN; i += NT) { cstart[i] = 0; cend[i] = 0; }
+  const int sk = sort256(cellw < 0 ? kInvalid : cellw << 8 | t, keys);
+  sorted[t] = sk;
+  // the event at sorted position t, moved there in place: gathered before the
+  // barrier, stored after it, so the node sums below read events without the
+  // sorted[] indirection
+  double gy = 0, gz = 0, gw[NQ];
+  if (sk != kInvalid) {
+    const int e = sk & 255;
+    gy = ev_y[e];
+    gz = ev_z[e];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) gw[q] = ev_w[q][e];
+  }
+  __syncthreads();
+  if (sk != kInvalid) {
+    ev_y[t] = gy;
+    ev_z[t] = gz;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) ev_w[q][t] = gw[q];
+    const int c = sk >> 8;
+    const int prev = t > 0 ? sorted[t - 1] : kInvalid;
+    const int next = t + 1 < NT ? sorted[t + 1] : kInvalid;
+    if (t == 0 || (prev >> 8) != c) cstart[c] = (short)t;
+    if (next == kInvalid || (next >> 8) != c) cend[c] = (short)(t + 1);
+  }
+  __syncthreads();
+  for (int n = t; n < NWIN; n += NT) {
+    double acc[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) acc[q] = wacc[q][n];
+    const int nl_j = n % W, nl_k = n / W;
+    // corners: own cell (1-y)(1-z); left y(1-z); below (1-y)z; both yz
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn) {
+      if (!cic && cn > 0) break;
+      const int cj = nl_j - (cn & 1), ck = nl_k - (cn >> 1);
+      if (cj < 0 || ck < 0) continue;
+      const int cw = ck * W + cj;
+      const int e1 = cend[cw];
+      for (int e = cstart[cw]; e < e1; ++e) {
+        if (cic) {
+          const double ayp = ev_y[e], ayc = 1. - ayp, azp = ev_z[e], azc = 1. - azp;
+          const double wy = (cn & 1) ? ayp : ayc;
+          const double wz = (cn >> 1) ? azp : azc;
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) acc[q] += ev_w[q][e] * wy * wz;
+        } else {
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) acc[q] += ev_w[q][e];
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) wacc[q][n] = acc[q];
+  }
+}
+
 // R: arithmetic of the push (double: the reference's; float: mixed modes).
 // FT: storage of the push field.  Positions and momenta are carried in
 // double in both: the float form computes each slice's kick, rotation and
 // displacement in float and adds them to the double state, and the deposit
-// weights are summed in double.  With R = double every expression below
+// weights are summed in double.  With R = double every expression of the push
 // evaluates exactly as the reference's (no contraction, same association).
 //
 // A tile's particles may be shared by nsplit work-groups (part p takes
 // chunks p, p + nsplit, ...): each part writes its own window, direction
 // counts and ranks, and the combine / reorder kernels visit the parts in
 // order, so results are a pure function of the input and nsplit.
-// 128 VGPRs at most: four waves per SIMD, so all the tiles of a 512^2 grid
-// (4 work-groups per CU) are resident at once.
+// 128 VGPRs and 40 KB of LDS at most (RHO: 46 KB): four waves per SIMD, so all the
+// tiles of a 512^2 grid (4 work-groups per CU) are resident at once.  The bound is
+// instruction issue and latency, not memory: at 512^2 and 4 per cell 58 MB in and
+// 15 MB out (full: 61 MB) in 34.4 us (full: 42.7), half of the wave cycles waiting at
+// barriers and for LDS.  What spilled registers here cost most: with uniform FP64
+// products made on the host, the sort's lane masks not kept over the loop and
+// machine LICM off (it keeps FP64 literals in registers) nothing spills, 37 us on
+// average of a step's three pushes against 42.6 with 104 scalar registers spilled.
+// FULL: the pushed particles are staged for the reorder.
 // RHO = false: the deposit sums Jx, Jy, Jz only and the windows' density
 // component stays 0 (inside a layer step nothing reads the deposited density:
 // the corrector takes rho from continuity in spectral space).
-template <typename R, typename FT, bool RHO>
+template <typename R, typename FT, bool RHO, bool FULL>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4)))
 void k_push_tile(TileArgs a0) {
   const TileArgs a = wake_view(a0, blockIdx.y);   // wake of a batch
   const long pw = (long)blockIdx.y * a0.npw;
-  __shared__ FT Fw[NF * 6];
-  __shared__ int keys_sh[NT];
-  __shared__ int sorted[NT];
-  __shared__ double ev_y[NT], ev_z[NT];
-  __shared__ double4 ev_w[NT];
-  __shared__ short cstart[NWIN], cend[NWIN];
+  // components in pairs and events component by component: neighbouring cells
+  // and neighbouring events then lie side by side, one access of a wave free of
+  // bank conflicts (a node's six or an event's four together cost 362 conflict
+  // cycles per wave and chunk, a third of the LDS time)
+  __shared__ pair_t<FT> Fw[3][NF];
+  constexpr int NQ = RHO ? 4 : 3;
+  // The float form always deposits through the sort: its fields are rounded to
+  // float between the steps, and another order of the FP64 sums would flip some of
+  // those roundings.
+  constexpr bool CELLS = sizeof(R) == 8;
+  __shared__ double ev_y[NT], ev_z[NT], ev_w[NQ][NT];
+  __shared__ double wacc[NQ][NWIN];   // the window's node sums
+  // the round's events of each cell, or the sort's arrays in a crowded round
+  __shared__ union {
+    struct {
+      int cnt[NWIN];
+      uint2 list[NWIN];   // kCell event indices, a byte each
+    } cell;
+    struct {
+      int keys[NT], sorted[NT];
+      short cstart[NWIN], cend[NWIN];
+    } sort;
+  } sh;
   __shared__ int dir_total[9];
   __shared__ int wave_cnt[NT / 64][9];
-  __shared__ int flag_sh;
+  // what a round's events say to all: some cell is crowded, some particle has
+  // another sub-step, events in the first and in the second half of the cells.
+  // Two sets: one is cleared while the other is read.
+  enum { FL_CROWDED, FL_MORE, FL_HALF0, FL_HALF1, FL_N };
+  __shared__ int flag_sh[2][FL_N];
 
   const int t = threadIdx.x;
   const int tile = blockIdx.x / a.nsplit, part = blockIdx.x - tile * a.nsplit;
   const int tj = tile % a.ntj, tk = tile / a.ntj;
   const int j0 = tj * T, k0 = tk * T;
   const int ny = a.ny, nz = a.nz;
-  const double hx = a.hx, hy = a.hy, hz = a.hz;
-  const double q2m = -1.0, djx0 = -1.0, djy0 = -1.0, djz0 = -1.0, drho0 = -1.0;
-  const double weight = a.weight;
+  const R kick = (R)a.kick, mweight = (R)a.mweight;
   const bool cic = a.shape == QSS_SHAPE_CIC;
   int status = 0;   // ST_* bits met by this thread, reported once at the end
+
+  const int base = a.tile_start[tile];
+  const int np = a.tile_start[tile + 1] - base;
 
   // 1. field window: nodes (j0..j0+T, k0..k0+T), periodic
   for (int i = t; i < NF; i += NT) {
     const int lj = i % FW, lk = i / FW;
-    const long g = wrapi(j0 + lj, ny) + (long)ny * wrapi(k0 + lk, nz);
+    const int gj = j0 + lj < ny ? j0 + lj : 0, gk = k0 + lk < nz ? k0 + lk : 0;   // at most one past
+    const long g = gj + (long)ny * gk;
     const long plane = (long)ny * nz;
+    const FT *const F = field_of<FT>(a);
 #pragma unroll
-    for (int q = 0; q < kPushComp; ++q) {
-      if constexpr (sizeof(FT) == 8) Fw[i * 6 + q] = a.F[q * plane + g];
-      else Fw[i * 6 + q] = a.Ff[q * plane + g];
-    }
+    for (int q = 0; q < 3; ++q) Fw[q][i] = {F[2 * q * plane + g], F[(2 * q + 1) * plane + g]};
   }
   if (t < 9) dir_total[t] = 0;
-  double acc0[4] = {0, 0, 0, 0}, acc1[4] = {0, 0, 0, 0};
-  const int n0 = t, n1 = t + NT;   // owned window nodes
+  if (t < 2 * FL_N) flag_sh[t / FL_N][t % FL_N] = 0;
+  int par = 0;
+  for (int i = t; i < NWIN; i += NT) {
+    if constexpr (CELLS) sh.cell.cnt[i] = 0;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) wacc[q][i] = 0.0;
+  }
   __syncthreads();
 
-  const int base = a.tile_start[tile];
-  const int np = a.tile_start[tile + 1] - base;
   for (int c0 = part * NT; c0 < np; c0 += a.nsplit * NT) {
     const int slot = base + c0 + t;
     const long gs = pw + slot;   // the wake's particle arrays, unmoved pointers
@@ -172,18 +406,16 @@ void k_push_tile(TileArgs a0) {
     double yp = 0, zp = 0, px = 0, py = 0, pz = 0;
     R djx = 0, djy = 0, djz = 0, drho = 0, dy = 0, dz = 0, partdx = 0, step = 1;
     if (active) {
-      const int32_t c = a0.cell[gs];
-      cell_jk(c, ny, a.ny_magic, j, k);
+      cell_jk(a0.cell[gs], ny, a.ny_magic, j, k);
       yp = a0.y[gs];
       zp = a0.z[gs];
       if (!(yp >= 0 && yp <= 1 && zp >= 0 && zp <= 1)) status |= (ST_PARTICLE);
       px = a0.px[gs]; py = a0.py[gs]; pz = a0.pz[gs];
       const R rpx = (R)px, rpy = (R)py, rpz = (R)pz;
-      const R gammap = sqrt(R(1) + rpx * rpx + rpy * rpy + rpz * rpz);
-      // one correctly rounded reciprocal per denominator, then products: the
-      // reference divides by the same gamma and 1 - Vx many times over
-      // (movepart_splitlayer.cpp:1239-1330); results agree to an ulp per step
-      const R igp = R(1) / gammap;
+      // one reciprocal per denominator, then products: the reference divides by
+      // the same gamma and 1 - Vx many times over (movepart_splitlayer.cpp:
+      // 1239-1330); results agree to an ulp per step
+      const R igp = inv_gamma(rpx, rpy, rpz);
       R Vx = rpx * igp;
       const R Vxp = Vx, Vyp = rpy * igp, Vzp = rpz * igp;
       // gather from the staged window: local node (j - j0, k - k0)
@@ -194,22 +426,29 @@ void k_push_tile(TileArgs a0) {
         lk = min(max(lk, 0), T - 1);
       }
       R f[6];
-      const FT *f00 = &Fw[(lj + FW * lk) * 6];
+      const int i00 = lj + FW * lk;
       if (!cic) {
 #pragma unroll
-        for (int q = 0; q < 6; ++q) f[q] = (R)f00[q];
+        for (int q = 0; q < 3; ++q) {
+          const pair_t<FT> v = Fw[q][i00];
+          f[2 * q] = (R)v.x;
+          f[2 * q + 1] = (R)v.y;
+        }
       } else {
-        const FT *f10 = f00 + 6, *f01 = f00 + 6 * FW, *f11 = f01 + 6;
         const R ayc = R(1. - yp), ayp = R(yp), azc = R(1. - zp), azp = R(zp);
         const R acc = ayc * azc, apc = ayp * azc, acp = ayc * azp, app = ayp * azp;
 #pragma unroll
-        for (int q = 0; q < 6; ++q)
-          f[q] = acc * (R)f00[q] + apc * (R)f10[q] + acp * (R)f01[q] + app * (R)f11[q];
+        for (int q = 0; q < 3; ++q) {
+          const pair_t<FT> f00 = Fw[q][i00], f10 = Fw[q][i00 + 1], f01 = Fw[q][i00 + FW],
+                           f11 = Fw[q][i00 + FW + 1];
+          f[2 * q] = acc * (R)f00.x + apc * (R)f10.x + acp * (R)f01.x + app * (R)f11.x;
+          f[2 * q + 1] = acc * (R)f00.y + apc * (R)f10.y + acp * (R)f01.y + app * (R)f11.y;
+        }
       }
       R ex = f[0], ey = f[1], ez = f[2], bx = f[3], by = f[4], bz = f[5];
-      ex *= R(q2m * hx / 2.);
-      ey *= R(q2m * hx / 2.);
-      ez *= R(q2m * hx / 2.);
+      ex *= kick;
+      ey *= kick;
+      ez *= kick;
       // half kick, carried in the double state
       const R iu = R(1) / (R(1) - Vx);
       const R kx = ex * iu, ky = ey * iu, kz = ez * iu;
@@ -217,12 +456,11 @@ void k_push_tile(TileArgs a0) {
       py += (double)ky;
       pz += (double)kz;
       const R hpx = (R)px, hpy = (R)py, hpz = (R)pz;
-      R gamma = sqrt(R(1) + hpx * hpx + hpy * hpy + hpz * hpz);
-      const R gamma_r = R(1) / gamma;
+      const R gamma_r = inv_gamma(hpx, hpy, hpz);
       bx += R(a.bext[0]);
       by += R(a.bext[1]);
       bz += R(a.bext[2]);
-      const R beta = gamma_r * R(q2m) * iu * R(0.5 * hx);
+      const R beta = gamma_r * iu * kick;
       bx = bx * beta;
       by = by * beta;
       bz = bz * beta;
@@ -240,16 +478,15 @@ void k_push_tile(TileArgs a0) {
       py += (double)(ky + py_new);
       pz += (double)(kz + pz_new);
       const R npx = (R)px, npy = (R)py, npz = (R)pz;
-      gamma = sqrt(R(1) + npx * npx + npy * npy + npz * npz);
-      const R ig = R(1) / gamma;
+      const R ig = inv_gamma(npx, npy, npz);
       const R Vxm = npx * ig, Vym = npy * ig, Vzm = npz * ig;
       Vx = R(0.5) * (Vxm + Vxp);
       const R Vy = R(0.5) * (Vym + Vyp), Vz = R(0.5) * (Vzm + Vzp);
       const R iv = R(1) / (R(1) - Vx);
-      djx = R(weight * djx0) * Vxm * iv;
-      djy = R(weight * djy0) * Vym * iv;
-      djz = R(weight * djz0) * Vzm * iv;
-      drho = R(weight * drho0) * iv;
+      djx = mweight * Vxm * iv;
+      djy = mweight * Vym * iv;
+      djz = mweight * Vzm * iv;
+      drho = mweight * iv;
       dy = Vy * R(a.hxy) * iv;
       dz = Vz * R(a.hxz) * iv;
       if (fabs(dy) > R(1) || fabs(dz) > R(1)) {
@@ -269,23 +506,24 @@ void k_push_tile(TileArgs a0) {
     // sub-step rounds: round r deposits every particle's r-th sub-step
     for (;;) {
       const bool have = active && partdx > 0.;
-      int key = kInvalid;
+      int cellw = -1;   // this round's window cell
       if (have) {
         R part_step;
-        if (partdx > R(1)) { partdx -= R(1); part_step = R(1) / step; }
+        if (step == R(1)) { part_step = R(1); partdx = R(0); }   // partdx is 1: one step
+        else if (partdx > R(1)) { partdx -= R(1); part_step = R(1) / step; }
         else { part_step = partdx / step; partdx = R(0); }
         // the reference restarts every sub-step from the start cell
         ytmp += (double)(dy * part_step) + j;
         ztmp += (double)(dz * part_step) + k;
-        if (!(ytmp > -2.0 * ny && ytmp < 3.0 * ny && ztmp > -2.0 * nz && ztmp < 3.0 * nz)) {
+        if (!(ytmp > a.lo[0] && ytmp < a.hi[0] && ztmp > a.lo[1] && ztmp < a.hi[1])) {
           status |= (ST_PARTICLE);
           ytmp = 0.0;
           ztmp = 0.0;
         }
-        while (ytmp > ny) ytmp -= ny;
-        while (ytmp < 0) ytmp += ny;
-        while (ztmp > nz) ztmp -= nz;
-        while (ztmp < 0) ztmp += nz;
+        while (ytmp > a.nyd) ytmp -= a.nyd;
+        while (ytmp < 0) ytmp += a.nyd;
+        while (ztmp > a.nzd) ztmp -= a.nzd;
+        while (ztmp < 0) ztmp += a.nzd;
         jj = (int)ytmp;
         kk = (int)ztmp;
         ytmp -= jj;
@@ -300,83 +538,49 @@ void k_push_tile(TileArgs a0) {
         else if (dk + H > W - 2) dk -= nz;
         const int lj = dj + H, lk = dk + H;
         if (lj >= 0 && lj <= W - 2 && lk >= 0 && lk <= W - 2) {
-          key = ((lk * W + lj) << 8) | t;
+          cellw = lk * W + lj;
           ev_y[t] = ytmp;
           ev_z[t] = ztmp;
-          ev_w[t] = make_double4((double)(djx * part_step), (double)(djy * part_step),
-                                 (double)(djz * part_step),
-                                 RHO ? (double)(drho * part_step) : 0.0);
+          ev_w[0][t] = (double)(djx * part_step);
+          ev_w[1][t] = (double)(djy * part_step);
+          ev_w[2][t] = (double)(djz * part_step);
+          if constexpr (RHO) ev_w[3][t] = (double)(drho * part_step);
+          if constexpr (CELLS) {
+            const int r = atomicAdd(&sh.cell.cnt[cellw], 1);
+            if (r < kCell) reinterpret_cast<uint8_t *>(&sh.cell.list[cellw])[r] = (uint8_t)t;
+            else flag_sh[par][FL_CROWDED] = 1;
+            flag_sh[par][cellw < NT ? FL_HALF0 : FL_HALF1] = 1;
+          }
         } else {
           status |= (ST_FAR);
         }
       }
-      // segmented reduction of this round's events
-      for (int i = t; i < NWIN; i += NT) { cstart[i] = 0; cend[i] = 0; }
-      const int sk = sort256(key, keys_sh);
-      sorted[t] = sk;
-      // the event at sorted position t, moved there in place: gathered before
-      // the barrier (the sort's barriers made every event visible), stored after
-      // it, so the node sums below read events without the sorted[] indirection
-      double gy = 0, gz = 0;
-      double4 gw = make_double4(0.0, 0.0, 0.0, 0.0);
-      if (sk != kInvalid) {
-        const int e = sk & 255;
-        gy = ev_y[e];
-        gz = ev_z[e];
-        gw = ev_w[e];
-      }
+      if (active && partdx > 0.) flag_sh[par][FL_MORE] = 1;
       __syncthreads();
-      if (sk != kInvalid) {
-        ev_y[t] = gy;
-        ev_z[t] = gz;
-        ev_w[t] = gw;
-        const int cellw = sk >> 8;
-        const int prev = t > 0 ? sorted[t - 1] : kInvalid;
-        const int next = t + 1 < NT ? sorted[t + 1] : kInvalid;
-        if (t == 0 || (prev >> 8) != cellw) cstart[cellw] = (short)t;
-        if (next == kInvalid || (next >> 8) != cellw) cend[cellw] = (short)(t + 1);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int o = 0; o < 2; ++o) {
-        const int n = o == 0 ? n0 : n1;
-        if (n >= NWIN) continue;
-        double *accn = o == 0 ? acc0 : acc1;
-        const int nl_j = n % W, nl_k = n / W;
-        // corners: own cell (1-y)(1-z); left y(1-z); below (1-y)z; both yz
-#pragma unroll
-        for (int cn = 0; cn < 4; ++cn) {
-          if (!cic && cn > 0) break;
-          const int cj = nl_j - (cn & 1), ck = nl_k - (cn >> 1);
-          if (cj < 0 || ck < 0) continue;
-          const int cw = ck * W + cj;
-          const int e1 = cend[cw];
-          for (int i = cstart[cw]; i < e1; ++i) {
-            const int e = i;   // events are stored in sorted order
-            const double4 wv = ev_w[e];
-            const double wq[4] = {wv.x, wv.y, wv.z, wv.w};
-            if (cic) {
-              const double ayp = ev_y[e], ayc = 1. - ayp, azp = ev_z[e], azc = 1. - azp;
-              const double wy = (cn & 1) ? ayp : ayc;
-              const double wz = (cn >> 1) ? azp : azc;
-#pragma unroll
-              for (int q = 0; q < (RHO ? 4 : 3); ++q) accn[q] += wq[q] * wy * wz;
-            } else {
-#pragma unroll
-              for (int q = 0; q < (RHO ? 4 : 3); ++q) accn[q] += wq[q];
-            }
-          }
+      const int *fl = flag_sh[par];
+      const bool more = fl[FL_MORE], crowded = !CELLS || fl[FL_CROWDED];
+      const bool half0 = fl[FL_HALF0], half1 = fl[FL_HALF1];
+      par ^= 1;
+      if (t < FL_N) flag_sh[par][t] = 0;   // last read a barrier ago
+      if (crowded) {
+        if constexpr (CELLS) __syncthreads();   // the lists give way to the sort
+        deposit_sorted<NQ>(cellw, sh.sort.keys, sh.sort.sorted, sh.sort.cstart, sh.sort.cend, ev_y,
+                           ev_z, ev_w, wacc, cic);
+        __syncthreads();
+        if constexpr (CELLS) {
+          for (int i = t; i < NWIN; i += NT) sh.cell.cnt[i] = 0;
+          __syncthreads();
         }
+      } else {
+        // rolled: the code of a work-group's first pass comes from L2 line by line
+#pragma unroll 1
+        for (int half = half0 ? 0 : 1; half < (half1 ? 2 : 1); ++half)
+          deposit_cells<NQ>(half, sh.cell.cnt, sh.cell.list, ev_y, ev_z, ev_w, wacc, cic);
+        if (!half0 && !half1) __syncthreads();   // the flags are clear before the next round
       }
-      if (t == 0) flag_sh = 0;
-      __syncthreads();
-      if (active && partdx > 0.) flag_sh = 1;
-      __syncthreads();
-      const int more = flag_sh;
-      __syncthreads();
       if (!more) break;
     }
-    if (a.full) {
+    if constexpr (FULL) {
       // destination tile direction (canonical for 1 or 2 tiles per axis)
       int dtj = 0, dtk = 0;
       if (active) {
@@ -392,7 +596,7 @@ void k_push_tile(TileArgs a0) {
       }
       const int dir = (dtj + 1) + 3 * (dtk + 1);
       // rank among this tile's particles with the same direction, slot order
-      const int lane = t & 63, wv = t >> 6;
+      const int ti = thread_index(), lane = ti & 63, wv = ti >> 6;
       const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
       int myrank_w = 0;
       // kept rolled: nine live ballot masks would spill scalar registers
@@ -425,11 +629,10 @@ void k_push_tile(TileArgs a0) {
   }
   if (status) atomicOr(&a.counters[1], status);
   // 4. window to HBM
-  double *wout = a.win + (long)blockIdx.x * NWIN * 4;
-  reinterpret_cast<double4 *>(wout)[n0] = make_double4(acc0[0], acc0[1], acc0[2], acc0[3]);
-  if (n1 < NWIN)
-    reinterpret_cast<double4 *>(wout)[n1] = make_double4(acc1[0], acc1[1], acc1[2], acc1[3]);
-  if (a.full && t < 9) a.tcount[blockIdx.x * 9 + t] = dir_total[t];
+  double4 *wout = reinterpret_cast<double4 *>(a.win + (long)blockIdx.x * NWIN * 4);
+  for (int i = t; i < NWIN; i += NT)
+    wout[i] = make_double4(wacc[0][i], wacc[1][i], wacc[2][i], RHO ? wacc[NQ - 1][i] : 0.0);
+  if (FULL && t < 9) a.tcount[blockIdx.x * 9 + t] = dir_total[t];
 }
 
 // sum of the windows covering each node, fixed (dtk, dtj, part) order.  Per
@@ -665,10 +868,14 @@ TileArgs make_args(qss_ctx *c, int full) {
   a.ntj = c->ntj; a.ntk = c->ntk; a.ny = c->ny; a.nz = c->nz;
   a.F = c->F;
   a.Ff = c->Ff;
-  a.hx = c->hxs; a.hy = c->hy; a.hz = c->hz; a.weight = c->pweight;
+  a.kick = -0.5 * c->hxs;
+  a.mweight = -c->pweight;
+  a.nyd = c->ny; a.nzd = c->nz;
+  a.lo[0] = -2.0 * c->ny; a.lo[1] = -2.0 * c->nz;
+  a.hi[0] = 3.0 * c->ny; a.hi[1] = 3.0 * c->nz;
   a.hxy = c->hxs / c->hy; a.hxz = c->hxs / c->hz;
   for (int q = 0; q < 3; ++q) a.bext[q] = c->p.b_ext[q];
-  a.shape = c->p.shape; a.full = full;
+  a.shape = c->p.shape;
   a.win = c->win;
   const long npall = c->np_cap * c->nw;
   a.sy = c->ev_y; a.sz = c->ev_z; a.spx = c->ev_p; a.spy = c->ev_p + npall;
@@ -686,9 +893,15 @@ TileArgs make_args(qss_ctx *c, int full) {
 
 hipError_t launch_push_tile(qss_ctx *c, int full, bool rho, hipEvent_t ev0, hipEvent_t ev1) {
   const dim3 grid(c->ntj * c->ntk * c->nsplit, c->nw), block(NT);
-  auto fn = c->mixed ? (rho ? k_push_tile<float, float, true> : k_push_tile<float, float, false>)
-                     : (rho ? k_push_tile<double, double, true>
-                            : k_push_tile<double, double, false>);
+  const auto pick = [&](auto r, auto f) {
+    using T = decltype(r);
+    constexpr bool F = decltype(f)::value;
+    return rho ? k_push_tile<T, T, true, F> : k_push_tile<T, T, false, F>;
+  };
+  const std::true_type yes;
+  const std::false_type no;
+  auto fn = c->mixed ? (full ? pick(0.0f, yes) : pick(0.0f, no))
+                     : (full ? pick(0.0, yes) : pick(0.0, no));
   if (ev0 || ev1)
     hipExtLaunchKernelGGL(fn, grid, block, 0, c->stream, ev0, ev1, 0, make_args(c, full));
   else

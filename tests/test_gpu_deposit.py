@@ -1,0 +1,66 @@
+"""GPU: the tiled push's deposit at the edges of its branches: cells with one event,
+with as many as the small and the large sorting network take (4 and 8) and one more
+(the second network; the sort of a crowded round), rows of cells in the first half
+of the window's cells only, in the second only and in both, CIC and NGP, and hot
+particles that take several rounds.
+
+Currents and density against the oracle at the push tests' bound (1e-13 of the
+largest value: the same contributions, associated differently), and the same bits
+when the pass is run again (the order in which events reach a cell's list differs
+from run to run, their sum must not)."""
+import numpy as np
+import pytest
+
+from tests.helpers import max_rel, smooth_field
+from tertia_amd.params import QSS_SHAPE_CIC, QSS_SHAPE_NGP_REF, small
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape", [QSS_SHAPE_CIC, QSS_SHAPE_NGP_REF])
+@pytest.mark.parametrize("rows", [(0, 6), (10, 16), (0, 16)])
+@pytest.mark.parametrize("per_cell,hot", [(1, 0), (4, 0), (5, 0), (8, 0), (9, 0), (70, 0), (3, 8)])
+def test_deposit_cell_counts(oracle_mod, shape, rows, per_cell, hot):
+    from tertia_amd.mesh import Mesh
+    ny = nz = 48
+    rng = np.random.default_rng(per_cell + 100 * rows[0] + 1000 * rows[1])
+    p = small(ny=ny, nz=nz, nslices=2, hx=0.4 if hot else 0.05, shape=shape, ppc_y=2, ppc_z=4)
+    # whole cells of per_cell particles in the given rows of every tile, as many as fit
+    cells = [j + ny * k for k in range(nz) for j in range(ny) if rows[0] <= k % 16 < rows[1]]
+    cells = np.sort(rng.permutation(cells)[: ny * nz * 8 // per_cell])
+    cell = np.repeat(cells, per_cell)
+    n = len(cell)
+    mom = rng.uniform(-0.1, 0.1, size=(3, n))
+    if hot:
+        # past one cell in a slice: several sub-steps
+        mom[0, ::hot] = 3.0
+        mom[1, ::hot] = rng.uniform(-4, 4, size=len(mom[1, ::hot]))
+    parts = ((cell % ny).astype(np.int32), (cell // ny).astype(np.int32),
+             rng.uniform(0.2, 0.8, n), rng.uniform(0.2, 0.8, n), *mom,
+             np.arange(n, dtype=np.int64))
+    fields = {f: smooth_field(rng, nz, ny, 0.1) for f in ("Ex", "Ey", "Ez", "Bx", "By", "Bz")}
+    m, o = Mesh(p, history=()), oracle_mod.Oracle(p, history=())
+    try:
+        for f, F in fields.items():
+            for lay, which in (("C", 0), ("P", 1)):
+                o.set_field(f, F, which=which)
+                m.set_field(f, F, layer=lay)
+        o.set_particles(*parts)
+        runs = []
+        for _ in range(2):
+            m.set_particles(*parts)
+            got = []
+            for full in (0, 1):
+                m.MoveParticlesLayerSplit(0, 0, full)
+                got += [m.get_field(f) for f in ("Jx", "Jy", "Jz", "Rho")]
+            runs.append(got)
+        ref = []
+        for full in (0, 1):
+            o.push_deposit(full)
+            ref += [o.get_field(f) for f in ("Jx", "Jy", "Jz", "Rho")]
+        for g, r in zip(runs[0], ref):
+            assert max_rel(g, r) <= 1e-13
+        for a, b in zip(*runs):
+            assert np.array_equal(a, b)
+    finally:
+        m.close()
