@@ -29,7 +29,8 @@ struct BeamArgs {
   double *rho, *jx;   // C-layer beam planes
   int layer;          // reference layer index i = nslices-1-slice
   int nsplit, isplit;
-  const int *slice_dev;   // graph replay: the slice is read from device memory
+  int *slice_dev;         // graph replay: the slice is read from device memory, and
+                          // kept in the next word for the layer's end
   uint16_t *xs0, *xs1;    // split-bf16 modes: the planes as split transform operands
   int npc;
 };
@@ -193,6 +194,8 @@ __global__ __launch_bounds__(NT) void k_beam_plane(BeamArgs a) {
   const int w = blockIdx.y;   // wake of a batch
   const qss_bunch *bun = a.wb ? a.wb + (long)w * QSS_MAX_BUNCH : a.b;
   const int layer = a.slice_dev ? a.nslices - 1 - *a.slice_dev : a.layer;
+  if (a.slice_dev && blockIdx.x == 0 && w == 0 && threadIdx.x == 0)
+    a.slice_dev[1] = a.nslices - 1 - layer;
   // x-cells layer - 1 .. layer (+ layer + 1 for the split interpolation)
   const int ci0 = layer - 1;
   const int nx = a.nsplit > 1 ? 3 : 2;

@@ -285,7 +285,7 @@ struct PlaneArgs {
   double inv;          // 2^-e
   long ncell;
   int L, layer, nsplit, isplit;
-  const int *slice_dev;
+  int *slice_dev;   // {slice, the same for the layer's end}
   double *rho, *jx;
   uint16_t *xs0, *xs1;
   int npc;
@@ -298,6 +298,7 @@ __global__ __launch_bounds__(NT) void k_driver_plane(PlaneArgs a) {
   const long n = (long)blockIdx.x * NT + threadIdx.x;
   if (n >= a.ncell) return;
   const int layer = a.slice_dev ? a.L - 1 - *a.slice_dev : a.layer;
+  if (a.slice_dev && blockIdx.x == 0 && threadIdx.x == 0) a.slice_dev[1] = a.L - 1 - layer;
   const long m = (long)layer * a.ncell + n;
   double rc = (double)(long long)a.acc_rho[m] * a.inv;
   double jc = (double)(long long)a.acc_jx[m] * a.inv;

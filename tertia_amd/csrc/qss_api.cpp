@@ -555,8 +555,7 @@ int line_fields(qss_ctx *c, bool psi, bool resid, bool keep_e, bool keep_b, bool
 }
 
 // in_step, keep_e: as do_guess
-int do_iterate(qss_ctx *c, int final_pass, double *res_dev, bool in_step = false,
-               bool keep_e = true) {
+int do_iterate(qss_ctx *c, int final_pass, bool in_step = false, bool keep_e = true) {
   if (use_lines(c)) {
     const bool lean = in_step && !final_pass, psi = final_pass && !c->skip_rho_psi;
     const int kz[3] = {QSS_KIND_C, QSS_KIND_C, QSS_KIND_S};
@@ -564,10 +563,6 @@ int do_iterate(qss_ctx *c, int final_pass, double *res_dev, bool in_step = false
     CHECK(line_cols(c, 3, kz, in, c->tmp, 1.0));
     CHECK(line_modes(c, false, !lean, final_pass, psi, !lean));
     CHECK(line_fields(c, psi, !lean, !lean || keep_e, !lean, final_pass));
-    if (res_dev) {
-      Timed t(c, KC_SPEC);
-      HIPCHECK(launch_residual_final(c, res_dev));
-    }
     return QSS_OK;
   }
   {
@@ -601,12 +596,7 @@ int do_iterate(qss_ctx *c, int final_pass, double *res_dev, bool in_step = false
   // rho and psi are outputs only (the next layer starts from the kept
   // spectra); a sweep that stores neither leaves them to its end
   const int nb = final_pass && !c->skip_rho_psi ? 8 : 6;
-  CHECK(transform_batch(c, nb, kz, ky, in, out, alpha, resid, push, pp, 0.0, false, true));
-  if (res_dev) {
-    Timed t(c, KC_SPEC);
-    HIPCHECK(launch_residual_final(c, res_dev));
-  }
-  return QSS_OK;
+  return transform_batch(c, nb, kz, ky, in, out, alpha, resid, push, pp, 0.0, false, true);
 }
 
 void swap_c_p(qss_ctx *c) {
@@ -682,9 +672,33 @@ double *tape_field(const qss_ctx *c, char *slot, int pass) {
                                     (size_t)pass * kPushComp * align256(c->ncell * 8));
 }
 
+// the finished layer into the history (movepart_splitlayer.cpp:467-473);
+// wake w of a batch at hist + (w * nslices + s) * ncell.  The layer's fields
+// are in P after the closing swap; its beam planes stay in C (the swap
+// leaves them, the next layer overwrites them).
+const double *history_source(const qss_ctx *c, int f) {
+  return f == QSS_RHOBEAM || f == QSS_JXBEAM ? c->C[f] : c->P[f];
+}
+
+// the step's residual -> res_dev, with keep the kept fields' planes -> history
+int layer_end(qss_ctx *c, int slice, double *res_dev, bool keep) {
+  const double *src[QSS_NFIELD];
+  double *hist[QSS_NFIELD];
+  int nf = 0;
+  for (int f = 0; keep && f < QSS_NFIELD; ++f)
+    if (c->hist[f]) {
+      src[nf] = history_source(c, f);
+      hist[nf++] = c->hist[f];
+    }
+  Timed t(c, KC_SPEC);
+  HIPCHECK(launch_layer_end(c, slice, res_dev, src, hist, nf));
+  return QSS_OK;
+}
+
 // tape != null: record the layer's start particles and every pass's push
 // field (the reverse sweep replays the pushes from them)
-int do_layer_step(qss_ctx *c, int slice, int isplit, double *res_dev, char *tape = nullptr) {
+int do_layer_step(qss_ctx *c, int slice, int isplit, double *res_dev, bool keep,
+                  char *tape = nullptr) {
   if (tape) CHECK(tape_particles(c, part_view(c, tape)));
   // recording: the inverse transforms' epilogue writes each pass's push field
   // straight into its tape slot, which that pass's push then reads
@@ -711,13 +725,13 @@ int do_layer_step(qss_ctx *c, int slice, int isplit, double *res_dev, char *tape
   for (int it = 0; it < c->p.n_iter; ++it) {
     CHECK(do_push_deposit(c, 0));
     field_of(it + 1);
-    CHECK(do_iterate(c, 0, nullptr, true, it == c->p.n_iter - 1));
+    CHECK(do_iterate(c, 0, true, it == c->p.n_iter - 1));
   }
   CHECK(do_push_deposit(c, 1));
   c->F = F0;   // the final corrector's push field is not replayed
-  CHECK(do_iterate(c, 1, res_dev, true));
+  CHECK(do_iterate(c, 1, true));
   swap_c_p(c);
-  return QSS_OK;
+  return layer_end(c, slice, res_dev, keep);
 }
 
 // checkpoint: particles + P planes + spectral state at a layer start
@@ -938,24 +952,6 @@ int adj_layer_step(qss_ctx *c, int slice, char *slot, const double *exbar, int &
   return QSS_OK;
 }
 
-// the finished layer into the history (movepart_splitlayer.cpp:467-473);
-// wake w of a batch at hist + (w * nslices + s) * ncell.  The layer's fields
-// are in P after the closing swap; its beam planes stay in C (the swap
-// leaves them, the next layer overwrites them).
-const double *history_source(const qss_ctx *c, int f) {
-  return f == QSS_RHOBEAM || f == QSS_JXBEAM ? c->C[f] : c->P[f];
-}
-
-int store_history(qss_ctx *c, int s) {
-  const size_t plane = c->ncell * sizeof(double);
-  for (int f = 0; f < QSS_NFIELD; ++f)
-    if (c->hist[f])
-      HIPCHECK(hipMemcpy2DAsync(c->hist[f] + (size_t)s * c->ncell, plane * c->p.nslices,
-                                history_source(c, f), plane, plane, c->nw,
-                                hipMemcpyDeviceToDevice, c->stream));
-  return QSS_OK;
-}
-
 void graph_free(qss_ctx *c) {
   if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
   if (c->graph) (void)hipGraphDestroy(c->graph);
@@ -966,15 +962,14 @@ void graph_free(qss_ctx *c) {
 
 // Layers s and s+1 by one graph launch.  The graph holds two layer steps
 // captured from the current pointer state; the layer index is read from
-// d_slice by the beam, residual and history kernels and advanced inside the
+// d_slice by the beam and layer-end kernels and advanced inside the
 // graph.  A replay from the other pointer parity runs one layer eagerly
 // first (returns 1 then: one layer done).
 int sweep_graph_pair(qss_ctx *c, int s, int *done) {
   const bool match = c->gexec && c->g_key_c0 == c->C[0] && c->g_key_cur == c->cur &&
                      c->g_key_rb == c->S[SP_RHOB] && c->g_key_skip == c->skip_rho_psi;
   if (c->gexec && !match) {
-    CHECK(do_layer_step(c, s, 0, c->d_res_hist + s));
-    CHECK(store_history(c, s));
+    CHECK(do_layer_step(c, s, 0, c->d_res_hist + s, true));
     *done = 1;
     return QSS_OK;
   }
@@ -988,11 +983,7 @@ int sweep_graph_pair(qss_ctx *c, int s, int *done) {
     int r = QSS_OK;
     for (int q = 0; q < 2 && r == QSS_OK; ++q) {
       // not the first layer; residual slot of layer 0 (+ d_slice at replay)
-      r = do_layer_step(c, 1, 0, c->d_res_hist);
-      for (int f = 0; f < QSS_NFIELD && r == QSS_OK; ++f)
-        if (c->hist[f] && launch_store_hist(c, history_source(c, f), c->hist[f]) != hipSuccess)
-          r = QSS_E_HIP;
-      if (r == QSS_OK && launch_add_i32(c->d_slice, 1, c->stream) != hipSuccess) r = QSS_E_HIP;
+      r = do_layer_step(c, 1, 0, c->d_res_hist, true);
     }
     c->capturing = false;
     hipGraph_t g = nullptr;
@@ -1039,8 +1030,7 @@ int adj_segment_graph(qss_ctx *c, int s0, const double *exbar, int &cur_adj, boo
     // does on the device
     for (int l = 0; l < a.K && r == QSS_OK; ++l) {
       // not the first layer; residual slot of layer 0 (+ d_slice at replay)
-      r = do_layer_step(c, 1, 0, c->d_res_hist, a.tape + (size_t)l * a.tape_stride);
-      if (r == QSS_OK && launch_add_i32(c->d_slice, 1, c->stream) != hipSuccess) r = QSS_E_HIP;
+      r = do_layer_step(c, 1, 0, c->d_res_hist, false, a.tape + (size_t)l * a.tape_stride);
     }
     for (int l = a.K - 1; l >= 0 && r == QSS_OK; --l) {
       if (launch_add_i32(c->d_slice, -1, c->stream) != hipSuccess) {
@@ -1375,7 +1365,7 @@ int qss_create(const qss_params *p, int device, uint32_t history_mask, qss_ctx *
       (r = dalloc(&c->off, nc)) || (r = dalloc(&c->off_main, nc)) ||
       (r = dalloc(&c->blk, c->nblk)) || (r = dalloc(&c->blk_main, c->nblk)) ||
       (r = dalloc(&c->list, np + ov)) || (r = dalloc(&c->d_resid, (long)kResidPerWake * nw)) ||
-      (r = dalloc(&c->d_slice, 1)) ||
+      (r = dalloc(&c->d_slice, 2)) ||
       (r = dalloc(&c->d_res_hist, (size_t)p->nslices * p->nx_split * nw)))
     return fail(r);
   if (c->tiled) {
@@ -1527,8 +1517,7 @@ int qss_sweep_range(qss_ctx *c, int first, int count, double *residuals) {
       continue;
     }
     for (int is = 0; is < S; ++is)
-      CHECK(do_layer_step(c, s, is, c->d_res_hist + (size_t)s * S + is));
-    CHECK(store_history(c, s));
+      CHECK(do_layer_step(c, s, is, c->d_res_hist + (size_t)s * S + is, is == S - 1));
     ++s;
   }
   if (c->skip_rho_psi && count > 0) CHECK(finish_rho_psi(c));
@@ -1614,10 +1603,8 @@ int qss_sweep_checkpointed(qss_ctx *c, int nrun, int every, double *residuals) {
   SkipRhoPsi skip(c);   // as the plain sweep, so that both take the same steps
   if (taped) {
     CHECK(checkpoint(c, a.chk, 0));
-    for (int s = 0; s < nrun; ++s) {
-      CHECK(do_layer_step(c, s, 0, c->d_res_hist + s, a.tape + (size_t)s * a.tape_stride));
-      CHECK(store_history(c, s));
-    }
+    for (int s = 0; s < nrun; ++s)
+      CHECK(do_layer_step(c, s, 0, c->d_res_hist + s, true, a.tape + (size_t)s * a.tape_stride));
     a.taped = true;
     every = nrun;   // skips the loop below
   }
@@ -1631,8 +1618,7 @@ int qss_sweep_checkpointed(qss_ctx *c, int nrun, int every, double *residuals) {
       s += done;
       continue;
     }
-    CHECK(do_layer_step(c, s, 0, c->d_res_hist + s));
-    CHECK(store_history(c, s));
+    CHECK(do_layer_step(c, s, 0, c->d_res_hist + s, true));
     ++s;
   }
   if (c->skip_rho_psi) CHECK(finish_rho_psi(c));
@@ -1689,7 +1675,8 @@ int qss_sweep_vjp(qss_ctx *c, const double *ex_bar, int on_host, double *grad_bi
       if (done) continue;
     }
     for (int s = s0; s < s1; ++s)
-      CHECK(do_layer_step(c, s, 0, c->d_res_hist + s, a.tape + (size_t)(s - s0) * a.tape_stride));
+      CHECK(do_layer_step(c, s, 0, c->d_res_hist + s, false,
+                          a.tape + (size_t)(s - s0) * a.tape_stride));
     for (int s = s1 - 1; s >= s0; --s)
       CHECK(adj_layer_step(c, s, a.tape + (size_t)(s - s0) * a.tape_stride, ex_bar_dev, cur_adj));
   }
@@ -1722,7 +1709,7 @@ int qss_layer_step(qss_ctx *c, int slice, int isplit, double *residual) {
   }
   HIPCHECK(hipSetDevice(c->device));
   double *dst = c->d_res_hist + (size_t)slice * c->p.nx_split + isplit;
-  CHECK(do_layer_step(c, slice, isplit, dst));
+  CHECK(do_layer_step(c, slice, isplit, dst, false));
   double r = 0;
   HIPCHECK(hipMemcpyAsync(&r, dst, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHECK(hipStreamSynchronize(c->stream));
@@ -1766,7 +1753,11 @@ int qss_iterate(qss_ctx *c, int final_pass, double *residual) {
   if (!c) return QSS_E_ARG;
   HIPCHECK(hipSetDevice(c->device));
   double *dst = c->d_res_hist;
-  CHECK(do_iterate(c, final_pass, dst));
+  CHECK(do_iterate(c, final_pass));
+  {
+    Timed t(c, KC_SPEC);
+    HIPCHECK(launch_layer_end(c, 0, dst, nullptr, nullptr, 0));
+  }
   double r = 0;
   HIPCHECK(hipMemcpyAsync(&r, dst, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHECK(hipStreamSynchronize(c->stream));

@@ -375,7 +375,7 @@ struct qss_ctx {
   // of a replay is read by the kernels from d_slice
   bool use_graph = false;
   bool capturing = false;
-  int *d_slice = nullptr;
+  int *d_slice = nullptr;   // {slice, the layer's own copy of it}
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   // one checkpoint segment of the reverse sweep (recomputation + reverse),
@@ -434,7 +434,11 @@ hipError_t launch_push(qss_ctx *c, int full_step);
 hipError_t launch_sort_scan(qss_ctx *c, int full_step);
 hipError_t launch_scatter(qss_ctx *c);
 hipError_t launch_tile_reduce(qss_ctx *c, int full_step);
-hipError_t launch_residual_final(qss_ctx *c, double *dst);
+// A layer's end: its residual -> *res and nf planes (wake-major) -> the given history
+// arrays at `slice`.  Capturing: res is the slot of slice 0, the slice is read from
+// d_slice at replay, and the launch steps d_slice to the next one.
+hipError_t launch_layer_end(qss_ctx *c, int slice, double *res, const double *const *src,
+                            double *const *hist, int nf);
 hipError_t launch_push_field(qss_ctx *c);
 // rho = false: the deposit leaves the density out (a layer step, whose
 // corrector takes rho from continuity)
@@ -446,8 +450,7 @@ hipError_t launch_tile_reorder(qss_ctx *c);
 hipError_t launch_seed_tiled(qss_ctx *c);
 hipError_t launch_axpy(double *y, const double *x, double a, long n, hipStream_t s,
                        const int *slice_dev = nullptr);
-// graph replay helpers: history store at the device-side slice, slice += v
-hipError_t launch_store_hist(qss_ctx *c, const double *src, double *hist);
+// graph replay helper: slice += v
 hipError_t launch_add_i32(int *p, int v, hipStream_t s);
 // adjoints of the spectral updates on the adjoint state A (flag: first layer
 // for the Guess, final pass for the Iterate)

@@ -261,27 +261,47 @@ __global__ __launch_bounds__(NT) void k_iterate_adj(SpecArgs a) {
 }
 
 // Eerr = max_c dif_c / max(1e-5, max_c)  (:1541, :1584-1621, :1641-1643)
-// wake w's residual slots -> dst[w * stride]; during a graph replay the
-// layer slot comes from device memory: dst += *slice_dev * per_slice
-__global__ void k_resid_final(const unsigned long long *r, double *dst, int nw, long stride,
-                              const int *slice_dev, int per_slice) {
-  // one wave per wake (blockIdx.x): max over the slots, lanes then shuffles;
-  // the bit patterns of non-negative doubles (and of +inf) order like the values
-  const int w = blockIdx.x, lane = threadIdx.x;
-  if (w >= nw) return;
-  r += (long)kResidPerWake * w;
-  dst += w * stride;
-  if (slice_dev) dst += (long)(*slice_dev) * per_slice;
+// What ends a layer, in one launch: wake w's residual slots -> res[w * stride] (the
+// first nw work-groups), the kept fields' planes -> their history (the others, 16 KB
+// each), and in a graph replay the step to the next slice.  A replay's slice is read
+// here from the copy that the layer's beam plane made of it, so that nothing reads
+// what one work-group writes.  Bound by the launch on small planes and by the copy
+// on large ones; a launch for the residual, for each field and for the slice took
+// 18.0 us at 512^2 and 8.2 us at 64^2 (two fields), this one 4.7 and 2.9.
+struct LayerEndArgs {
+  const unsigned long long *rslots;
+  double *res;
+  long res_stride;
+  const double *src[QSS_NFIELD];
+  double *hist[QSS_NFIELD];
+  long n;                // nodes of a plane
+  int nf, nw, nslices, per_slice, slice;
+  int *slice_dev;        // replays only: {the next slice, to be set; this slice}
+};
+
+__device__ inline void layer_residual(const unsigned long long *r, double *dst) {
+  // one wave: max over the slots, lanes then shuffles; the bit patterns of
+  // non-negative doubles (and of +inf) order like the values
+  const int lane = threadIdx.x;
+  static_assert(kResidSlots % 64 == 0, "slots of a lane");
   unsigned long long m[6] = {0, 0, 0, 0, 0, 0};
-  for (int s = lane; s < kResidSlots; s += 64)
-    for (int q = 0; q < 6; ++q) m[q] = m[q] > r[s * 8 + q] ? m[q] : r[s * 8 + q];
+#pragma unroll
+  for (int s = 0; s < kResidSlots; s += 64)
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+      const unsigned long long v = r[(s + lane) * 8 + q];
+      m[q] = m[q] > v ? m[q] : v;
+    }
+#pragma unroll
   for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
     for (int q = 0; q < 6; ++q) {
       const unsigned long long v = __shfl_xor(m[q], o, 64);
       m[q] = m[q] > v ? m[q] : v;
     }
   if (lane != 0) return;
   double err = 0.0;
+#pragma unroll
   for (int c = 0; c < 3; ++c) {
     double dif = __longlong_as_double((long long)m[c]);
     double mx = __longlong_as_double((long long)m[3 + c]);
@@ -290,6 +310,42 @@ __global__ void k_resid_final(const unsigned long long *r, double *dst, int nw, 
     err = (e > err || e != e) ? e : err;
   }
   *dst = err;
+}
+
+// nodes per work-group of a copy: four 16-byte moves a thread, loaded together (into
+// vectors the compiler keeps in registers: as double2 the array went to LDS, 17 us)
+constexpr int kEndMoves = 4, kEndNodes = NT * 2 * kEndMoves;
+__global__ __launch_bounds__(NT) void k_layer_end(LayerEndArgs a) {
+  int slice = a.slice;
+  if (a.slice_dev) slice = a.slice_dev[1];
+  if (a.slice_dev && blockIdx.x == 0 && threadIdx.x == 0) a.slice_dev[0] = slice + 1;
+  if ((int)blockIdx.x < a.nw) {
+    const long w = blockIdx.x;
+    if (threadIdx.x < 64)
+      layer_residual(a.rslots + w * kResidPerWake,
+                     a.res + w * a.res_stride + (long)slice * a.per_slice);
+  } else {
+    const int per = (int)((a.n + kEndNodes - 1) / kEndNodes);   // work-groups of a plane
+    const int b = blockIdx.x - a.nw, fw = b / per;
+    const int w = fw / a.nf, f = fw - w * a.nf;
+    const long i0 = (long)(b - fw * per) * kEndNodes;
+    const double *src = a.src[f] + w * a.n;
+    double *dst = a.hist[f] + ((long)w * a.nslices + slice) * a.n;
+    if (a.n % 2 == 0) {   // planes and history start on 256 bytes
+      typedef double pair __attribute__((ext_vector_type(2)));
+      const pair *s2 = reinterpret_cast<const pair *>(src);
+      pair *d2 = reinterpret_cast<pair *>(dst);
+      const long i = i0 / 2 + threadIdx.x, n2 = a.n / 2, last = n2 - 1;
+      pair v[kEndMoves];
+#pragma unroll
+      for (int q = 0; q < kEndMoves; ++q) v[q] = s2[i + q * NT < n2 ? i + q * NT : last];
+#pragma unroll
+      for (int q = 0; q < kEndMoves; ++q)
+        if (i + q * NT < n2) d2[i + q * NT] = v[q];
+    } else {
+      for (long i = i0 + threadIdx.x; i < i0 + kEndNodes && i < a.n; i += NT) dst[i] = src[i];
+    }
+  }
 }
 
 // F = (P + C)/2 as 6 planes, for layers edited from the host; fp32 copy in
@@ -331,16 +387,6 @@ SpecArgs make_adj_args(qss_ctx *c, double *const *A, int flag) {
   SpecArgs a = make_args(c, flag);
   for (int s = 0; s < SP_N; ++s) a.S[s] = A[s];
   return a;
-}
-
-// history store inside a replayed graph: wake w's plane of `src` into
-// hist + (w * nslices + *slice_dev) * n
-__global__ void k_store_hist(const double *src, double *hist, long n, int nw, int nslices,
-                             const int *slice_dev) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n * nw) return;
-  const long w = i / n;
-  hist[(w * nslices + *slice_dev) * n + i % n] = src[i];
 }
 
 __global__ void k_add_i32(int *p, int v) {
@@ -438,17 +484,26 @@ hipError_t launch_iterate_update(qss_ctx *c, int final_pass) {
   return hipGetLastError();
 }
 
-hipError_t launch_residual_final(qss_ctx *c, double *dst) {
-  // capturing: dst is the slot of slice 0 and the slice is read at replay
-  hipLaunchKernelGGL(k_resid_final, dim3(c->nw), dim3(64), 0, c->stream,
-                     c->d_resid, dst, c->nw, (long)c->p.nslices * c->p.nx_split,
-                     c->capturing ? c->d_slice : nullptr, c->p.nx_split);
-  return hipGetLastError();
-}
-
-hipError_t launch_store_hist(qss_ctx *c, const double *src, double *hist) {
-  hipLaunchKernelGGL(k_store_hist, grid1(c->ncell * c->nw), dim3(NT), 0, c->stream, src, hist,
-                     c->ncell, c->nw, c->p.nslices, c->d_slice);
+hipError_t launch_layer_end(qss_ctx *c, int slice, double *res, const double *const *src,
+                            double *const *hist, int nf) {
+  LayerEndArgs a;
+  a.rslots = c->d_resid;
+  a.res = res;
+  a.res_stride = (long)c->p.nslices * c->p.nx_split;
+  for (int f = 0; f < nf; ++f) {
+    a.src[f] = src[f];
+    a.hist[f] = hist[f];
+  }
+  a.n = c->ncell;
+  a.nf = nf;
+  a.nw = c->nw;
+  a.nslices = c->p.nslices;
+  a.per_slice = c->capturing ? c->p.nx_split : 0;   // else res is the slice's own slot
+  a.slice = slice;
+  a.slice_dev = c->capturing ? c->d_slice : nullptr;
+  const long per = (a.n + kEndNodes - 1) / kEndNodes;
+  hipLaunchKernelGGL(k_layer_end, dim3((unsigned)(a.nw + per * nf * a.nw)), dim3(NT), 0, c->stream,
+                     a);
   return hipGetLastError();
 }
 

@@ -68,3 +68,18 @@ def test_graph_batched():
              [Bunch(nb=2.0, sigma_r=0.3, sigma_xi=0.3, xi0=0.5)]]
     p = small(ny=32, nz=32, nslices=15, bunches=list(wakes[0]), wakes=wakes)
     same(sweep(p, False), sweep(p, True))
+
+
+@pytest.mark.parametrize("ny,nz,nw,prec", [
+    (17, 19, 1, "fp64"),     # odd plane: single nodes
+    (34, 37, 1, "fp64"),     # even plane, one copy work-group
+    (48, 32, 3, "fp64"),     # the same, of three wakes
+    (64, 48, 2, "fp64"),     # two work-groups per plane, the second half full
+    (48, 48, 1, "bf16x6")])
+def test_layer_end_in_replays(ny, nz, nw, prec):
+    """The residuals and every kept plane that a replay writes, and the slice it moves
+    on to, for plane sizes on both sides of the layer end's moves."""
+    wakes = [[Bunch(nb=0.5 + w, sigma_r=0.5, sigma_xi=0.3, xi0=0.3)] for w in range(nw)]
+    p = small(ny=ny, nz=nz, nslices=14, precision=PRECISIONS[prec], bunches=list(wakes[0]),
+              wakes=wakes if nw > 1 else [])
+    same(sweep(p, False), sweep(p, True))
