@@ -25,7 +25,7 @@
 //
 // Full step: the pushed particle is staged with its destination tile
 // direction and its rank among the tile's particles going that way (slot
-// order); k_tile_scan / k_permute rebuild the tile-sorted storage: each
+// order); tile_scan / k_permute rebuild the tile-sorted storage: each
 // destination tile holds the groups from its 9 source directions in a fixed
 // order, each group in source slot order.  The storage order, and so every
 // summation order, is a pure function of the input.
@@ -73,7 +73,7 @@ struct TileArgs {
   // full step staging (indexed by the old slot)
   double *sy, *sz, *spx, *spy, *spz;
   int32_t *scell, *sdest;  // sdest = direction | rank << 4
-  int32_t *tcount;         // ntiles x nsplit x 9
+  int32_t *tcount;         // 9 directions x nsplit x ntiles
   int32_t *counters;
   long npw;                // particle slots per wake (batched contexts)
   int nsplit;              // work-groups per tile (each takes every nsplit-th chunk)
@@ -632,7 +632,86 @@ void k_push_tile(TileArgs a0) {
   double4 *wout = reinterpret_cast<double4 *>(a.win + (long)blockIdx.x * NWIN * 4);
   for (int i = t; i < NWIN; i += NT)
     wout[i] = make_double4(wacc[0][i], wacc[1][i], wacc[2][i], RHO ? wacc[NQ - 1][i] : 0.0);
-  if (FULL && t < 9) a.tcount[blockIdx.x * 9 + t] = dir_total[t];
+  if (FULL && t < 9)
+    a.tcount[(t * a.nsplit + part) * (a.ntj * a.ntk) + tile] = dir_total[t];
+}
+
+// New tile starts and group offsets: destination tile u receives the groups
+// of source tiles u - dir(d) for d = 0..8 in that order, each as the groups
+// of the source's parts 0..NS-1.  One work-group per wake takes one or two tiles a
+// thread at a time (as many as the combine's registers allow), all loads together; counts and
+// offsets are stored direction by direction, so that neighbouring lanes read
+// neighbouring tiles.  It depends on the push only, as the combine does, and takes
+// less time than a plane's combine at every size (per 1024 tiles 2.5 us against
+// 5.6), so it is that launch's first work-group: by itself it was 3.6 us at 64^2,
+// 9.5 at 256^2 (four parts) and 6.6 at 512^2.
+template <int NS>
+__device__ inline void tile_scan(const int32_t *tcount, int ntj, int ntk, int32_t *tile_start,
+                                 int32_t *goff) {
+  constexpr int B = NS == 1 ? 2 : 1, NG = 9 * NS, NW = NT / 64;
+  __shared__ int wsum[B][NW];
+  const int nt = ntj * ntk;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  int carry = 0;
+  for (int b0 = 0; b0 < nt; b0 += NT * B) {
+    int g[B][NG], tot[B], incl[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const int u = b0 + b * NT + (int)threadIdx.x;
+      tot[b] = 0;
+      const int uu = u < nt ? u : 0;
+      const int uk = uu / ntj, uj = uu - uk * ntj;
+#pragma unroll
+      for (int d = 0; d < 9; ++d) {
+        int sj = uj - (d % 3 - 1), sk = uk - (d / 3 - 1);
+        sj = sj < 0 ? sj + ntj : (sj >= ntj ? sj - ntj : sj);
+        sk = sk < 0 ? sk + ntk : (sk >= ntk ? sk - ntk : sk);
+#pragma unroll
+        for (int q = 0; q < NS; ++q) {
+          const int v = tcount[(d * NS + q) * nt + sk * ntj + sj];
+          g[b][d * NS + q] = u < nt ? v : 0;
+        }
+      }
+    }
+    // exclusive scan over the tiles: inclusive scans within each wave, then
+    // the totals of the waves before this one (integer sums: exact)
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+#pragma unroll
+      for (int e = 0; e < NG; ++e) tot[b] += g[b][e];
+      incl[b] = tot[b];
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(incl[b], o, 64);
+        if (lane >= o) incl[b] += v;
+      }
+      if (lane == 63) wsum[b][wv] = incl[b];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const int u = b0 + b * NT + (int)threadIdx.x;
+      int before = 0, all = 0;
+#pragma unroll
+      for (int q = 0; q < NW; ++q) {
+        const int v = wsum[b][q];
+        before += q < wv ? v : 0;
+        all += v;
+      }
+      int o = carry + before + incl[b] - tot[b];
+      if (u < nt) {
+        tile_start[u] = o;
+#pragma unroll
+        for (int e = 0; e < NG; ++e) {
+          goff[e * nt + u] = o;
+          o += g[b][e];
+        }
+      }
+      carry += all;
+    }
+    __syncthreads();   // wsum is rewritten by the next tiles
+  }
+  if (threadIdx.x == 0) tile_start[nt] = carry;
 }
 
 // sum of the windows covering each node, fixed (dtk, dtj, part) order.  Per
@@ -644,7 +723,8 @@ void k_push_tile(TileArgs a0) {
 // unchanged (the sum starts at +0.0, so it is never -0.0).
 // xs0..xs2 (split-bf16 modes, one wake): Jx, Jy, Jz also written as the split
 // operands of the forward transform that follows.
-// grid: (node blocks of one plane, wakes); 32-bit node index (ny, nz <= 2^14)
+// grid: (node blocks of one plane, wakes); 32-bit node index (ny, nz <= 2^14); with
+// tcount one more work-group, the first, does the full step's tile scan
 static_assert(W - T - H <= T - H, "at most two tiles per axis cover a node");
 // RHO = false: the density plane J3 is neither summed nor written
 template <int NS, bool RHO>
@@ -652,9 +732,17 @@ __global__ __launch_bounds__(NT) void k_combine(const double *win, int ntj, int 
                                                 int nz, uint64_t ny_magic, double *J0,
                                                 double *J1, double *J2, double *J3,
                                                 uint16_t *xs0, uint16_t *xs1, uint16_t *xs2,
-                                                int npc) {
+                                                int npc, const int32_t *tcount,
+                                                int32_t *tile_start, int32_t *goff) {
+  int block = blockIdx.x;
+  if (tcount && block-- == 0) {
+    const long nt = (long)ntj * ntk, w = blockIdx.y;
+    tile_scan<NS>(tcount + w * nt * NS * 9, ntj, ntk, tile_start + w * (nt + 1),
+                  goff + w * nt * NS * 9);
+    return;
+  }
   const int plane = ny * nz;
-  const int n1 = blockIdx.x * NT + threadIdx.x;   // node of the wake's plane
+  const int n1 = block * NT + threadIdx.x;   // node of the wake's plane
   if (n1 >= plane) return;
   const double4 *w4 = reinterpret_cast<const double4 *>(win) +
                       (long)blockIdx.y * ntj * ntk * NS * NWIN;   // the wake's windows
@@ -710,75 +798,6 @@ __global__ __launch_bounds__(NT) void k_combine(const double *win, int ntj, int 
   }
 }
 
-// new tile starts and group offsets: destination tile u receives the groups
-// of source tiles u - dir(d) for d = 0..8 in that order, each as the groups
-// of the source's parts 0..nsplit-1.  One 1024-thread work-group per wake:
-// a thread holds one destination tile's 9 x nsplit counts in registers.
-constexpr int NTS = 1024;
-__global__ __launch_bounds__(NTS) void k_tile_scan(const int32_t *tcount, int ntj, int ntk,
-                                                   int nsplit, int32_t *tile_start,
-                                                   int32_t *goff) {
-  __shared__ int wsum[NTS / 64];
-  const int nt = ntj * ntk;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int w = blockIdx.x;   // one work-group per wake
-  tcount += (long)w * nt * nsplit * 9;
-  goff += (long)w * nt * nsplit * 9;
-  tile_start += (long)w * (nt + 1);
-  int carry = 0;
-  for (int b0 = 0; b0 < nt; b0 += NTS) {
-    const int u = b0 + threadIdx.x;
-    int tot = 0;
-    int g[9][kMaxSplit];
-    if (u < nt) {
-      const int uj = u % ntj, uk = u / ntj;
-#pragma unroll
-      for (int d = 0; d < 9; ++d) {
-        const int dj = d % 3 - 1, dk = d / 3 - 1;
-        const int src = wrapi(uk - dk, ntk) * ntj + wrapi(uj - dj, ntj);
-#pragma unroll
-        for (int q = 0; q < kMaxSplit; ++q) {
-          g[d][q] = q < nsplit ? tcount[(src * nsplit + q) * 9 + d] : 0;
-          tot += g[d][q];
-        }
-      }
-    }
-    // block exclusive scan of tot: inclusive scans within each wave, then
-    // the totals of the waves before this one (integer sums: exact)
-    int incl = tot;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += v;
-    }
-    if (lane == 63) wsum[wv] = incl;
-    __syncthreads();
-    int before = 0, blk_tot = 0;
-#pragma unroll
-    for (int q = 0; q < NTS / 64; ++q) {
-      const int v = wsum[q];
-      before += q < wv ? v : 0;
-      blk_tot += v;
-    }
-    const int start = carry + before + incl - tot;
-    if (u < nt) {
-      tile_start[u] = start;
-      int o = start;
-#pragma unroll
-      for (int d = 0; d < 9; ++d)
-#pragma unroll
-        for (int q = 0; q < kMaxSplit; ++q)
-          if (q < nsplit) {
-            goff[(u * 9 + d) * nsplit + q] = o;
-            o += g[d][q];
-          }
-    }
-    __syncthreads();   // wsum is rewritten by the next block of tiles
-    carry += blk_tot;
-  }
-  if (threadIdx.x == 0) tile_start[nt] = carry;
-}
-
 __global__ __launch_bounds__(NT) void k_permute(TileArgs a0, const int32_t *goff, long np,
                                                 int nw, double *y, double *z, double *px,
                                                 double *py, double *pz, int32_t *cell,
@@ -796,7 +815,8 @@ __global__ __launch_bounds__(NT) void k_permute(TileArgs a0, const int32_t *goff
   cell_jk(c, a.ny, a.ny_magic, cj, ck);
   const int dst_tile = (ck / T) * a.ntj + cj / T;
   const int sd = a.sdest[s];   // direction | part << 4 | rank << 8
-  const long o = goff[(dst_tile * 9 + (sd & 15)) * a.nsplit + ((sd >> 4) & 15)] + (sd >> 8);
+  const int group = (sd & 15) * a.nsplit + ((sd >> 4) & 15);
+  const long o = goff[group * (a.ntj * a.ntk) + dst_tile] + (sd >> 8);
   y[o] = a.sy[s];
   z[o] = a.sz[s];
   px[o] = a.spx[s];
@@ -909,7 +929,7 @@ hipError_t launch_push_tile(qss_ctx *c, int full, bool rho, hipEvent_t ev0, hipE
   return hipGetLastError();
 }
 
-hipError_t launch_combine(qss_ctx *c, bool rho, double *const *out) {
+hipError_t launch_combine(qss_ctx *c, bool rho, double *const *out, bool scan) {
   double *const J[4] = {c->C[QSS_JX], c->C[QSS_JY], c->C[QSS_JZ], c->C[QSS_RHO]};
   const bool split = c->npc && !out;   // sweep deposits only (not the tuning runs)
   if (!out) out = J;
@@ -923,18 +943,15 @@ hipError_t launch_combine(qss_ctx *c, bool rho, double *const *out) {
                    : c->nsplit == 2 ? k_combine<2, false>
                                     : k_combine<4, false>);
   if (c->nsplit != 1 && c->nsplit != 2 && c->nsplit != 4) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(fn, dim3(grid1(c->ncell).x, c->nw), dim3(NT), 0, c->stream, c->win,
-                     c->ntj, c->ntk, c->ny, c->nz, ny_magic, out[0], out[1], out[2], out[3],
-                     c->xs[0], c->xs[1], c->xs[2], split ? c->npc : 0);
+  hipLaunchKernelGGL(fn, dim3(grid1(c->ncell).x + (scan ? 1 : 0), c->nw), dim3(NT), 0, c->stream,
+                     c->win, c->ntj, c->ntk, c->ny, c->nz, ny_magic, out[0], out[1], out[2], out[3],
+                     c->xs[0], c->xs[1], c->xs[2], split ? c->npc : 0,
+                     scan ? c->tcount : nullptr, c->tile_start[c->cur ^ 1], c->goff);
   return hipGetLastError();
 }
 
 hipError_t launch_tile_reorder(qss_ctx *c) {
   const int nb = c->cur ^ 1;
-  hipLaunchKernelGGL(k_tile_scan, dim3(c->nw), dim3(NTS), 0, c->stream, c->tcount, c->ntj,
-                     c->ntk, c->nsplit, c->tile_start[nb], c->goff);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_permute, grid1(c->np * c->nw), dim3(NT), 0, c->stream, make_args(c, 1),
                      c->goff, c->np, c->nw, c->py_[nb], c->pz_[nb], c->ppx[nb], c->ppy[nb],
                      c->ppz[nb], c->pcell[nb], c->pid[nb]);

@@ -506,7 +506,7 @@ int do_push_deposit(qss_ctx *c, int full) {
     }
     {
       Timed t(c, KC_REDUCE);
-      HIPCHECK(launch_combine(c, c->deposit_rho));
+      HIPCHECK(launch_combine(c, c->deposit_rho, nullptr, full));
       if (full) HIPCHECK(launch_tile_reorder(c));
     }
     if (full) c->cur ^= 1;

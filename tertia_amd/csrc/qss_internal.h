@@ -357,8 +357,8 @@ struct qss_ctx {
   bool skip_rho_psi = false;     // inside a sweep: final passes leave rho, psi
   int32_t *tile_start[2] = {};   // ping-pong with the particle arrays
   double *win = nullptr;         // ntiles x nsplit x 441 x 4 deposit windows
-  int32_t *tcount = nullptr;     // ntiles x nsplit x 9 full-step direction counts
-  int32_t *goff = nullptr;       // ntiles x 9 x nsplit group offsets
+  int32_t *tcount = nullptr;     // 9 x nsplit x ntiles full-step direction counts
+  int32_t *goff = nullptr;       // 9 x nsplit x ntiles group offsets
 
   unsigned long long *d_resid = nullptr;   // kResidPerWake per wake and pass
   double *d_res_hist = nullptr;            // residual of each layer step
@@ -445,7 +445,8 @@ hipError_t launch_push_field(qss_ctx *c);
 hipError_t launch_push_tile(qss_ctx *c, int full, bool rho, hipEvent_t ev0 = nullptr,
                             hipEvent_t ev1 = nullptr);
 // out (optional): 4 destination planes instead of the C-layer Jx, Jy, Jz, Rho
-hipError_t launch_combine(qss_ctx *c, bool rho, double *const *out = nullptr);
+// scan: a full push's tile scan too, which launch_tile_reorder then needs
+hipError_t launch_combine(qss_ctx *c, bool rho, double *const *out = nullptr, bool scan = false);
 hipError_t launch_tile_reorder(qss_ctx *c);
 hipError_t launch_seed_tiled(qss_ctx *c);
 hipError_t launch_axpy(double *y, const double *x, double a, long n, hipStream_t s,

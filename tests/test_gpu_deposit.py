@@ -64,3 +64,41 @@ def test_deposit_cell_counts(oracle_mod, shape, rows, per_cell, hot):
             assert np.array_equal(a, b)
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("ny,nz,nsplit", [
+    (16, 16, 1), (32, 16, 2), (16, 48, 4),   # one, two and three tiles on an axis
+    (256, 256, 4), (272, 256, 2),            # one full round of the scan, and one tile row more
+    (368, 368, 1)])                          # two rounds of two tiles a thread
+def test_reorder_scan_edges(oracle_mod, ny, nz, nsplit):
+    """The tile scan that rides on the combine's launch: every particle keeps its id,
+    cell, position and momentum through two reorders (bars of the push tests), and
+    the second full step, which reads the storage the first one wrote, deposits what
+    the oracle does."""
+    from tertia_amd.mesh import Mesh
+    rng = np.random.default_rng(ny + nz + nsplit)
+    p = small(ny=ny, nz=nz, nslices=2, hx=0.4, ppc_y=1, ppc_z=1)
+    n = ny * nz
+    cell = np.sort(rng.integers(0, n, size=n))
+    parts = ((cell % ny).astype(np.int32), (cell // ny).astype(np.int32),
+             rng.uniform(0, 1, n), rng.uniform(0, 1, n), *rng.uniform(-0.8, 0.8, size=(3, n)),
+             np.arange(n, dtype=np.int64))
+    m, o = Mesh(p, history=()), oracle_mod.Oracle(p, history=())
+    try:
+        m.particle_split = nsplit
+        o.set_particles(*parts)
+        m.set_particles(*parts)
+        for _ in range(2):
+            o.push_deposit(1)
+            m.MoveParticlesLayerSplit(0, 0, 1)
+            for f in ("Jx", "Jy", "Jz", "Rho"):
+                assert max_rel(m.get_field(f), o.get_field(f)) <= 1e-13
+        po, pg = o.particles(), m.particles()
+        oo, og = np.argsort(po["id"]), np.argsort(pg["id"])
+        for k in ("id", "cj", "ck"):
+            assert np.array_equal(po[k][oo], pg[k][og]), k
+        for k in ("fy", "fz", "px", "py", "pz"):
+            bar = 1e-14 * (max(ny, nz) if k in ("fy", "fz") else max(1.0, np.abs(po[k]).max()))
+            assert np.abs(po[k][oo] - pg[k][og]).max() <= bar, k
+    finally:
+        m.close()
