@@ -41,14 +41,133 @@ __device__ inline int wrapi(int a, int n) {
   return a < 0 ? a + n : a;
 }
 
+using qss_tile::kCell;
+
+// The six field adjoints of one cell's events over its four nodes, in the order of
+// the events' indices.
+template <int N>
+__device__ inline void cell_sums(uint2 bytes, int n, const double (*ev_f)[NT],
+                                 const double (*ev_w)[NT], double (*s)[6]) {
+  int e[N];
+  qss_tile::cell_order<N>(bytes, n, e);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if (i >= n) break;
+    const int ei = e[i];
+    double f[6];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) f[q] = ev_f[q][ei];
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn) {
+      const double w = ev_w[cn][ei];
+#pragma unroll
+      for (int q = 0; q < 6; ++q) s[cn][q] += w * f[q];
+    }
+  }
+}
+
+// Transposed gather of a chunk by cells: a tile's 256 cells are one per lane; its
+// owner sums a cell's events over the four corners in registers, and the corners
+// are added to the window's node sums in turns (in one corner's turn no two cells
+// share a node).  Cells are dealt to the waves in turn.  Leaves the counts at zero.
+__device__ inline void scatter_cells(int *cnt, const uint2 *list, const double (*ev_f)[NT],
+                                     const double (*ev_w)[NT], double (*acc)[NF]) {
+  static_assert(T * T == NT, "a cell per lane");
+  const int t = qss_tile::thread_index();
+  const int cell = 4 * (t & 63) + (t >> 6);
+  const int n = cnt[cell];
+  double s[4][6] = {};
+  if (n) {
+    cnt[cell] = 0;
+    const uint2 bytes = list[cell];
+    if (n <= 4) cell_sums<4>(bytes, n, ev_f, ev_w, s);
+    else cell_sums<8>(bytes, n, ev_f, ev_w, s);
+  }
+#pragma unroll
+  for (int cn = 0; cn < 4; ++cn) {
+    if (n) {
+      const int node = (cell % T + (cn & 1)) + FW * (cell / T + (cn >> 1));
+#pragma unroll
+      for (int q = 0; q < 6; ++q) acc[q][node] += s[cn][q];
+    }
+    __syncthreads();
+  }
+}
+
+// A chunk with more than kCell events in some cell: the events sorted by cell and
+// index, every node summing the runs of its four cells.
+__device__ inline void scatter_sorted(int cell, int *keys, int *sorted, short *cstart, short *cend,
+                                      double (*ev_f)[NT], double (*ev_w)[NT], double (*acc)[NF]) {
+  const int t = qss_tile::thread_index();
+  for (int i = t; i < T * T; i += NT) { cstart[i] = 0; cend[i] = 0; }
+  const int sk = qss_tile::sort256(cell < 0 ? kInvalid : cell << 8 | t, keys);
+  sorted[t] = sk;
+  // the event at sorted position t, moved there in place: gathered before the
+  // barrier (the sort's barriers made every event visible), stored after it
+  double gf[6], gw[4];
+  if (sk != kInvalid) {
+    const int e = sk & 255;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) gf[q] = ev_f[q][e];
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn) gw[cn] = ev_w[cn][e];
+  }
+  __syncthreads();
+  if (sk != kInvalid) {
+#pragma unroll
+    for (int q = 0; q < 6; ++q) ev_f[q][t] = gf[q];
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn) ev_w[cn][t] = gw[cn];
+    const int cl = sk >> 8;
+    const int prev = t > 0 ? sorted[t - 1] : kInvalid;
+    const int next = t + 1 < NT ? sorted[t + 1] : kInvalid;
+    if (t == 0 || (prev >> 8) != cl) cstart[cl] = (short)t;
+    if (next == kInvalid || (next >> 8) != cl) cend[cl] = (short)(t + 1);
+  }
+  __syncthreads();
+  for (int n = t; n < NF; n += NT) {
+    double a[6];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) a[q] = acc[q][n];
+    const int nl_j = n % FW, nl_k = n / FW;
+#pragma unroll 1
+    for (int cn = 0; cn < 4; ++cn) {
+      const int cj = nl_j - (cn & 1), ck = nl_k - (cn >> 1);
+      if (cj < 0 || ck < 0 || cj >= T || ck >= T) continue;
+      const int cl = ck * T + cj, e1 = cend[cl];
+      for (int e = cstart[cl]; e < e1; ++e) {
+        const double w = ev_w[cn][e];
+#pragma unroll
+        for (int q = 0; q < 6; ++q) a[q] += w * ev_f[q][e];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 6; ++q) acc[q][n] = a[q];
+  }
+}
+
+// Bound by FP64 issue and latency at two work-groups per CU (62 KB of LDS, 256
+// registers): some 900 FP64 operations a particle, the adjoints of its state read
+// and written by id (asked for before the push, whose time hides them).  256^2, 4 per
+// cell: 52.9 us with every chunk sorted, a division for each quotient and the node
+// sums in HBM between chunks; 31.1 like this.
 __global__ __launch_bounds__(NT) void k_push_tile_adj(AdjTileArgs a) {
-  __shared__ double Fw[NF * 6];
-  __shared__ double Jw[NWIN * 3];
-  __shared__ int keys_sh[NT];
-  __shared__ int sorted[NT];
-  __shared__ double ev_f[NT * 6];
-  __shared__ double ev_w[NT * 4];
-  __shared__ short cstart[T * T], cend[T * T];
+  __shared__ double Fw[6][NF];
+  __shared__ double Jw[3][NWIN];
+  __shared__ double acc[6][NF];   // the window's node sums
+  __shared__ double ev_f[6][NT], ev_w[4][NT];
+  // the chunk's events of each cell, or the sort's arrays of a crowded chunk
+  __shared__ union {
+    struct {
+      int cnt[T * T];
+      uint2 list[T * T];
+    } cell;
+    struct {
+      int keys[NT], sorted[NT];
+      short cstart[T * T], cend[T * T];
+    } sort;
+  } sh;
+  __shared__ int crowded_sh[2];   // one is cleared while the other is in use
 
   const int t = threadIdx.x;
   // a tile's particles shared by nsplit work-groups, as in the forward push
@@ -58,22 +177,26 @@ __global__ __launch_bounds__(NT) void k_push_tile_adj(AdjTileArgs a) {
   const int ny = a.ny, nz = a.nz;
   const long plane = (long)ny * nz;
 
+  // a window index lies less than one period outside the plane (ny, nz >= T)
+  const auto wrap1 = [](int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); };
   for (int i = t; i < NF; i += NT) {
     const int lj = i % FW, lk = i / FW;
-    const long g = wrapi(j0 + lj, ny) + (long)ny * wrapi(k0 + lk, nz);
+    const long g = wrap1(j0 + lj, ny) + (long)ny * wrap1(k0 + lk, nz);
 #pragma unroll
-    for (int q = 0; q < 6; ++q) Fw[i * 6 + q] = a.F[q * plane + g];
+    for (int q = 0; q < 6; ++q) {
+      Fw[q][i] = a.F[q * plane + g];
+      acc[q][i] = 0.0;
+    }
   }
   for (int i = t; i < NWIN; i += NT) {
     const int lj = i % W, lk = i / W;
-    const long g = wrapi(j0 - H + lj, ny) + (long)ny * wrapi(k0 - H + lk, nz);
+    const long g = wrap1(j0 - H + lj, ny) + (long)ny * wrap1(k0 - H + lk, nz);
 #pragma unroll
-    for (int q = 0; q < 3; ++q) Jw[i * 3 + q] = a.Jb[q * plane + g];
+    for (int q = 0; q < 3; ++q) Jw[q][i] = a.Jb[q * plane + g];
   }
-  // this work-group's window: chunk sums written by the first chunk, added
-  // by later ones (each thread owns nodes t and t + NT)
-  double *wout = a.fwin + (long)blockIdx.x * NF * 6;
-  bool first = true;
+  sh.cell.cnt[t] = 0;
+  if (t < 2) crowded_sh[t] = 0;
+  int par = 0;
   __syncthreads();
 
   qss_adj::Consts cs;
@@ -86,10 +209,18 @@ __global__ __launch_bounds__(NT) void k_push_tile_adj(AdjTileArgs a) {
   const int npt = a.tile_start[tile + 1] - base;
   for (int c0 = part * NT; c0 < npt; c0 += a.nsplit * NT) {
     const int slot = base + c0 + t;
-    int key = kInvalid;
+    int cellw = -1;
     if (c0 + t < npt) {
+      const long id = a.pid[slot];
+      // full step: the adjoint of the new position (0, 1) and momentum (2..4);
+      // else what the passes before have left of the start state's.  Asked for
+      // here, used after the push.
+      double nb[5];
+      const double *const from = a.full ? a.pin : a.pout;
+#pragma unroll
+      for (int i = 0; i < 5; ++i) nb[i] = from[i * np + id];
       const int32_t c = a.cell[slot];
-      const int j = c % ny, k = c / ny;
+      const int k = c / ny, j = c - k * ny;
       int lj = j - j0, lk = k - k0;
       if (lj < 0 || lj >= T || lk < 0 || lk >= T) {
         atomicOr(&a.counters[1], ST_FAR);
@@ -98,10 +229,8 @@ __global__ __launch_bounds__(NT) void k_push_tile_adj(AdjTileArgs a) {
       }
       const double y0 = a.y[slot], z0 = a.z[slot];
       const double P0[3] = {a.px[slot], a.py[slot], a.pz[slot]};
-      const long id = a.pid[slot];
-      // adjoint of the new position (0, 1) and momentum (2..4), full step only
-      auto NB = [&](int i) { return a.pin[i * np + id]; };
-      auto Fn = [&](int q, int dj, int dk) { return Fw[((lj + dj) + FW * (lk + dk)) * 6 + q]; };
+      auto NB = [&](int i) { return nb[i]; };
+      auto Fn = [&](int q, int dj, int dk) { return Fw[q][(lj + dj) + FW * (lk + dk)]; };
       bool far = false;
       auto JBn = [&](int q, int nj, int nk) -> double {
         if (q > 2) return 0.0;   // the deposited density is not transformed
@@ -114,86 +243,42 @@ __global__ __launch_bounds__(NT) void k_push_tile_adj(AdjTileArgs a) {
           far = true;
           return 0.0;
         }
-        return Jw[((dk + H) * W + dj + H) * 3 + q];
+        return Jw[q][(dk + H) * W + dj + H];
       };
       qss_adj::AdjOut o;
       qss_adj::push_adjoint_cb(cs, j, k, y0, z0, P0, Fn, JBn, a.full != 0, NB, o);
       if (far) atomicOr(&a.counters[1], ST_FAR);
-      if (a.full) {
-        a.pout[id] = o.y0;
-        a.pout[np + id] = o.z0;
-        a.pout[2 * np + id] = o.P0[0];
-        a.pout[3 * np + id] = o.P0[1];
-        a.pout[4 * np + id] = o.P0[2];
-      } else {
-        a.pout[id] += o.y0;
-        a.pout[np + id] += o.z0;
-        a.pout[2 * np + id] += o.P0[0];
-        a.pout[3 * np + id] += o.P0[1];
-        a.pout[4 * np + id] += o.P0[2];
-      }
+      const double out[5] = {o.y0, o.z0, o.P0[0], o.P0[1], o.P0[2]};
 #pragma unroll
-      for (int q = 0; q < 6; ++q) ev_f[t * 6 + q] = o.f[q];
+      for (int i = 0; i < 5; ++i) a.pout[i * np + id] = a.full ? out[i] : nb[i] + out[i];
 #pragma unroll
-      for (int cn = 0; cn < 4; ++cn) ev_w[t * 4 + cn] = o.w[cn];
-      key = ((lk * T + lj) << 8) | t;
-    }
-    // transposed gather: every node sums the events of its four cells
-    for (int i = t; i < T * T; i += NT) { cstart[i] = 0; cend[i] = 0; }
-    const int sk = qss_tile::sort256(key, keys_sh);
-    sorted[t] = sk;
-    // the event at sorted position t, moved there in place: gathered before the
-    // barrier (the sort's barriers made every event visible), stored after it
-    double gf[6], gw[4];
-    if (sk != kInvalid) {
-      const int e = sk & 255;
+      for (int q = 0; q < 6; ++q) ev_f[q][t] = o.f[q];
 #pragma unroll
-      for (int q = 0; q < 6; ++q) gf[q] = ev_f[e * 6 + q];
-#pragma unroll
-      for (int cn = 0; cn < 4; ++cn) gw[cn] = ev_w[e * 4 + cn];
+      for (int cn = 0; cn < 4; ++cn) ev_w[cn][t] = o.w[cn];
+      cellw = lk * T + lj;
+      const int r = atomicAdd(&sh.cell.cnt[cellw], 1);
+      if (r < kCell) reinterpret_cast<uint8_t *>(&sh.cell.list[cellw])[r] = (uint8_t)t;
+      else crowded_sh[par] = 1;
     }
     __syncthreads();
-    if (sk != kInvalid) {
-#pragma unroll
-      for (int q = 0; q < 6; ++q) ev_f[t * 6 + q] = gf[q];
-#pragma unroll
-      for (int cn = 0; cn < 4; ++cn) ev_w[t * 4 + cn] = gw[cn];
-      const int cl = sk >> 8;
-      const int prev = t > 0 ? sorted[t - 1] : kInvalid;
-      const int next = t + 1 < NT ? sorted[t + 1] : kInvalid;
-      if (t == 0 || (prev >> 8) != cl) cstart[cl] = (short)t;
-      if (next == kInvalid || (next >> 8) != cl) cend[cl] = (short)(t + 1);
+    const bool crowded = crowded_sh[par];
+    par ^= 1;
+    if (t == 0) crowded_sh[par] = 0;   // last read a barrier ago
+    if (crowded) {
+      __syncthreads();   // the lists give way to the sort
+      scatter_sorted(cellw, sh.sort.keys, sh.sort.sorted, sh.sort.cstart, sh.sort.cend, ev_f, ev_w,
+                     acc);
+      __syncthreads();
+      sh.cell.cnt[t] = 0;
+      __syncthreads();
+    } else {
+      scatter_cells(sh.cell.cnt, sh.cell.list, ev_f, ev_w, acc);
     }
-    __syncthreads();
-#pragma unroll
-    for (int oi = 0; oi < 2; ++oi) {
-      const int n = t + oi * NT;
-      if (n >= NF) continue;
-      double accn[6] = {0, 0, 0, 0, 0, 0};
-      const int nl_j = n % FW, nl_k = n / FW;
-#pragma unroll
-      for (int cn = 0; cn < 4; ++cn) {
-        const int cj = nl_j - (cn & 1), ck = nl_k - (cn >> 1);
-        if (cj < 0 || ck < 0 || cj >= T || ck >= T) continue;
-        const int cl = ck * T + cj;
-        const int e1 = cend[cl];
-        for (int i = cstart[cl]; i < e1; ++i) {
-          const int e = i;   // events are stored in sorted order
-          const double wv = ev_w[e * 4 + cn];
-#pragma unroll
-          for (int q = 0; q < 6; ++q) accn[q] += wv * ev_f[e * 6 + q];
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < 6; ++q) wout[n * 6 + q] = first ? accn[q] : wout[n * 6 + q] + accn[q];
-    }
-    first = false;
-    __syncthreads();
   }
-  if (first)   // no particles for this work-group
-    for (int n = t; n < NF; n += NT)
+  double *const wout = a.fwin + (long)blockIdx.x * NF * 6;
+  for (int n = t; n < NF; n += NT)
 #pragma unroll
-      for (int q = 0; q < 6; ++q) wout[n * 6 + q] = 0.0;
+    for (int q = 0; q < 6; ++q) wout[n * 6 + q] = acc[q][n];
 }
 
 // out[q][node] = sum of the 17x17 windows holding the node, fixed order

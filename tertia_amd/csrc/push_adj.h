@@ -27,11 +27,7 @@
 
 #include <math.h>
 
-#ifdef __HIPCC__
-#define QSS_HD __host__ __device__
-#else
-#define QSS_HD
-#endif
+#include "inv_gamma.h"
 
 namespace qss_adj {
 
@@ -57,10 +53,10 @@ QSS_HD inline void cic_weights(double y, double z, double w[4], double wy[4], do
 
 // forward intermediates of the momentum update of one particle
 struct Kin {
-  double P0[3], g0, Vp[3];
+  double P0[3], ig0, Vp[3];   // ig0, ig1, ig2: 1/gamma at P0, H and P1
   double fE[3], fB[3];
-  double e[3], u, K[3], H[3], g1, beta, b[3], co, Q[3], p3[3], R[3], P1[3], g2, Vm[3];
-  double Vb[3], v, dj[4], d[2];
+  double e[3], iu, K[3], H[3], ig1, beta, b[3], co, Q[3], p3[3], R[3], P1[3], ig2, Vm[3];
+  double Vb[3], iv, dj[4], d[2];   // iu = 1 / (1 - Vp_x), iv = 1 / (1 - Vb_x)
   double s;    // sub-step divisor (1: no sub-cycling)
   int nsub;    // number of sub-steps
   bool frozen; // displacement zeroed by the sub-step guard
@@ -73,17 +69,14 @@ QSS_HD inline void kinematics(const Consts &c, const double P0[3], const double 
   const double q2m = kQ2m, hx = c.hx;
   for (int q = 0; q < 3; ++q) k.P0[q] = P0[q];
   const double px = P0[0], py = P0[1], pz = P0[2];
-  k.g0 = sqrt(1. + px * px + py * py + pz * pz);
-  const double ig0 = 1. / k.g0;
+  const double ig0 = k.ig0 = inv_gamma(px, py, pz);
   k.Vp[0] = px * ig0; k.Vp[1] = py * ig0; k.Vp[2] = pz * ig0;
   for (int q = 0; q < 3; ++q) { k.fE[q] = f[q]; k.fB[q] = f[3 + q] + c.bext[q]; }
   for (int q = 0; q < 3; ++q) k.e[q] = f[q] * (q2m * hx / 2.);
-  k.u = 1. - k.Vp[0];
-  const double iu = 1. / k.u;
+  const double iu = k.iu = 1. / (1. - k.Vp[0]);
   for (int q = 0; q < 3; ++q) k.K[q] = k.e[q] * iu;
   for (int q = 0; q < 3; ++q) k.H[q] = P0[q] + k.K[q];
-  k.g1 = sqrt(1. + k.H[0] * k.H[0] + k.H[1] * k.H[1] + k.H[2] * k.H[2]);
-  const double gr = 1. / k.g1;
+  const double gr = k.ig1 = inv_gamma(k.H[0], k.H[1], k.H[2]);
   k.beta = gr * q2m * iu * (0.5 * hx);
   for (int q = 0; q < 3; ++q) k.b[q] = k.fB[q] * k.beta;
   const double *b = k.b, *H = k.H;
@@ -96,12 +89,10 @@ QSS_HD inline void kinematics(const Consts &c, const double P0[3], const double 
   k.R[1] = k.p3[2] * b[0] - k.p3[0] * b[2];
   k.R[2] = k.p3[0] * b[1] - k.p3[1] * b[0];
   for (int q = 0; q < 3; ++q) k.P1[q] = H[q] + (k.K[q] + k.R[q]);
-  k.g2 = sqrt(1. + k.P1[0] * k.P1[0] + k.P1[1] * k.P1[1] + k.P1[2] * k.P1[2]);
-  const double ig2 = 1. / k.g2;
+  const double ig2 = k.ig2 = inv_gamma(k.P1[0], k.P1[1], k.P1[2]);
   for (int q = 0; q < 3; ++q) k.Vm[q] = k.P1[q] * ig2;
   for (int q = 0; q < 3; ++q) k.Vb[q] = 0.5 * (k.Vm[q] + k.Vp[q]);
-  k.v = 1. - k.Vb[0];
-  const double iv = 1. / k.v;
+  const double iv = k.iv = 1. / (1. - k.Vb[0]);
   const double wdj = c.weight * kDj0;
   for (int q = 0; q < 3; ++q) k.dj[q] = wdj * k.Vm[q] * iv;
   k.dj[3] = c.weight * kDrho0 * iv;
@@ -306,26 +297,26 @@ QSS_HD inline bool push_adjoint_cb(const Consts &c, int j, int k, double y0, dou
     gather6(F, fresh(0), w, nullptr, nullptr, f, nullptr, nullptr);
     kinematics(c, Pr, f, kn);
   }
-  const double cy = c.hx / c.hy, cz = c.hx / c.hz, v = kn.v;
+  const double cy = c.hxy, cz = c.hxz, iv = kn.iv;
   const double wdj = c.weight * kDj0;
   double a_v = 0;
-  if (!kn.frozen) a_v -= (kn.d[0] * a_d[0] + kn.d[1] * a_d[1]) / v;
-  for (int q = 0; q < 4; ++q) a_v -= kn.dj[q] * a_dj[q] / v;
+  if (!kn.frozen) a_v -= (kn.d[0] * a_d[0] + kn.d[1] * a_d[1]) * iv;
+  for (int q = 0; q < 4; ++q) a_v -= kn.dj[q] * a_dj[q] * iv;
   double a_Vm[3], a_Vb[3], a_Vp[3];
-  for (int q = 0; q < 3; ++q) a_Vm[q] = wdj / v * a_dj[q];
+  for (int q = 0; q < 3; ++q) a_Vm[q] = wdj * iv * a_dj[q];
   a_Vb[0] = -a_v;
-  a_Vb[1] = kn.frozen ? 0. : cy / v * a_d[0];
-  a_Vb[2] = kn.frozen ? 0. : cz / v * a_d[1];
+  a_Vb[1] = kn.frozen ? 0. : cy * iv * a_d[0];
+  a_Vb[2] = kn.frozen ? 0. : cz * iv * a_d[1];
   for (int q = 0; q < 3; ++q) {
     a_Vm[q] += 0.5 * a_Vb[q];
     a_Vp[q] = 0.5 * a_Vb[q];
   }
   double a_P1[3];
   {
-    const double *P1 = kn.P1, g2 = kn.g2;
+    const double *P1 = kn.P1, ig2 = kn.ig2;
     const double dot = P1[0] * a_Vm[0] + P1[1] * a_Vm[1] + P1[2] * a_Vm[2];
     for (int q = 0; q < 3; ++q)
-      a_P1[q] = a_Vm[q] / g2 - P1[q] * dot / (g2 * g2 * g2) + (full ? NB(2 + q) : 0.);
+      a_P1[q] = a_Vm[q] * ig2 - P1[q] * dot * (ig2 * ig2 * ig2) + (full ? NB(2 + q) : 0.);
   }
   double a_H[3], a_K[3], a_R[3], a_p3[3], a_b[3], a_Q[3];
   for (int q = 0; q < 3; ++q) { a_H[q] = a_P1[q]; a_K[q] = a_P1[q]; a_R[q] = a_P1[q]; }
@@ -347,21 +338,21 @@ QSS_HD inline bool push_adjoint_cb(const Consts &c, int j, int k, double y0, dou
     a_fB[q] = kn.beta * a_b[q];
     a_beta += kn.fB[q] * a_b[q];
   }
-  const double a_g1 = -kn.beta / kn.g1 * a_beta;
-  double a_u = -kn.beta / kn.u * a_beta;
-  for (int q = 0; q < 3; ++q) a_H[q] += kn.H[q] / kn.g1 * a_g1;
+  const double a_g1 = -kn.beta * kn.ig1 * a_beta;
+  double a_u = -kn.beta * kn.iu * a_beta;
+  for (int q = 0; q < 3; ++q) a_H[q] += kn.H[q] * kn.ig1 * a_g1;
   double a_P0[3];
   for (int q = 0; q < 3; ++q) { a_P0[q] = a_H[q]; a_K[q] += a_H[q]; }
   double a_e[3];
   for (int q = 0; q < 3; ++q) {
-    a_e[q] = a_K[q] / kn.u;
-    a_u -= kn.e[q] * a_K[q] / (kn.u * kn.u);
+    a_e[q] = a_K[q] * kn.iu;
+    a_u -= kn.e[q] * a_K[q] * (kn.iu * kn.iu);
   }
   a_Vp[0] -= a_u;
   {
-    const double g0 = kn.g0;
+    const double ig0 = kn.ig0;
     const double dot = P0[0] * a_Vp[0] + P0[1] * a_Vp[1] + P0[2] * a_Vp[2];
-    for (int q = 0; q < 3; ++q) a_P0[q] += a_Vp[q] / g0 - P0[q] * dot / (g0 * g0 * g0);
+    for (int q = 0; q < 3; ++q) a_P0[q] += a_Vp[q] * ig0 - P0[q] * dot * (ig0 * ig0 * ig0);
   }
   const double c1 = kQ2m * c.hx / 2.;
   for (int q = 0; q < 3; ++q) {

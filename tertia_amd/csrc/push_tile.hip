@@ -36,6 +36,7 @@
 
 #include "qss_internal.h"
 #include "split_bf16.h"
+#include "inv_gamma.h"
 #include "tile_sort.h"
 
 namespace {
@@ -111,7 +112,10 @@ __host__ __device__ inline TileArgs wake_view(const TileArgs &a0, int w) {
   return a;
 }
 
+using qss_tile::cell_order;
+using qss_tile::kCell;
 using qss_tile::sort256;
+using qss_tile::thread_index;
 
 template <typename T>
 struct alignas(2 * sizeof(T)) pair_t {
@@ -123,34 +127,6 @@ __device__ inline const FT *field_of(const TileArgs &a) {
   else return a.Ff;
 }
 
-// 1 / sqrt(1 + p^2).  In double: the hardware's estimate (about 2^-24) and two
-// Newton steps on g = x y, h = y / 2 (Goldschmidt's coupled form), then a last
-// correction, 13 operations with an error under an ulp, where the square root and
-// the division it replaces are 29 with two roundings.
-__device__ inline float inv_gamma(float px, float py, float pz) {
-  return 1.0f / sqrt(1.0f + px * px + py * py + pz * pz);
-}
-__device__ inline double inv_gamma(double px, double py, double pz) {
-  const double x = 1.0 + px * px + py * py + pz * pz;
-  double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  const double r = __builtin_fma(-h, g, 0.5);
-  g = __builtin_fma(g, r, g);
-  h = __builtin_fma(h, r, h);
-  y = __builtin_fma(h, __builtin_fma(-h, g, 0.5), h);   // half of 1/sqrt(x)
-  y = y + y;
-  return __builtin_fma(0.5 * y, __builtin_fma(-(x * y), y, 1.0), y);
-}
-
-// threadIdx.x through a register the compiler cannot see into, where the masks and
-// addresses it gives should be remade in each round: kept over the chunk loop they
-// spill what the loop needs
-__device__ inline int thread_index() {
-  int t = threadIdx.x;
-  asm volatile("" : "+v"(t));
-  return t;
-}
-
 // ---- deposit of one round (at most one event per thread) ----------------------
 // By cells: 256 particles of 4 per cell make lists of about 4, and each event is
 // read once, where the sort of 256 keys (36 exchange stages, six of them through LDS
@@ -159,24 +135,6 @@ __device__ inline int thread_index() {
 // the sort, 34.4 (42.7) by cells, all else as it is here.
 // kCell: events of a cell that its owner lane sums directly: the bytes of one 8-byte
 // list, and past 8 the longest list sets the pace of its wave.
-constexpr int kCell = 8;
-
-template <int N>
-__device__ inline void sort_network(int *v) {
-  const auto cx = [&](int i, int j) {
-    const int a = v[i], b = v[j];
-    v[i] = min(a, b);
-    v[j] = max(a, b);
-  };
-  if constexpr (N == 4) {
-    cx(0, 1); cx(2, 3); cx(0, 2); cx(1, 3); cx(1, 2);
-  } else {   // 19 exchanges for 8
-    static_assert(N == 8, "networks for 4 and 8");
-    cx(0, 2); cx(1, 3); cx(4, 6); cx(5, 7); cx(0, 4); cx(1, 5); cx(2, 6); cx(3, 7);
-    cx(0, 1); cx(2, 3); cx(4, 5); cx(6, 7); cx(2, 4); cx(3, 5); cx(1, 4); cx(3, 6);
-    cx(1, 2); cx(3, 4); cx(5, 6);
-  }
-}
 
 // Sums of one cell's events over its four nodes, in the order of the events'
 // indices: the order in which they reached the list does not matter.
@@ -184,10 +142,7 @@ template <int N, int NQ>
 __device__ inline void cell_sums(uint2 bytes, int n, const double *ev_y, const double *ev_z,
                                  const double (*ev_w)[NT], bool cic, double (*s)[NQ]) {
   int e[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i)
-    e[i] = i < n ? (int)((i < 4 ? bytes.x >> 8 * i : bytes.y >> 8 * (i - 4)) & 255) : NT + i;
-  sort_network<N>(e);
+  cell_order<N>(bytes, n, e);
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     if (i >= n) break;

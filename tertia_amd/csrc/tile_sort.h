@@ -10,6 +10,15 @@
 
 namespace qss_tile {
 
+// threadIdx.x through a register the compiler cannot see into, where the masks and
+// addresses it gives should be remade in each round: kept over the chunk loop they
+// spill what the loop needs
+__device__ inline int thread_index() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 // value held by lane (lane ^ J) of this wave64
 template <int J>
 __device__ inline int xor_lane(int v, int t) {
@@ -72,9 +81,37 @@ __device__ inline int bitonic_sort(int key, int *sh, int t) {
 // otherwise keep every stage's lane masks (36 pairs of scalar registers) alive over
 // the caller's whole loop and spill what the loop needs.
 __device__ inline int sort256(int key, int *sh) {
-  int t = threadIdx.x;
-  asm volatile("" : "+v"(t));
-  return bitonic_sort<256>(key, sh, t);
+  return bitonic_sort<256>(key, sh, thread_index());
+}
+
+// Events of a cell that one lane sums: the bytes of one 8-byte list (indices of the
+// round's 256 events), put in the order of the indices by networks of 4 or 8.
+constexpr int kCell = 8;
+
+template <int N>
+__device__ inline void sort_network(int *v) {
+  const auto cx = [&](int i, int j) {
+    const int a = v[i], b = v[j];
+    v[i] = min(a, b);
+    v[j] = max(a, b);
+  };
+  if constexpr (N == 4) {
+    cx(0, 1); cx(2, 3); cx(0, 2); cx(1, 3); cx(1, 2);
+  } else {   // 19 exchanges for 8
+    static_assert(N == 8, "networks for 4 and 8");
+    cx(0, 2); cx(1, 3); cx(4, 6); cx(5, 7); cx(0, 4); cx(1, 5); cx(2, 6); cx(3, 7);
+    cx(0, 1); cx(2, 3); cx(4, 5); cx(6, 7); cx(2, 4); cx(3, 5); cx(1, 4); cx(3, 6);
+    cx(1, 2); cx(3, 4); cx(5, 6);
+  }
+}
+
+// the list's indices in order, sentinels past n
+template <int N>
+__device__ inline void cell_order(uint2 bytes, int n, int *e) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    e[i] = i < n ? (int)((i < 4 ? bytes.x >> 8 * i : bytes.y >> 8 * (i - 4)) & 255) : 256 + i;
+  sort_network<N>(e);
 }
 
 }  // namespace qss_tile

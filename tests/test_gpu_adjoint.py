@@ -227,3 +227,23 @@ sys.exit(0 if abs(loss.item() - l2) <= 1e-12 * abs(l2) and d < 1e-12 and stale_r
                        timeout=300, cwd=ROOT)
     print(r.stdout, r.stderr[-2000:])
     assert r.returncode == 0
+
+
+@pytest.mark.parametrize("ppc_y,ppc_z,split", [(1, 1, 1), (2, 2, 2), (2, 4, 1), (3, 3, 1), (4, 4, 4)])
+def test_adjoint_cell_counts(ppc_y, ppc_z, split):
+    """The reverse push's transposed gather with 1, 4, 8 particles per cell (the lists)
+    and 9 and 16 (the sort of a crowded chunk), shared by 1, 2 and 4 work-groups."""
+    from tertia_amd.mesh import Mesh
+    p = small_bins(ppc_y=ppc_y, ppc_z=ppc_z)
+    nrun = 56
+    m = Mesh(p, history=("Ex",))
+    try:
+        m.particle_split = split
+        _, g, _ = adjoint_grad(m, p, nrun, 8, WIN_SMALL)
+        idx = [2, 8, 14]
+        gf = fd_grad(m, p, nrun, WIN_SMALL, idx)
+    finally:
+        m.close()
+    scale = np.abs(g).max()
+    assert scale > 0
+    assert (np.abs(g[idx] - gf) / scale).max() < 1e-4
