@@ -4,21 +4,32 @@
 //
 // qss_transform2d runs on a context, whose creation allocates the transform
 // tables and the intermediate plane of the two GEMM passes.  This entry point
-// needs no context: both tables and the intermediate live in `scratch`, a
-// fixed device array of this file (3 planes of kMaxN^2 doubles, 6 MiB per
-// device, held until the process ends).  Each call rebuilds the two tables in
-// it (the same exact integer argument reduction as the context's host-built
-// tables), runs the y pass into the intermediate and the z pass into the
-// caller's output, all enqueued on the caller's stream: no allocation, no
-// synchronisation.  Every call on a device shares that device's scratch, so
-// calls that overlap on one device race; one stream serialises them.
+// needs no context: tables and intermediate live in `scratch`, a fixed device
+// array of this file (3 planes of kMaxN^2 doubles, 6 MiB per device, held until
+// the process ends).  Each call rebuilds the tables in it (the same exact integer
+// argument reduction as the context's host-built tables), runs the y pass into the
+// intermediate and the z pass into the caller's output, all enqueued on the
+// caller's stream: no allocation, no synchronisation.  Every call on a device
+// shares that device's scratch, so calls that overlap on one device race; one
+// stream serialises them.
+//
+// Planes whose sides both have a chain of radices (even, no prime factor of the half
+// above 13) go through the line transforms (line.hip): a chain's tables are a few
+// hundred entries where the dense ones are n^2 cosines, and the passes a fraction of
+// the dense products' work.  Dense against lines, us a call: 512 x 512 54.0 / 16.1,
+// 312 x 200 38.0 / 18.2, 100 x 100 22.0 / 15.9, 66 x 52 17.8 / 16.8, 12 x 10 16.6 /
+// 14.2 (a context, whose tables stand ready, keeps dense products for loose chains
+// below 192); what is left is three launches and two passes over the plane.
 //
 // The array's name is not a device address in host code: its per-device
 // address comes from hipGetSymbolAddress, taken once per device with that
 // device current, and only that address is handed to kernels.
 
+#include <algorithm>
+#include <exception>
 #include <mutex>
 
+#include "line_plan.h"
 #include "qss_internal.h"
 
 namespace {
@@ -42,6 +53,63 @@ __global__ __launch_bounds__(256) void k_half_integer_table(double *T, int n, in
   const long m = ((long)(2 * j + 1) * (2 * k + 1)) % (8L * n);
   const double a = M_PI * (double)m / (4.0 * n);
   T[i] = 2.0 * (kind == QSS_KIND_C ? cos(a) : sin(a));
+}
+
+// 2 cos, -2 sin and the like of whole multiples q of pi / 4n: the first quadrant's
+// value (its half nearer to zero), turned by quadrants
+__device__ inline void phase(int q, int n, double &c, double &s) {
+  q %= 8 * n;
+  const int quad = q / (2 * n), r = q - quad * 2 * n;
+  const bool far = r > n;
+  const double x = (double)(far ? 2 * n - r : r) / (4.0 * n);   // at most 1/4
+  const double cx = cospi(x), sx = sinpi(x), c0 = far ? sx : cx, s0 = far ? cx : sx;
+  c = quad == 0 ? c0 : quad == 1 ? -s0 : quad == 2 ? -c0 : s0;
+  s = quad == 0 ? s0 : quad == 1 ? c0 : quad == 2 ? -s0 : -c0;
+}
+
+// the tables of both axes' chains (line_table in line_plan.h); blockIdx.y: axis
+__global__ __launch_bounds__(256) void k_line_tables(LineAxis y, LineAxis z, double *ty,
+                                                     double *tz) {
+  const LineAxis ax = blockIdx.y ? z : y;
+  double *const tw = blockIdx.y ? tz : ty;
+  const int e = blockIdx.x * 256 + threadIdx.x, n = ax.n, m = ax.m;
+  if (e >= (ax.np - 1) * m) return;
+  const int p = 1 + e / m, i = e - (p - 1) * m;
+  int ns = ax.radix(0);
+  for (int q = 1; q < p; ++q) ns *= ax.radix(q);
+  const int R = ax.radix(p), mr = m / R, b = i % mr, r = i / mr;
+  int q = (b % ns) * r % (ns * R) * (8 * n / (ns * R));
+  double scale = 1.0;
+  if (p == 1) q += 4 * (i / ax.radix(0)) + 1;
+  if (p == ax.np - 1) {
+    q += 4 * b;
+    scale = 2.0;
+  }
+  double c, s;
+  phase(q, n, c, s);
+  tw[2 * e] = scale * c;
+  tw[2 * e + 1] = -scale * s;
+}
+
+// The chain of a length, searched for once per process (guarded by g_mu); np = 0
+// where it has none.
+struct Chain {
+  bool known = false;
+  LineAxis ax;
+};
+Chain g_chain[kMaxN + 1];
+LineAxis chain_of(int n) {
+  Chain &c = g_chain[n];
+  if (!c.known) {
+    LineAxis ax;
+    try {
+      if (line_chain(n, &ax)) c.ax = ax;
+    } catch (const std::exception &) {   // no memory for the search: dense this time
+      return LineAxis{};
+    }
+    c.known = true;
+  }
+  return c.ax;
 }
 
 int fail(const std::string &m, int code) {
@@ -68,8 +136,11 @@ extern "C" int qss_transform2d_noalloc(int ny, int nz, int kind_z, int kind_y,
   if (e != hipSuccess) return fail(hipGetErrorString(e), QSS_E_HIP);
   if (dev < 0 || dev >= kMaxDevices) return fail("device index out of range", QSS_E_ARG);
   double *base = nullptr;
+  LineAxis y, z;
   {
     std::lock_guard<std::mutex> lk(g_mu);
+    y = chain_of(ny);
+    z = chain_of(nz);
     if (!g_scratch[dev]) {   // first call on this device, the device current
       void *p = nullptr;
       e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
@@ -80,6 +151,36 @@ extern "C" int qss_transform2d_noalloc(int ny, int nz, int kind_z, int kind_y,
   }
   double *Ty = base, *Tz = base + kPlane, *mid = base + 2 * kPlane;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (y.np && z.np) {
+    const int most = std::max((y.np - 1) * y.m, (z.np - 1) * z.m);
+    hipLaunchKernelGGL(k_line_tables, dim3((unsigned)(most + 255) / 256, 2), dim3(256), 0, s, y, z,
+                       Ty, Tz);
+    if ((e = hipGetLastError()) != hipSuccess) return fail(hipGetErrorString(e), QSS_E_HIP);
+    y.tw = Ty;
+    z.tw = Tz;
+    if (line_plane_ok(y, z)) {
+      SmallPlaneArgs a{};
+      a.y = y; a.z = z;
+      a.nbatch = a.nw = 1; a.alpha = scale;
+      a.in[0] = in_dev; a.out[0] = out_dev;
+      a.ky[0] = kind_y; a.kz[0] = kind_z;
+      e = launch_line_plane(a, s);
+    } else {
+      RowArgs r{};
+      r.ax = y;
+      r.nz = nz; r.nbatch = r.nw = 1;
+      r.in[0] = in_dev; r.out[0] = mid; r.ky[0] = kind_y;
+      ColArgs c{};
+      c.ax = z;
+      c.ny = ny; c.nbatch = c.nw = 1;
+      c.in[0] = mid; c.out[0] = out_dev; c.kz[0] = kind_z;
+      c.resid[0] = c.push[0] = -1;
+      c.store[0] = 1;
+      c.alpha = scale;
+      if ((e = launch_line_rows(r, s)) == hipSuccess) e = launch_line_cols(c, s);
+    }
+    return e == hipSuccess ? QSS_OK : fail(hipGetErrorString(e), QSS_E_HIP);
+  }
   hipLaunchKernelGGL(k_half_integer_table, dim3((unsigned)(((long)ny * ny + 255) / 256)),
                      dim3(256), 0, s, Ty, ny, kind_y);
   hipLaunchKernelGGL(k_half_integer_table, dim3((unsigned)(((long)nz * nz + 255) / 256)),

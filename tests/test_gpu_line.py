@@ -55,3 +55,30 @@ def test_sweep_on_line_grids_vs_oracle(oracle_mod, ny, nz, kw):
     finally:
         m.close()
         o.close()
+
+
+@pytest.mark.parametrize("nz,ny", [(32, 32), (64, 48), (40, 128), (312, 200), (512, 512),
+                                   (8, 4), (66, 36), (26, 286),                  # lines
+                                   (194, 256), (17, 19), (31, 64)])              # dense
+def test_noalloc_lines_vs_oracle(oracle_mod, nz, ny):
+    """The context-free transform on both sides of its rule (lengths compiled in, loose
+    chains, down to the shortest; a side without a chain makes both dense), out of place and in place; its tables
+    are built on the device."""
+    import ctypes
+    from tertia_amd.mesh import Mesh
+    m = Mesh(small(ny=ny, nz=nz, nslices=2), history=())
+    try:
+        x = np.random.default_rng(nz + 1000 * ny).standard_normal((nz, ny))
+        s = ctypes.c_void_p(m.stream)
+        for kz in (0, 1):
+            for ky in (0, 1):
+                ref = 0.25 * oracle_mod.transform2d(x, kz, ky, use_fft=False, nthreads=4)
+                m.set_field("Rho", x)
+                for dst in ("Jx", "Rho"):
+                    assert m.L.qss_transform2d_noalloc(ny, nz, kz, ky, m.layer_ptr("Rho"),
+                                                       m.layer_ptr(dst), 0.25, s) == 0
+                got = m.get_field("Jx")
+                assert max_rel(got, ref) < 1e-13, (kz, ky)
+                assert np.array_equal(m.get_field("Rho"), got)
+    finally:
+        m.close()
