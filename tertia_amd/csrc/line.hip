@@ -58,6 +58,8 @@ constexpr int kXcd = 8;
 constexpr int kLines = 8;     // lines per work-group (columns of a strip, rows of a row kernel)
 constexpr int kMaxT = kLineT;
 constexpr int NTL = kLines * kMaxT;
+constexpr int kDenseModesNT = 1024;   // threads of k_line_modes with the dense table
+static_assert(kLineDenseY <= kDenseModesNT, "a mode per thread");
 constexpr int kPer = 2;       // elements of a line per thread of the work-group at most
 constexpr int kPre = 8;       // result pairs whose epilogue operands a thread loads ahead
 
@@ -464,13 +466,38 @@ __global__ __launch_bounds__(kDenseNT) void k_line_cols_dense(ColArgs a) {
   const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
   const int j = s.j0 + li;
   ColEnd e(a, s.f, s.w);
-  for (int i = threadIdx.x; i < N * kDenseL; i += kDenseNT) {
-    const int n = i / kDenseL, l = i % kDenseL;
-    xs[i] = s.j0 + l < ny ? in[(long)n * ny + l] : 0.0;
+  // the whole strip and the first steps of the table are asked for before anything
+  // is waited for: one latency, where a loop that stores each value pays one for
+  // every 32 rows (97 rows: 8.1 us a launch, 7.3 like this)
+  constexpr int PER = kLineDenseZ * kDenseL / kDenseNT;
+  static_assert(PER * kDenseNT == kLineDenseZ * kDenseL, "a strip in registers");
+  double v[PER];
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    const int i = threadIdx.x + kDenseNT * q, n = i / kDenseL, l = i % kDenseL;
+    v[q] = n < N && s.j0 + l < ny ? in[(long)n * ny + l] : 0.0;
+  }
+  const double *T = a.kz[s.f] == QSS_KIND_C ? a.ax.Tc : a.ax.Ts;
+  constexpr int S = 8;   // steps of 4 n fetched ahead
+  double t[S], next[S];
+  const auto fetch = [&](int n0, int kk, double(&v)[S]) {
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+      const int n = n0 + 4 * q + lk < N ? n0 + 4 * q + lk : N - 1;
+      v[q] = T[n * N + kk];
+    }
+  };
+  // the table is symmetric: T[n][k]
+  const auto column = [&](int k0) { return k0 + li < N ? k0 + li : N - 1; };
+  const int first = (threadIdx.x >> 6) * 16;
+  fetch(0, column(first), t);
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    const int i = threadIdx.x + kDenseNT * q;
+    if (i < N * kDenseL) xs[i] = v[q];
   }
   __syncthreads();
-  const double *T = a.kz[s.f] == QSS_KIND_C ? a.ax.Tc : a.ax.Ts;
-  for (int k0 = (threadIdx.x >> 6) * 16; k0 < N; k0 += kDenseNT / 4) {
+  for (int k0 = first; k0 < N; k0 += kDenseNT / 4) {
     double o[4] = {0, 0, 0, 0};
     const bool want = EPI == 1 ? e.push : EPI == 3 || (EPI && e.resid);
     const double *from = EPI == 1 ? e.P : e.C;
@@ -480,20 +507,11 @@ __global__ __launch_bounds__(kDenseNT) void k_line_cols_dense(ColArgs a) {
         if (k0 + lk + 4 * r < N) o[r] = from[(long)(k0 + lk + 4 * r) * ny + j];
     }
     double4v d = {0, 0, 0, 0};
-    const int kk = k0 + li < N ? k0 + li : N - 1;   // the table is symmetric: T[n][k]
-    constexpr int S = 8;   // steps of 4 n fetched ahead
-    double t[S], next[S];
-    const auto fetch = [&](int n0, double(&v)[S]) {
-#pragma unroll
-      for (int q = 0; q < S; ++q) {
-        const int n = n0 + 4 * q + lk < N ? n0 + 4 * q + lk : N - 1;
-        v[q] = T[n * N + kk];
-      }
-    };
-    fetch(0, t);
+    const int kk = column(k0);
+    if (k0 != first) fetch(0, kk, t);
 #pragma unroll 1
     for (int n0 = 0; n0 < N; n0 += 4 * S) {
-      fetch(n0 + 4 * S, next);   // past the end: the last row again, not used
+      fetch(n0 + 4 * S, kk, next);   // past the end: the last row again, not used
 #pragma unroll
       for (int q = 0; q < S; ++q) {
         // past the strip's end: zero
@@ -557,63 +575,68 @@ __device__ inline cplx *lines_fft(const LineAxis &ax, cplx *src, cplx *dst, cons
   return out;
 }
 
-// the same with the dense table, NL <= 16 lines, from x to y (pitch in doubles):
-// D[line][k] = sum_n X[line][n] T[n][k] with both tables, each line taking its
-// kind's.  A wave makes two 16-column tiles at a time and fetches the table
-// entries of four steps ahead of the products of the last four: the table comes
-// from L2, and unhidden its latency is all the time there is.
-template <int NL>
-__device__ inline void lines_dense(const LineAxis &ax, const double *x, double *y, int pitch,
-                                   unsigned sine_mask) {
-  constexpr int S = 4;   // steps of 4 n
-  const int N = ax.n, lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-  const double *const T[2] = {ax.Tc, ax.Ts};
-  const double *const xl = x + (li < NL ? li : 0) * pitch;
-  for (int k0 = (threadIdx.x >> 6) * 32; k0 < N; k0 += NTL / 2) {
-    double4v d[2][2] = {};   // [tile][kind]
-    int kk[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) kk[h] = k0 + 16 * h + li < N ? k0 + 16 * h + li : N - 1;
-    double t[S][2][2];
-    const auto fetch = [&](int n0, double(&v)[S][2][2]) {
-#pragma unroll
-      for (int q = 0; q < S; ++q) {
-        const int n = n0 + 4 * q + lk < N ? n0 + 4 * q + lk : N - 1;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int u = 0; u < 2; ++u) v[q][h][u] = T[u][n * N + kk[h]];
-      }
-    };
-    fetch(0, t);
+// Lines of one kind by fours, for v_mfma_f64_4x4x4_4b: group g's line i in the low 4
+// bits of nibble 4 g + i (15: none); the first nc groups are cosine lines.
+struct LineGroups {
+  unsigned long long lines;
+  int n, nc;
+};
+constexpr LineGroups line_groups(int nl, unsigned sine) {
+  LineGroups r{~0ull, 0, 0};
+  for (int kind = 0; kind < 2; ++kind) {
+    int used = 0;
+    for (int l = 0; l < nl; ++l) {
+      if ((int)(sine >> l & 1u) != kind) continue;
+      const int at = 4 * (4 * (r.n + used / 4) + used % 4);
+      r.lines = (r.lines & ~(15ull << at)) | (unsigned long long)l << at;
+      ++used;
+    }
+    r.n += (used + 3) / 4;
+    if (kind == 0) r.nc = r.n;
+  }
+  return r;
+}
+
+// the same with the dense table, NL lines (SINE: which take the sine table), from x
+// to y (pitch in doubles): D[line][k] = sum_n X[line][n] T[n][k].  A wave makes 16
+// columns of up to four lines of one kind at a time with v_mfma_f64_4x4x4_4b (lane
+// l: A[l % 4][l / 16] in each block, B[l / 16][l % 16], D[l / 16][l % 16] over the four
+// blocks' columns), and asks for 64 rows of its columns of the table before the
+// first product: the table comes from beyond L2, and its latency, once per 16 rows
+// of it, was most of the time when 16-line tiles were made by four waves (121
+// columns: 23.0 us a launch for 3 in and 6 out, 15.1 like this).
+template <int NL, unsigned SINE>
+__device__ inline void lines_dense(const LineAxis &ax, const double *x, double *y, int pitch) {
+  constexpr LineGroups G = line_groups(NL, SINE);
+  constexpr int S = 16;   // steps of 4 n whose table entries are asked for at once
+  const int N = ax.n, lane = threadIdx.x & 63, lk = lane >> 4;
+  const int tiles = (N + 15) / 16;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int task = wave; task < tiles * G.n; task += kDenseModesNT / 64) {
+    const int g = task / tiles, col = (task - g * tiles) * 16 + (lane & 15);
+    const char *const T = reinterpret_cast<const char *>(g < G.nc ? ax.Tc : ax.Ts);
+    const int in = (int)(G.lines >> (16 * g + 4 * (lane & 3))) & 15;
+    const double *const xl = x + (in < NL ? in : 0) * pitch;
+    double d[2] = {};
 #pragma unroll 1
     for (int n0 = 0; n0 < N; n0 += 4 * S) {
-      double next[S][2][2];
-      fetch(n0 + 4 * S, next);   // past the end: the last row again, not used
+      double t[S];
+#pragma unroll
+      for (int q = 0; q < S; ++q) {
+        const int n = n0 + 4 * q + lk;   // 32-bit byte offsets: a table is below 2 MB
+        const unsigned at = 8u * ((n < N ? n : N - 1) * N + (col < N ? col : N - 1));
+        t[q] = *reinterpret_cast<const double *>(T + at);
+      }
 #pragma unroll
       for (int q = 0; q < S; ++q) {
         const int n = n0 + 4 * q + lk;
-        const double v = xl[n < N ? n : N - 1], xv = li < NL && n < N ? v : 0.0;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int u = 0; u < 2; ++u)
-            d[h][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv, t[q][h][u], d[h][u], 0, 0, 0);
+        const double v = xl[n < N ? n : N - 1];
+        d[q & 1] = __builtin_amdgcn_mfma_f64_4x4x4f64(in < NL && n < N ? v : 0.0, t[q], d[q & 1],
+                                                      0, 0, 0);
       }
-#pragma unroll
-      for (int q = 0; q < S; ++q)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int u = 0; u < 2; ++u) t[q][h][u] = next[q][h][u];
     }
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int line = lk + 4 * r, k = k0 + 16 * h + li;
-        if (line < NL && k < N) y[line * pitch + k] = sine_mask >> line & 1u ? d[h][1][r] : d[h][0][r];
-      }
+    const int to = (int)(G.lines >> (16 * g + 4 * lk)) & 15;
+    if (to < NL && col < N) y[to * pitch + col] = d[0] + d[1];
   }
   __syncthreads();
 }
@@ -787,21 +810,23 @@ constexpr int kIterIn[10] = {SP_RHOP, SP_JXP, SP_JYP, SP_JZP, SP_RHOB,
                              SP_RHOBP, SP_EYP, SP_EZP, SP_RHO, SP_JXB};
 
 template <bool GUESS, int NOUT, bool DENSE, class C>
-__global__ __launch_bounds__(NTL) void k_line_modes(ModeArgs a) {
+__global__ __launch_bounds__(DENSE ? kDenseModesNT : NTL) void k_line_modes(ModeArgs a) {
   using namespace qss_spec;
   extern __shared__ cplx lds[];   // two sides of NOUT * pitch, then the tables
   constexpr int NIN = GUESS ? 2 : 3, NS = GUESS ? 8 : 10;
   const LineAxis &ax = a.ax;
-  const int N = C::n(ax), pitch = 2 * pitch_of<C>(ax), NT = kLines * C::threads();
+  const int N = C::n(ax), pitch = 2 * pitch_of<C>(ax);
+  const int NT = DENSE ? kDenseModesNT : kLines * C::threads();
+  constexpr int PER = DENSE ? 1 : kPer;   // a dense axis has at most kLineDenseY modes
   cplx *const side = lds + NOUT * pitch / 2, *const tw = side + NOUT * pitch / 2;
   double *x = reinterpret_cast<double *>(lds);
   const int item = xcd_item(blockIdx.x, gridDim.x);
   const int w = item / a.nz, kz = item - w * a.nz;
   const long row = (long)w * a.nc + (long)kz * N;
   double *const *S = a.S;
-  double v[kPer][NIN], sp[kPer][NS];
+  double v[PER][NIN], sp[PER][NS];
 #pragma unroll
-  for (int q = 0; q < kPer; ++q) {
+  for (int q = 0; q < PER; ++q) {
     const int i = threadIdx.x + NT * q;
     if (i < N) {
 #pragma unroll
@@ -809,7 +834,7 @@ __global__ __launch_bounds__(NTL) void k_line_modes(ModeArgs a) {
     }
   }
 #pragma unroll
-  for (int q = 0; q < kPer; ++q) {
+  for (int q = 0; q < PER; ++q) {
     const int i = threadIdx.x + NT * q;
     if (i < N) {
 #pragma unroll
@@ -823,7 +848,7 @@ __global__ __launch_bounds__(NTL) void k_line_modes(ModeArgs a) {
          i += (long)gridDim.x * NT)
       a.rslots[i] = 0ull;
 #pragma unroll
-  for (int q = 0; q < kPer; ++q) {
+  for (int q = 0; q < PER; ++q) {
     const int i = threadIdx.x + NT * q;
     if (i < N) {
 #pragma unroll
@@ -834,7 +859,7 @@ __global__ __launch_bounds__(NTL) void k_line_modes(ModeArgs a) {
   __syncthreads();
   if constexpr (DENSE) {
     double *y = reinterpret_cast<double *>(side);
-    lines_dense<NIN>(ax, x, y, pitch, GUESS ? 0u : kSineJ);
+    lines_dense<NIN, GUESS ? 0u : kSineJ>(ax, x, y, pitch);
     x = y;
   } else {
     x = reinterpret_cast<double *>(
@@ -845,7 +870,7 @@ __global__ __launch_bounds__(NTL) void k_line_modes(ModeArgs a) {
   m.hx = a.hx;
   m.akz = M_PI / a.lz * (kz + 0.5);
 #pragma unroll
-  for (int q = 0; q < kPer; ++q) {
+  for (int q = 0; q < PER; ++q) {
     const int i = threadIdx.x + NT * q;
     if (i >= N) continue;
     const long n1 = row + i;
@@ -931,7 +956,7 @@ __global__ __launch_bounds__(NTL) void k_line_modes(ModeArgs a) {
     cplx *const from = reinterpret_cast<cplx *>(x), *const to = from == lds ? side : lds;
     if constexpr (DENSE) {
       double *y = reinterpret_cast<double *>(to);
-      lines_dense<NOUT>(ax, x, y, pitch, kSineEB);
+      lines_dense<NOUT, kSineEB>(ax, x, y, pitch);
       x = y;
     } else {
       x = reinterpret_cast<double *>(lines_fft<C>(ax, from, to, tw, NOUT, kSineEB));
@@ -1053,6 +1078,6 @@ hipError_t launch_line_modes(const ModeArgs &a, bool guess, hipStream_t s, hipEv
   };
   auto fn = with_shape(a.ax, [&](auto shape) { return pick(std::false_type(), shape); });
   return launch(a.ax.np ? fn : pick(std::true_type(), Loose<false>()),
-                (unsigned)(a.nz * a.nw), line_threads(a.ax),
+                (unsigned)(a.nz * a.nw), a.ax.np ? line_threads(a.ax) : kDenseModesNT,
                 rows_lds(a.ax, a.psi && !guess ? 8 : 6), s, ev0, ev1, a);
 }

@@ -515,9 +515,7 @@ int do_push_deposit(qss_ctx *c, int full) {
   forget_splits(c);   // the global deposit writes J without its split form
   {
     Timed t(c, KC_SORT);
-    HIPCHECK(launch_fill_i32(c->cnt, c->ncell, 0, c->stream));
-    if (full) HIPCHECK(launch_fill_i32(c->cnt_main, c->ncell, 0, c->stream));
-    HIPCHECK(launch_fill_i32(c->d_counters, 1, 0, c->stream));
+    HIPCHECK(launch_clear_counts(c, full));
   }
   {
     Timed t(c, KC_PUSH);

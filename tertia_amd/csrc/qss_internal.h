@@ -431,6 +431,7 @@ hipError_t launch_driver_plane(qss_ctx *c, int slice, int isplit);
 hipError_t launch_guess_update(qss_ctx *c, int first_layer);
 hipError_t launch_iterate_update(qss_ctx *c, int final_pass);
 hipError_t launch_push(qss_ctx *c, int full_step);
+hipError_t launch_clear_counts(qss_ctx *c, int full_step);
 hipError_t launch_sort_scan(qss_ctx *c, int full_step);
 hipError_t launch_scatter(qss_ctx *c);
 hipError_t launch_tile_reduce(qss_ctx *c, int full_step);

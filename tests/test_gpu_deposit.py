@@ -102,3 +102,46 @@ def test_reorder_scan_edges(oracle_mod, ny, nz, nsplit):
             assert np.abs(po[k][oo] - pg[k][og]).max() <= bar, k
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("shape", [QSS_SHAPE_CIC, QSS_SHAPE_NGP_REF])
+@pytest.mark.parametrize("per_cell,hot", [(1, 0), (4, 0), (8, 0), (9, 0), (30, 0), (3, 6)])
+def test_global_deposit_cell_counts(oracle_mod, shape, per_cell, hot):
+    """The same on a grid that is not made of tiles: lists of up to 8 events are ordered
+    in registers, longer ones selected from, sub-steps of one particle by their
+    number; the full step also stores the particles in that order."""
+    from tertia_amd.mesh import Mesh
+    ny, nz = 37, 50
+    rng = np.random.default_rng(7 * per_cell + hot)
+    p = small(ny=ny, nz=nz, nslices=2, hx=0.4 if hot else 0.05, shape=shape, ppc_y=2, ppc_z=4)
+    cells = np.sort(rng.permutation(ny * nz)[: ny * nz * 8 // per_cell])
+    cell = np.repeat(cells, per_cell)
+    n = len(cell)
+    mom = rng.uniform(-0.1, 0.1, size=(3, n))
+    if hot:
+        mom[0, ::hot] = 3.0
+        mom[1, ::hot] = rng.uniform(-4, 4, size=len(mom[1, ::hot]))
+    parts = ((cell % ny).astype(np.int32), (cell // ny).astype(np.int32),
+             rng.uniform(0.2, 0.8, n), rng.uniform(0.2, 0.8, n), *mom,
+             np.arange(n, dtype=np.int64))
+    m, o = Mesh(p, history=()), oracle_mod.Oracle(p, history=())
+    try:
+        o.set_particles(*parts)
+        runs = []
+        for _ in range(2):
+            m.set_particles(*parts)
+            got = []
+            for full in (0, 1, 0):
+                m.MoveParticlesLayerSplit(0, 0, full)
+                got += [m.get_field(f) for f in ("Jx", "Jy", "Jz", "Rho")]
+            runs.append(got + [m.particles()["id"]])
+        ref = []
+        for full in (0, 1, 0):
+            o.push_deposit(full)
+            ref += [o.get_field(f) for f in ("Jx", "Jy", "Jz", "Rho")]
+        for g, r in zip(runs[0], ref):
+            assert max_rel(g, r) <= 1e-13
+        for a, b in zip(*runs):
+            assert np.array_equal(a, b)
+    finally:
+        m.close()
