@@ -69,12 +69,12 @@ __device__ inline void cell_sums(uint2 bytes, int n, const double (*ev_f)[NT],
 // Transposed gather of a chunk by cells: a tile's 256 cells are one per lane; its
 // owner sums a cell's events over the four corners in registers, and the corners
 // are added to the window's node sums in turns (in one corner's turn no two cells
-// share a node).  Cells are dealt to the waves in turn.  Leaves the counts at zero.
+// share a node).  Leaves the counts at zero.
 __device__ inline void scatter_cells(int *cnt, const uint2 *list, const double (*ev_f)[NT],
                                      const double (*ev_w)[NT], double (*acc)[NF]) {
   static_assert(T * T == NT, "a cell per lane");
   const int t = qss_tile::thread_index();
-  const int cell = 4 * (t & 63) + (t >> 6);
+  const int cell = t;
   const int n = cnt[cell];
   double s[4][6] = {};
   if (n) {

@@ -164,15 +164,17 @@ __device__ inline void cell_sums(uint2 bytes, int n, const double *ev_y, const d
 // A lane sums the events of the window cell it owns in this half (cells 0 .. NT - 1
 // or the rest) over the four corners in registers, each event read once, and the
 // four corners are added to the node sums one after the other, a barrier
-// between: in one corner's turn no two cells share a node.  Cells are dealt to
-// the waves in turn, since a chunk's events lie in few neighbouring rows.
+// between: in one corner's turn no two cells share a node.  A chunk's events lie in
+// few neighbouring rows, so with the cells in order some waves have all the work
+// and the others none to issue (dealt to the waves in turn: 34.4 us a push at 512^2
+// against 32.0).
 // Leaves the counts at zero.
 template <int NQ>
 __device__ inline void deposit_cells(int half, int *cnt, const uint2 *list, const double *ev_y,
                                      const double *ev_z, const double (*ev_w)[NT],
                                      double (*wacc)[NWIN], bool cic) {
   const int t = thread_index();
-  const int cell = 4 * (t & 63) + (t >> 6) + NT * half;
+  const int cell = t + NT * half;
   double s[4][NQ];
   const int n = cell < NWIN ? cnt[cell] : 0;
 #pragma unroll
@@ -276,11 +278,11 @@ __device__ inline void deposit_sorted(int cellw, int *keys, int *sorted, short *
 // 128 VGPRs and 40 KB of LDS at most (RHO: 46 KB): four waves per SIMD, so all the
 // tiles of a 512^2 grid (4 work-groups per CU) are resident at once.  The bound is
 // instruction issue and latency, not memory: at 512^2 and 4 per cell 58 MB in and
-// 15 MB out (full: 61 MB) in 34.4 us (full: 42.7), half of the wave cycles waiting at
+// 15 MB out (full: 61 MB) in 31.8 us (full: 38.0), half of the wave cycles waiting at
 // barriers and for LDS.  What spilled registers here cost most: with uniform FP64
 // products made on the host, the sort's lane masks not kept over the loop and
-// machine LICM off (it keeps FP64 literals in registers) nothing spills, 37 us on
-// average of a step's three pushes against 42.6 with 104 scalar registers spilled.
+// machine LICM off (it keeps FP64 literals in registers) nothing spills: 37 us on
+// average of a step's three pushes at that point, against 42.6 with 104 scalar registers spilled.
 // FULL: the pushed particles are staged for the reorder.
 // RHO = false: the deposit sums Jx, Jy, Jz only and the windows' density
 // component stays 0 (inside a layer step nothing reads the deposited density:
@@ -330,18 +332,30 @@ void k_push_tile(TileArgs a0) {
   const bool cic = a.shape == QSS_SHAPE_CIC;
   int status = 0;   // ST_* bits met by this thread, reported once at the end
 
-  const int base = a.tile_start[tile];
-  const int np = a.tile_start[tile + 1] - base;
+  const int base = __builtin_amdgcn_readfirstlane(a.tile_start[tile]);
+  const int np = __builtin_amdgcn_readfirstlane(a.tile_start[tile + 1]) - base;
 
   // 1. field window: nodes (j0..j0+T, k0..k0+T), periodic
-  for (int i = t; i < NF; i += NT) {
-    const int lj = i % FW, lk = i / FW;
-    const int gj = j0 + lj < ny ? j0 + lj : 0, gk = k0 + lk < nz ? k0 + lk : 0;   // at most one past
-    const long g = gj + (long)ny * gk;
+  {
+    // both nodes of a thread asked for before either is stored
+    constexpr int PER = (NF + NT - 1) / NT;
     const long plane = (long)ny * nz;
     const FT *const F = field_of<FT>(a);
+    FT v[PER][6];
 #pragma unroll
-    for (int q = 0; q < 3; ++q) Fw[q][i] = {F[2 * q * plane + g], F[(2 * q + 1) * plane + g]};
+    for (int e = 0; e < PER; ++e) {
+      const int i = t + NT * e < NF ? t + NT * e : NF - 1;
+      const int lj = i % FW, lk = i / FW;
+      const int gj = j0 + lj < ny ? j0 + lj : 0, gk = k0 + lk < nz ? k0 + lk : 0;   // at most one past
+      const unsigned g = gj + ny * gk;
+#pragma unroll
+      for (int q = 0; q < 6; ++q) v[e][q] = (F + q * plane)[g];
+    }
+#pragma unroll
+    for (int e = 0; e < PER; ++e)
+      if (t + NT * e < NF)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) Fw[q][t + NT * e] = {v[e][2 * q], v[e][2 * q + 1]};
   }
   if (t < 9) dir_total[t] = 0;
   if (t < 2 * FL_N) flag_sh[t / FL_N][t % FL_N] = 0;
@@ -354,18 +368,21 @@ void k_push_tile(TileArgs a0) {
   __syncthreads();
 
   for (int c0 = part * NT; c0 < np; c0 += a.nsplit * NT) {
-    const int slot = base + c0 + t;
-    const long gs = pw + slot;   // the wake's particle arrays, unmoved pointers
+    // the chunk's place in the wake's particle arrays, unmoved pointers: one for the
+    // whole work-group, so that a lane's address is its index beside it (opaque: 13
+    // pointers per lane carried from chunk to chunk would spill)
+    const long g0 = pw + base + c0;
+    const unsigned tl = thread_index();
     const bool active = c0 + t < np;
     int j = 0, k = 0;
     double yp = 0, zp = 0, px = 0, py = 0, pz = 0;
     R djx = 0, djy = 0, djz = 0, drho = 0, dy = 0, dz = 0, partdx = 0, step = 1;
     if (active) {
-      cell_jk(a0.cell[gs], ny, a.ny_magic, j, k);
-      yp = a0.y[gs];
-      zp = a0.z[gs];
+      cell_jk((a0.cell + g0)[tl], ny, a.ny_magic, j, k);
+      yp = (a0.y + g0)[tl];
+      zp = (a0.z + g0)[tl];
       if (!(yp >= 0 && yp <= 1 && zp >= 0 && zp <= 1)) status |= (ST_PARTICLE);
-      px = a0.px[gs]; py = a0.py[gs]; pz = a0.pz[gs];
+      px = (a0.px + g0)[tl]; py = (a0.py + g0)[tl]; pz = (a0.pz + g0)[tl];
       const R rpx = (R)px, rpy = (R)py, rpz = (R)pz;
       // one reciprocal per denominator, then products: the reference divides by
       // the same gamma and 1 - Vx many times over (movepart_splitlayer.cpp:
@@ -550,28 +567,33 @@ void k_push_tile(TileArgs a0) {
         if (d2 > 1 && d2 < ntk_ - 1) status |= (ST_FAR);
       }
       const int dir = (dtj + 1) + 3 * (dtk + 1);
-      // rank among this tile's particles with the same direction, slot order
-      const int ti = thread_index(), lane = ti & 63, wv = ti >> 6;
-      const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+      // rank among this tile's particles with the same direction, slot order: a turn
+      // for each direction that the wave has (most particles stay in the tile)
+      const unsigned ti = thread_index();
+      const int lane = ti & 63, wv = ti >> 6;
       int myrank_w = 0;
-      // kept rolled: nine live ballot masks would spill scalar registers
-#pragma unroll 1
-      for (int d = 0; d < 9; ++d) {
+      if (lane < 9) wave_cnt[wv][lane] = 0;
+      unsigned long long left = __ballot(active);
+      while (left) {
+        const int d = __builtin_amdgcn_readlane(dir, __builtin_ctzll(left));
         const unsigned long long m = __ballot(active && dir == d);
         if (lane == 0) wave_cnt[wv][d] = __popcll(m);
-        if (active && dir == d) myrank_w = __popcll(m & below);
+        if (dir == d)
+          myrank_w = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                               __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+        left &= ~m;
       }
       __syncthreads();
       int off = dir_total[dir];
       for (int q = 0; q < wv; ++q) off += wave_cnt[q][dir];
       if (active) {
-        a0.sy[gs] = ytmp;
-        a0.sz[gs] = ztmp;
-        a0.spx[gs] = px;
-        a0.spy[gs] = py;
-        a0.spz[gs] = pz;
-        a0.scell[gs] = jj + ny * kk;
-        a0.sdest[gs] = dir | (part << 4) | ((off + myrank_w) << 8);
+        (a0.sy + g0)[ti] = ytmp;
+        (a0.sz + g0)[ti] = ztmp;
+        (a0.spx + g0)[ti] = px;
+        (a0.spy + g0)[ti] = py;
+        (a0.spz + g0)[ti] = pz;
+        (a0.scell + g0)[ti] = jj + ny * kk;
+        (a0.sdest + g0)[ti] = dir | (part << 4) | ((off + myrank_w) << 8);
       }
       __syncthreads();
       if (t < 9) {
