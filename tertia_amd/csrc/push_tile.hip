@@ -199,6 +199,77 @@ __device__ inline void deposit_cells(int half, int *cnt, const uint2 *list, cons
   }
 }
 
+// The float form's round: the owner lanes put the lists in order, then every node
+// adds the events of its four corner cells one after the other.  The sums are the
+// sort's below, bit by bit (the same events in the same order): the fields of the
+// split modes are rounded to float between the steps, and another order of these
+// FP64 sums would flip some of those roundings.  Leaves the counts at zero.
+template <int NQ>
+__device__ inline void deposit_lists(int *cnt, uint2 *list, const double *ev_y, const double *ev_z,
+                                     const double (*ev_w)[NT], double (*wacc)[NWIN], bool cic) {
+  const int t = thread_index();
+#pragma unroll 1
+  for (int cell = t; cell < NWIN; cell += NT) {
+    const int n = cnt[cell];
+    if (n < 2) continue;
+    int e[kCell];
+    cell_order<kCell>(list[cell], n, e);
+    uint2 b = {0, 0};
+#pragma unroll
+    for (int i = 0; i < kCell; ++i) (i < 4 ? b.x : b.y) |= (unsigned)(e[i] & 255) << 8 * (i % 4);
+    list[cell] = b;
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int n = t; n < NWIN; n += NT) {
+    double acc[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) acc[q] = wacc[q][n];
+    const int nl_j = n % W, nl_k = n / W;
+    int c[4];
+    uint2 b[4];
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn) {
+      const int cj = nl_j - (cn & 1), ck = nl_k - (cn >> 1);
+      const bool in = cj >= 0 && ck >= 0 && (cic || cn == 0);
+      c[cn] = in ? cnt[ck * W + cj] : 0;
+      b[cn] = list[in ? ck * W + cj : 0];
+    }
+#pragma unroll
+    for (int cn = 0; cn < 4; ++cn) {
+      // four events at a time, their loads together
+#pragma unroll 1
+      for (int i = 0; i < c[cn]; i += 4) {
+        const unsigned four = i ? b[cn].y : b[cn].x;
+        double w[4][NQ], y[4], z[4];
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const int e = i + h < c[cn] ? four >> 8 * h & 255 : four & 255;
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) w[h][q] = ev_w[q][e];
+          y[h] = ev_y[e];
+          z[h] = ev_z[e];
+        }
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const double wy = (cn & 1) ? y[h] : 1. - y[h];
+          const double wz = (cn >> 1) ? z[h] : 1. - z[h];
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) {
+            const double v = cic ? w[h][q] * wy * wz : w[h][q];
+            acc[q] = i + h < c[cn] ? acc[q] + v : acc[q];
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) wacc[q][n] = acc[q];
+  }
+  __syncthreads();
+  for (int i = t; i < NWIN; i += NT) cnt[i] = 0;
+  __syncthreads();
+}
+
 // A round with more than kCell events in some cell: the events sorted by cell and
 // index, every node summing the runs of its four corner cells.
 template <int NQ>
@@ -298,10 +369,6 @@ void k_push_tile(TileArgs a0) {
   // cycles per wave and chunk, a third of the LDS time)
   __shared__ pair_t<FT> Fw[3][NF];
   constexpr int NQ = RHO ? 4 : 3;
-  // The float form always deposits through the sort: its fields are rounded to
-  // float between the steps, and another order of the FP64 sums would flip some of
-  // those roundings.
-  constexpr bool CELLS = sizeof(R) == 8;
   __shared__ double ev_y[NT], ev_z[NT], ev_w[NQ][NT];
   __shared__ double wacc[NQ][NWIN];   // the window's node sums
   // the round's events of each cell, or the sort's arrays in a crowded round
@@ -361,7 +428,7 @@ void k_push_tile(TileArgs a0) {
   if (t < 2 * FL_N) flag_sh[t / FL_N][t % FL_N] = 0;
   int par = 0;
   for (int i = t; i < NWIN; i += NT) {
-    if constexpr (CELLS) sh.cell.cnt[i] = 0;
+    sh.cell.cnt[i] = 0;
 #pragma unroll
     for (int q = 0; q < NQ; ++q) wacc[q][i] = 0.0;
   }
@@ -517,12 +584,10 @@ void k_push_tile(TileArgs a0) {
           ev_w[1][t] = (double)(djy * part_step);
           ev_w[2][t] = (double)(djz * part_step);
           if constexpr (RHO) ev_w[3][t] = (double)(drho * part_step);
-          if constexpr (CELLS) {
-            const int r = atomicAdd(&sh.cell.cnt[cellw], 1);
-            if (r < kCell) reinterpret_cast<uint8_t *>(&sh.cell.list[cellw])[r] = (uint8_t)t;
-            else flag_sh[par][FL_CROWDED] = 1;
-            flag_sh[par][cellw < NT ? FL_HALF0 : FL_HALF1] = 1;
-          }
+          const int r = atomicAdd(&sh.cell.cnt[cellw], 1);
+          if (r < kCell) reinterpret_cast<uint8_t *>(&sh.cell.list[cellw])[r] = (uint8_t)t;
+          else flag_sh[par][FL_CROWDED] = 1;
+          flag_sh[par][cellw < NT ? FL_HALF0 : FL_HALF1] = 1;
         } else {
           status |= (ST_FAR);
         }
@@ -530,19 +595,19 @@ void k_push_tile(TileArgs a0) {
       if (active && partdx > 0.) flag_sh[par][FL_MORE] = 1;
       __syncthreads();
       const int *fl = flag_sh[par];
-      const bool more = fl[FL_MORE], crowded = !CELLS || fl[FL_CROWDED];
+      const bool more = fl[FL_MORE], crowded = fl[FL_CROWDED];
       const bool half0 = fl[FL_HALF0], half1 = fl[FL_HALF1];
       par ^= 1;
       if (t < FL_N) flag_sh[par][t] = 0;   // last read a barrier ago
       if (crowded) {
-        if constexpr (CELLS) __syncthreads();   // the lists give way to the sort
+        __syncthreads();   // the lists give way to the sort
         deposit_sorted<NQ>(cellw, sh.sort.keys, sh.sort.sorted, sh.sort.cstart, sh.sort.cend, ev_y,
                            ev_z, ev_w, wacc, cic);
         __syncthreads();
-        if constexpr (CELLS) {
-          for (int i = t; i < NWIN; i += NT) sh.cell.cnt[i] = 0;
-          __syncthreads();
-        }
+        for (int i = t; i < NWIN; i += NT) sh.cell.cnt[i] = 0;
+        __syncthreads();
+      } else if constexpr (sizeof(R) == 4) {
+        deposit_lists<NQ>(sh.cell.cnt, sh.cell.list, ev_y, ev_z, ev_w, wacc, cic);
       } else {
         // rolled: the code of a work-group's first pass comes from L2 line by line
 #pragma unroll 1
