@@ -145,3 +145,37 @@ def test_global_deposit_cell_counts(oracle_mod, shape, per_cell, hot):
             assert np.array_equal(a, b)
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("shape", [QSS_SHAPE_CIC, QSS_SHAPE_NGP_REF])
+@pytest.mark.parametrize("per_cell", [1, 4, 5, 8, 9])
+def test_float_deposit_cell_counts(oracle_mod, shape, per_cell):
+    """The float form's ordered lists at the same edges.  No fields: a current is the
+    sum of some per_cell terms of a few float products each, so 1e-6 of the largest
+    (ten float roundings are 6e-7); and the same bits twice."""
+    from tertia_amd.mesh import Mesh
+    from tertia_amd.params import PRECISIONS
+    ny = nz = 48
+    rng = np.random.default_rng(per_cell)
+    kw = dict(ny=ny, nz=nz, nslices=2, hx=0.05, shape=shape, ppc_y=2, ppc_z=4)
+    cells = np.sort(rng.permutation(ny * nz)[: ny * nz * 8 // per_cell])
+    cell = np.repeat(cells, per_cell)
+    n = len(cell)
+    parts = ((cell % ny).astype(np.int32), (cell // ny).astype(np.int32),
+             rng.uniform(0.2, 0.8, n), rng.uniform(0.2, 0.8, n),
+             *rng.uniform(-0.1, 0.1, size=(3, n)), np.arange(n, dtype=np.int64))
+    m = Mesh(small(precision=PRECISIONS["mixed32"], **kw), history=())
+    o = oracle_mod.Oracle(small(**kw), history=())
+    try:
+        o.set_particles(*parts)
+        runs = []
+        for _ in range(2):
+            m.set_particles(*parts)
+            m.MoveParticlesLayerSplit(0, 0, 1)
+            runs.append([m.get_field(f) for f in ("Jx", "Jy", "Jz", "Rho")])
+        o.push_deposit(1)
+        for f, a, b in zip(("Jx", "Jy", "Jz", "Rho"), *runs):
+            assert np.array_equal(a, b)
+            assert max_rel(a, o.get_field(f)) <= 1e-6, f
+    finally:
+        m.close()
