@@ -21,14 +21,17 @@ split-BF16-MFMA transforms) and each mode's whole sweep is compared with the
 FP64 sweep: relative L2 over every 8th layer of Ex (the longitudinal field,
 E_z in the usual wakefield notation) and psi.
 
-roofline: the dominant kernel is the transform GEMM; achieved = the flops of
-the transform method in use (2*M*N*K per GEMM pass and field: 4N^3 per 2-D
-transform with the dense tables, 2N^3 with the factored form, whose radix-2
-step halves the multiply-adds; 35 2-D transforms per slice) / its summed
-duration over the instrumented window, each launch timed by a HIP event pair
-that the dispatch itself stamps with its start and end (hipExtLaunchKernel,
-on the context's stream), against MI355X's 78.6 TFLOP/s FP64 MFMA peak;
-dense_equivalent_tflops restates the rate in the dense tables' flops.
+roofline: the transforms along z of the 35 2-D transforms per slice (with the
+fast line transforms, the FP64 default, those along y run inside the Guess and
+Iterate kernels); achieved = the bytes that a pass over a plane cannot do
+without (one plane read, one written per field) / the summed duration over the
+instrumented window, each launch timed by a HIP event pair that the dispatch
+itself stamps with its start and end (hipExtLaunchKernel, on the context's
+stream), against the 8 TB/s HBM peak.  Where a GEMM method was asked for, the
+flops of the method (2*M*N*K per pass and field: 4N^3 per 2-D transform with
+the dense tables, 2N^3 with the factored form, whose radix-2 step halves the
+multiply-adds) against MI355X's 78.6 TFLOP/s FP64 MFMA peak;
+dense_equivalent_tflops restates that rate in the dense tables' flops.
 traffic = HBM bytes per launch from the committed rocprofv3
 FETCH_SIZE/WRITE_SIZE summary of that kernel.  roofline_push: the push+deposit
 kernel against the 8 TB/s HBM peak, its algorithmic bytes per launch being
@@ -681,18 +684,29 @@ def main():
     if "gemm" in base:
         g = base["gemm"]
         factored = base["gemm_tiles"].get("transform_method") == 1
-        line["roofline"] = {"bound": "mfma", "achieved": g["achieved_tflops"],
-                            "peak": PEAK_TFLOPS["fp64"], "unit": "TFLOP/s",
-                            "frac": g["achieved_tflops"] / PEAK_TFLOPS["fp64"],
-                            "traffic": profiled_traffic("k_fact_fp64_512x512" if factored
-                                                        else "k_gemm_fp64_512x512"),
-                            "kernel": ("k_fact_y / k_fact_z (fused factored transform GEMMs, "
-                                       "2N^3 flop per 2-D transform)" if factored else
-                                       "k_gemm<MathF64,...> (transform GEMM, 4N^3 flop per "
-                                       "2-D transform)"),
-                            "dense_equivalent_tflops": g["achieved_tflops"] * (2 if factored
-                                                                               else 1),
-                            "avg_launch_us": g["avg_launch_us"], "launches": g["launches"]}
+        # what the library counts for a slice: tens of N log N per node with the
+        # line transforms, 35 x 2N^3 at least with a GEMM
+        if g["flops"] < a.steps * 2.0 * 512 ** 3:
+            gbs = a.steps * 35 * 2 * 512 * 512 * 8 / (g["ms"] * 1e-3) / 1e9
+            line["roofline"] = {"bound": "hbm", "achieved": gbs, "peak": 8000.0, "unit": "GB/s",
+                                "frac": gbs / 8000.0,
+                                "traffic": profiled_traffic("k_line_cols_fp64_512x512"),
+                                "kernel": "k_line_cols (fast half-integer transforms along z, "
+                                          "with the push field and the residual)",
+                                "flops": g["flops"]}
+        else:
+            line["roofline"] = {"bound": "mfma", "achieved": g["achieved_tflops"],
+                                "peak": PEAK_TFLOPS["fp64"], "unit": "TFLOP/s",
+                                "frac": g["achieved_tflops"] / PEAK_TFLOPS["fp64"],
+                                "traffic": profiled_traffic("k_fact_fp64_512x512" if factored
+                                                            else "k_gemm_fp64_512x512"),
+                                "kernel": ("k_fact_y / k_fact_z (fused factored transform GEMMs, "
+                                           "2N^3 flop per 2-D transform)" if factored else
+                                           "k_gemm<MathF64,...> (transform GEMM, 4N^3 flop per "
+                                           "2-D transform)"),
+                                "dense_equivalent_tflops": g["achieved_tflops"] * (2 if factored
+                                                                                   else 1)}
+        line["roofline"].update(avg_launch_us=g["avg_launch_us"], launches=g["launches"])
         pu = base["push"]
         line["roofline_push"] = {"bound": "hbm", "achieved": pu["achieved_gbs"], "peak": 8000.0,
                                  "unit": "GB/s", "frac": pu["achieved_gbs"] / 8000.0,
