@@ -462,13 +462,16 @@ int  qss_driver_timing(qss_ctx *c, double *ms_clear, double *ms_push);
 
 /* ---- timing of the last qss_sweep/qss_sweep_range (HIP events) --------- */
 /* No counterpart in the reference's layer call surface.
- * Kernel classes: 0 push, 1 transform GEMM, 2 spectral update, 3 beam,
- * 4 counting sort (fill+scan+scatter), 5 deposit tile reduce.              */
+ * Kernel classes: 0 push, 1 transforms (line transforms along z, plain ones,
+ * GEMMs), 2 spectral update (with the row transforms where those are line
+ * transforms; the residual and the history store), 3 beam, 4 counting sort
+ * (clear+scan+scatter), 5 deposit tile reduce.                             */
 #define QSS_NKCLASS 6
 /* on != 0: record a HIP event pair around every launch of the next sweeps.
  * ms_total: wall time of the last sweep window on the stream; ms_kernel[i],
  * launches[i]: summed event time / launch count per class; gemm_flops:
- * algorithmic flops (2*M*N*K per transform pass and field) of the GEMMs.   */
+ * algorithmic flops of class 1 (2*M*N*K per GEMM pass and field, 2.5 N log2 N
+ * per line).                                                               */
 int  qss_enable_timing(qss_ctx *c, int on);
 int  qss_timing(qss_ctx *c, double *ms_total, double *ms_kernel,
                 int64_t *launches, double *gemm_flops);
