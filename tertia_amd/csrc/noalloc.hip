@@ -13,10 +13,11 @@
 // shares that device's scratch, so calls that overlap on one device race; one
 // stream serialises them.
 //
-// Planes whose sides both have a chain of radices (even, no prime factor of the half
-// above 13) go through the line transforms (line.hip): a chain's tables are a few
+// A side that has a chain of radices (even, no prime factor of the half above 13)
+// goes through the line transforms (line.hip): a chain's tables are a few
 // hundred entries where the dense ones are n^2 cosines, and the passes a fraction of
-// the dense products' work.  Dense against lines, us a call: 512 x 512 54.0 / 16.1,
+// the dense products' work; beside a side without one, from kLinePassMin on.  Dense
+// against lines, us a call: 512 x 512 54.0 / 16.1,
 // 312 x 200 38.0 / 18.2, 100 x 100 22.0 / 15.9, 66 x 52 17.8 / 16.8, 12 x 10 16.6 /
 // 14.2 (a context, whose tables stand ready, keeps dense products for loose chains
 // below 192); what is left is three launches and two passes over the plane.
@@ -73,7 +74,7 @@ __global__ __launch_bounds__(256) void k_line_tables(LineAxis y, LineAxis z, dou
   const LineAxis ax = blockIdx.y ? z : y;
   double *const tw = blockIdx.y ? tz : ty;
   const int e = blockIdx.x * 256 + threadIdx.x, n = ax.n, m = ax.m;
-  if (e >= (ax.np - 1) * m) return;
+  if (!ax.np || e >= (ax.np - 1) * m) return;
   const int p = 1 + e / m, i = e - (p - 1) * m;
   int ns = ax.radix(0);
   for (int q = 1; q < p; ++q) ns *= ax.radix(q);
@@ -151,60 +152,73 @@ extern "C" int qss_transform2d_noalloc(int ny, int nz, int kind_z, int kind_y,
   }
   double *Ty = base, *Tz = base + kPlane, *mid = base + 2 * kPlane;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (y.np && z.np) {
-    const int most = std::max((y.np - 1) * y.m, (z.np - 1) * z.m);
+  // one side without a chain: the other one's is worth it from kLinePassMin on
+  // (121 x 256 30.3 / 18.9 us, 300 x 97 32.2 / 21.9, 200 x 35 23.3 / 20.4; 64 x 35 16.7
+  // / 16.8, 26 x 35 16.5 / 19.8)
+  if (!(y.np && z.np)) {
+    if (ny < kLinePassMin) y.np = 0;
+    if (nz < kLinePassMin) z.np = 0;
+  }
+  y.tw = Ty;
+  z.tw = Tz;
+  if (y.np || z.np) {
+    const int most = std::max(y.np ? (y.np - 1) * y.m : 0, z.np ? (z.np - 1) * z.m : 0);
     hipLaunchKernelGGL(k_line_tables, dim3((unsigned)(most + 255) / 256, 2), dim3(256), 0, s, y, z,
                        Ty, Tz);
-    if ((e = hipGetLastError()) != hipSuccess) return fail(hipGetErrorString(e), QSS_E_HIP);
-    y.tw = Ty;
-    z.tw = Tz;
-    if (line_plane_ok(y, z)) {
-      SmallPlaneArgs a{};
-      a.y = y; a.z = z;
-      a.nbatch = a.nw = 1; a.alpha = scale;
-      a.in[0] = in_dev; a.out[0] = out_dev;
-      a.ky[0] = kind_y; a.kz[0] = kind_z;
-      e = launch_line_plane(a, s);
-    } else {
-      RowArgs r{};
-      r.ax = y;
-      r.nz = nz; r.nbatch = r.nw = 1;
-      r.in[0] = in_dev; r.out[0] = mid; r.ky[0] = kind_y;
-      ColArgs c{};
-      c.ax = z;
-      c.ny = ny; c.nbatch = c.nw = 1;
-      c.in[0] = mid; c.out[0] = out_dev; c.kz[0] = kind_z;
-      c.resid[0] = c.push[0] = -1;
-      c.store[0] = 1;
-      c.alpha = scale;
-      if ((e = launch_line_rows(r, s)) == hipSuccess) e = launch_line_cols(c, s);
-    }
+  }
+  if (!y.np)
+    hipLaunchKernelGGL(k_half_integer_table, dim3((unsigned)(((long)ny * ny + 255) / 256)),
+                       dim3(256), 0, s, Ty, ny, kind_y);
+  if (!z.np)
+    hipLaunchKernelGGL(k_half_integer_table, dim3((unsigned)(((long)nz * nz + 255) / 256)),
+                       dim3(256), 0, s, Tz, nz, kind_z);
+  if ((e = hipGetLastError()) != hipSuccess) return fail(hipGetErrorString(e), QSS_E_HIP);
+  if (y.np && z.np && line_plane_ok(y, z)) {
+    SmallPlaneArgs a{};
+    a.y = y; a.z = z;
+    a.nbatch = a.nw = 1; a.alpha = scale;
+    a.in[0] = in_dev; a.out[0] = out_dev;
+    a.ky[0] = kind_y; a.kz[0] = kind_z;
+    e = launch_line_plane(a, s);
     return e == hipSuccess ? QSS_OK : fail(hipGetErrorString(e), QSS_E_HIP);
   }
-  hipLaunchKernelGGL(k_half_integer_table, dim3((unsigned)(((long)ny * ny + 255) / 256)),
-                     dim3(256), 0, s, Ty, ny, kind_y);
-  hipLaunchKernelGGL(k_half_integer_table, dim3((unsigned)(((long)nz * nz + 255) / 256)),
-                     dim3(256), 0, s, Tz, nz, kind_z);
-  if ((e = hipGetLastError()) != hipSuccess) return fail(hipGetErrorString(e), QSS_E_HIP);
-  // the two passes of transform_batch for one FP64 plane, default tile shape
+  // a dense pass: transform_batch's for one FP64 plane, default tile shape
   GemmArgs g{};
   g.nbatch = 1;
   g.nw = 1;
   g.b[0].resid = -1;
   g.b[0].push = -1;
-  g.M = nz; g.N = ny; g.K = ny;
-  g.alpha = 1.0;
-  g.b[0].A = in_dev;
-  g.b[0].B = Ty;
-  g.b[0].C = mid;
-  if ((e = launch_gemm(g, s, QSS_PREC_FP64, 0)) != hipSuccess)
-    return fail(hipGetErrorString(e), QSS_E_HIP);
-  g.M = nz; g.N = ny; g.K = nz;
-  g.alpha = scale;
-  g.b[0].A = Tz;
-  g.b[0].B = mid;
-  g.b[0].C = out_dev;
-  if ((e = launch_gemm(g, s, QSS_PREC_FP64, 0)) != hipSuccess)
-    return fail(hipGetErrorString(e), QSS_E_HIP);
-  return QSS_OK;
+  if (y.np) {
+    RowArgs r{};
+    r.ax = y;
+    r.nz = nz; r.nbatch = r.nw = 1;
+    r.in[0] = in_dev; r.out[0] = mid; r.ky[0] = kind_y;
+    e = launch_line_rows(r, s);
+  } else {
+    g.M = nz; g.N = ny; g.K = ny;
+    g.alpha = 1.0;
+    g.b[0].A = in_dev;
+    g.b[0].B = Ty;
+    g.b[0].C = mid;
+    e = launch_gemm(g, s, QSS_PREC_FP64, 0);
+  }
+  if (e != hipSuccess) return fail(hipGetErrorString(e), QSS_E_HIP);
+  if (z.np) {
+    ColArgs c{};
+    c.ax = z;
+    c.ny = ny; c.nbatch = c.nw = 1;
+    c.in[0] = mid; c.out[0] = out_dev; c.kz[0] = kind_z;
+    c.resid[0] = c.push[0] = -1;
+    c.store[0] = 1;
+    c.alpha = scale;
+    e = launch_line_cols(c, s);
+  } else {
+    g.M = nz; g.N = ny; g.K = nz;
+    g.alpha = scale;
+    g.b[0].A = Tz;
+    g.b[0].B = mid;
+    g.b[0].C = out_dev;
+    e = launch_gemm(g, s, QSS_PREC_FP64, 0);
+  }
+  return e == hipSuccess ? QSS_OK : fail(hipGetErrorString(e), QSS_E_HIP);
 }

@@ -262,6 +262,12 @@ double line_flops(const LineAxis &ax, double cells) {
 }
 
 bool use_lines(const qss_ctx *c) { return c->line_use && c->gemm_force < 0; }
+// the pass along axis i of a plain transform of n fields is a line transform beside
+// a GEMM along the other
+bool use_line_pass(const qss_ctx *c, int i, int n) {
+  return c->line_pass[i] && c->gemm_force < 0 &&
+         (c->line[i].n >= kLinePassMin || (i == 1 && n >= kLinePassBatch));
+}
 
 // transforms along z with the corrector's epilogue; store[b] = 0: the result
 // is not kept, only its push field
@@ -289,6 +295,18 @@ int line_cols(qss_ctx *c, int n, const int *kz, const double *const *in, double 
 }
 
 // transform_batch: y pass in -> tmp, z pass tmp -> out
+int line_rows(qss_ctx *c, int n, const int *ky, const double *const *in, bool one_wake) {
+  RowArgs r{};
+  r.ax = c->line[0];
+  r.nz = c->nz; r.nbatch = n; r.nw = one_wake ? 1 : c->nw;
+  r.nc = c->ncell;
+  for (int b = 0; b < n; ++b) { r.in[b] = in[b]; r.out[b] = c->tmp[b]; r.ky[b] = ky[b]; }
+  Timed t(c, KC_GEMM, true);
+  HIPCHECK(launch_line_rows(r, c->stream, t.e0, t.e1));
+  if (c->timing) c->gemm_flops += line_flops(r.ax, (double)c->ncell * n * r.nw);
+  return QSS_OK;
+}
+
 int transform_line(qss_ctx *c, int n, const int *kz, const int *ky, const double *const *in,
                    double *const *out, double alpha, const int *resid, const int *push,
                    const double *const *pplane, double beta, bool one_wake) {
@@ -306,16 +324,7 @@ int transform_line(qss_ctx *c, int n, const int *kz, const int *ky, const double
                        line_flops(a.z, (double)c->ncell * n * a.nw);
     return QSS_OK;
   }
-  RowArgs r{};
-  r.ax = c->line[0];
-  r.nz = c->nz; r.nbatch = n; r.nw = one_wake ? 1 : c->nw;
-  r.nc = c->ncell;
-  for (int b = 0; b < n; ++b) { r.in[b] = in[b]; r.out[b] = c->tmp[b]; r.ky[b] = ky[b]; }
-  {
-    Timed t(c, KC_GEMM, true);
-    HIPCHECK(launch_line_rows(r, c->stream, t.e0, t.e1));
-  }
-  if (c->timing) c->gemm_flops += line_flops(r.ax, (double)c->ncell * n * r.nw);
+  CHECK(line_rows(c, n, ky, in, one_wake));
   return line_cols(c, n, kz, c->tmp, out, alpha, resid, push, pplane, beta, one_wake);
 }
 
@@ -388,11 +397,17 @@ int transform_batch(qss_ctx *c, int n, const int *kz, const int *ky,
     g.b[b].resid = -1;
     g.b[b].push = -1;
   }
-  {
-    Timed t(c, KC_GEMM, true);
-    HIPCHECK(launch_gemm(g, c->stream, c->p.precision, gemm_pick(c, 0, n), t.e0, t.e1));
+  if (use_line_pass(c, 0, n)) {
+    CHECK(line_rows(c, n, ky, in, one_wake));
+  } else {
+    {
+      Timed t(c, KC_GEMM, true);
+      HIPCHECK(launch_gemm(g, c->stream, c->p.precision, gemm_pick(c, 0, n), t.e0, t.e1));
+    }
+    if (c->timing) c->gemm_flops += 2.0 * g.M * g.N * g.K * n * g.nw;
   }
-  if (c->timing) c->gemm_flops += 2.0 * g.M * g.N * g.K * n * g.nw;
+  if (use_line_pass(c, 1, n))
+    return line_cols(c, n, kz, c->tmp, out, alpha, resid, push, pplane, beta, one_wake);
   g.M = c->nz; g.N = c->ny; g.K = c->nz;
   g.alpha = alpha;
   g.beta = beta;
@@ -1293,18 +1308,17 @@ int qss_create(const qss_params *p, int device, uint32_t history_mask, qss_ctx *
     }
   }
   // line transforms (line.hip)
-  c->line_plain = c->line_use = p->precision == QSS_PREC_FP64;
-  for (int i = 0; i < 2 && c->line_use; ++i) {
+  c->line_use = p->precision == QSS_PREC_FP64;
+  for (int i = 0; i < 2 && p->precision == QSS_PREC_FP64; ++i) {
     LineAxis &ax = c->line[i];
     const bool fast = line_chain(i == 0 ? c->ny : c->nz, &ax);
     ax.Tc = c->d_T[2 * i];
     ax.Ts = c->d_T[2 * i + 1];
     if (!fast) {
-      c->line_plain = false;
-      c->line_use = ax.n <= (i == 0 ? kLineDenseY : kLineDenseZ);
+      c->line_use = c->line_use && ax.n <= (i == 0 ? kLineDenseY : kLineDenseZ);
       continue;
     }
-    if (!line_fixed(ax) && ax.n < kLineLooseMin) c->line_plain = false;
+    c->line_pass[i] = line_fixed(ax) || ax.n >= kLineLooseMin;
     std::vector<double> tw;
     line_table(ax, tw);
     if ((r = dalloc(&c->d_linetw[i], tw.size())) != QSS_OK) return fail(r);
@@ -1315,6 +1329,10 @@ int qss_create(const qss_params *p, int device, uint32_t history_mask, qss_ctx *
       return fail(QSS_E_HIP);
     }
   }
+  c->line_plain = c->line_use && c->line_pass[0] && c->line_pass[1];
+  if (!c->line_plain)
+    for (int i = 0; i < 2; ++i)
+      c->line_pass[i] = c->line_pass[i] && line_fixed(c->line[i]);
   if ((r = dalloc(&c->F, ncw * kPushComp)) != QSS_OK) return fail(r);
   if (c->mixed && (r = dalloc(&c->Ff, ncw * kPushComp)) != QSS_OK) return fail(r);
   if (nw > 1) {
@@ -1965,7 +1983,8 @@ int qss_set_transform_method(qss_ctx *c, int method) {
     return QSS_E_ARG;
   }
   graph_free(c);   // a captured graph holds the other method's launches
-  c->line_plain = c->line_use = false;   // a GEMM method was asked for
+  // a GEMM method was asked for
+  c->line_plain = c->line_use = c->line_pass[0] = c->line_pass[1] = false;
   c->fact_use = method == QSS_TRANSFORM_FACTORED;
   return QSS_OK;
 }

@@ -148,6 +148,15 @@ void fact_fused_twiddles(int n, std::vector<double> &tw);
 // 1.17)
 // ---------------------------------------------------------------------------
 constexpr int kLineDenseY = 128, kLineDenseZ = 256, kLineLooseMin = 192;
+// A line pass next to a GEMM pass (one side without a chain), planes in us, GEMM only
+// against this: side 512 31.7 / 24.0 (by 121, one plane) and 37.0 / 27.7 (by 121,
+// eight), 256 35.5 / 30.9 (by 313, four); 96 23.9 / 24.1, 64 21.8 / 22.0, 32 20.5 /
+// 20.7; a chain not compiled, 200 24.0 / 28.0 (by 35, eight)
+constexpr int kLinePassMin = 128;
+// ... or, along z, batches of a Guess or Iterate: 24 layers of a 199 x 64 deck 7.22 ms
+// by GEMMs, 6.88 with its six and eight fields' passes along z as lines; a batch of
+// eight 20.9 us / 19.7 at 33 x 48 (along y, 48 x 33, 20.8 / 21.4)
+constexpr int kLinePassBatch = 6;
 // transforms along z of nbatch planes: out = alpha T_z in (+ beta out), with
 // the corrector epilogue
 struct ColArgs {
@@ -312,6 +321,10 @@ struct qss_ctx {
   // line transforms (line.hip), in use until a GEMM method or tile shape is
   // asked for
   bool line_plain = false, line_use = false;   // transforms by themselves; layer steps
+  // the passes of a plain transform (y, z) that are line transforms: a compiled chain
+  // or one from kLineLooseMin on; where only one side has that, a compiled one (from
+  // kLinePassMin on, along z also for batches from kLinePassBatch on), and the other pass is a GEMM
+  bool line_pass[2] = {};
   LineAxis line[2];                  // y, z
   double *d_linetw[2] = {};
   double *F = nullptr;               // push field

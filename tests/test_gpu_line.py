@@ -82,3 +82,42 @@ def test_noalloc_lines_vs_oracle(oracle_mod, nz, ny):
                 assert np.array_equal(m.get_field("Rho"), got)
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("nz,ny", [(35, 64), (64, 35), (97, 200), (313, 256), (192, 313), (19, 32)])
+def test_one_line_pass_vs_oracle(oracle_mod, nz, ny):
+    """One side with a chain, the other dense: a line pass and a GEMM pass, of one plane,
+    of a batch and of the context-free call."""
+    import ctypes
+    from tertia_amd.mesh import Mesh
+    m = Mesh(small(ny=ny, nz=nz, nslices=1), history=())
+    try:
+        x = np.random.default_rng(ny + 1000 * nz).standard_normal((nz, ny))
+        for kz in (0, 1):
+            for ky in (0, 1):
+                ref = 0.25 * oracle_mod.transform2d(x, kz, ky, use_fft=False, nthreads=4)
+                assert max_rel(m.transform2d(x, kz, ky, 0.25), ref) < 1e-13, (kz, ky)
+                m.set_field("Rho", x)
+                assert m.L.qss_transform2d_noalloc(ny, nz, kz, ky, m.layer_ptr("Rho"),
+                                                   m.layer_ptr("Jx"), 0.25,
+                                                   ctypes.c_void_p(m.stream)) == 0
+                assert max_rel(m.get_field("Jx"), ref) < 1e-13, (kz, ky)
+    finally:
+        m.close()
+
+
+@pytest.mark.parametrize("ny,nz,kw", [(151, 96, {}), (64, 313, {"n_iter": 1}), (313, 35, {})])
+def test_sweep_with_one_line_pass_vs_oracle(oracle_mod, ny, nz, kw):
+    """Sides beyond the dense rows' limit: the layer step's transforms by passes, the
+    push field and the residual in the column pass or in the GEMM."""
+    from tertia_amd.mesh import Mesh
+    p = small(ny=ny, nz=nz, nslices=8, **kw)
+    m, o = Mesh(p, history=("Ex", "Psi")), oracle_mod.Oracle(p, history=("Ex", "Psi"))
+    try:
+        rg, ro = m.MoveAllSplitLayers(), o.sweep()
+        for f in ("Ex", "Psi"):
+            a = np.stack([m.history(f, s) for s in range(p.nslices)])
+            b = np.stack([o.history(f, s) for s in range(p.nslices)])
+            assert np.linalg.norm(a - b) <= 1e-10 * np.linalg.norm(b), f
+    finally:
+        m.close()
