@@ -215,9 +215,12 @@ int  qss_transform2d_batched(qss_ctx *c, int n, const int *kind_z,
  * uses (1..8 fields, both passes, the 6- and 8-field inverse passes with
  * their corrector epilogue) and keeps the fastest.  It also picks the
  * particles per work-group of the tiled push (qss_set_particle_split) by
- * timing a predictor pass.  It overwrites only scratch state (transform
- * intermediates, the push field and residual slots that the next layer step
- * rebuilds).  reps >= 1.                                                   */
+ * timing a predictor pass.  In the mixed modes, where another order of the
+ * sums shows in the results, it keeps the fastest of the shapes that sum in
+ * one order, and order and particle split depend on grid and precision only:
+ * tuned contexts of the same parameters return the same bits.  It overwrites
+ * only scratch state (transform intermediates, the push field and residual
+ * slots that the next layer step rebuilds).  reps >= 1.                     */
 int  qss_autotune(qss_ctx *c, int reps, float *table_ms);
 /* table_ms (may be NULL): 2*8*qss_gemm_variants(precision) floats, the mean
  * time of one launch for [pass][nbatch-1][variant].                         */

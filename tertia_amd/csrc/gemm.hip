@@ -642,7 +642,7 @@ __global__ __launch_bounds__(256) void k_split(SplitArgs a) {
 // ---------------------------------------------------------------------------
 typedef void (*GemmFn)(GemmArgs);
 struct Variant {
-  int bm, bn, bk, nt;
+  int bm, bn, bk, ks, nt;
   // [guarded][store]: store 0 = plain, 1 = with epilogue work (beta, residual,
   // push field), 2 = transposed split store (split-bf16 y pass)
   GemmFn fn[2][3];
@@ -650,7 +650,7 @@ struct Variant {
 };
 
 #define QSS_GEMM_DENSE(MT, BM, BN, BK, WGM, WGN, KS)                                   \
-  Variant{BM, BN, BK, Cfg<BM, BN, BK, WGM, WGN, KS>::NT,                               \
+  Variant{BM, BN, BK, KS, Cfg<BM, BN, BK, WGM, WGN, KS>::NT,                           \
           {{k_gemm<MT, BM, BN, BK, WGM, WGN, KS, false, false>,                        \
             k_gemm<MT, BM, BN, BK, WGM, WGN, KS, false, true>, nullptr},               \
            {k_gemm<MT, BM, BN, BK, WGM, WGN, KS, true, false>,                         \
@@ -658,7 +658,7 @@ struct Variant {
           #BM "x" #BN "x" #BK "_w" #WGM "x" #WGN "_k" #KS}
 
 #define QSS_GEMM_BF16(NPC, BM, BN, BK, WGM, WGN)                                       \
-  Variant{BM, BN, BK, WGM * WGN * 64,                                                  \
+  Variant{BM, BN, BK, 1, WGM * WGN * 64,                                               \
           {{k_gemm_bf16<BM, BN, BK, WGM, WGN, NPC, false, false, false>,               \
             k_gemm_bf16<BM, BN, BK, WGM, WGN, NPC, false, false, true>,                \
             k_gemm_bf16<BM, BN, BK, WGM, WGN, NPC, false, true>},                      \
@@ -709,7 +709,7 @@ const Variant kF32[] = {
 };
 
 #define QSS_GEMM_BF16K(NPC, BM, BN, BK, WGM, WGN, KS)                                  \
-  Variant{BM, BN, BK, WGM * WGN * KS * 64,                                             \
+  Variant{BM, BN, BK, KS, WGM * WGN * KS * 64,                                         \
           {{k_gemm_bf16<BM, BN, BK, WGM, WGN, NPC, false, false, false, KS>,           \
             k_gemm_bf16<BM, BN, BK, WGM, WGN, NPC, false, false, true, KS>,            \
             k_gemm_bf16<BM, BN, BK, WGM, WGN, NPC, false, true, true, KS>},            \
@@ -756,6 +756,62 @@ Table table(int prec) {
 }  // namespace
 
 int gemm_num_variants(int prec) { return table(prec).n; }
+
+// The order in which a mixed-precision shape sums an element's products is its slab
+// depth bk and the waves ks that share a slab: shapes that agree in both give the
+// same bits, others differ in the last bits of a float, 1e-8 of a field after a
+// sweep.  Which of two shapes is the faster often turns on a per cent that changes
+// from one timing to the next (y pass of three 512^2 planes, split in three: 64 deep
+// by two waves 14.3 us, 32 deep 14.3 us, 17 and 11 of 28 contexts), so the tuner picks
+// the shape and this rule the order: what a tuned sweep returns does not depend on a
+// clock.  The rule is the order that was fastest most often on 95 grids of 48 to 512
+// (sides multiples of 16; passes of 2, 3, 6 and 8 planes), by
+//   t32, t64  work-groups of 32- and 64-sided tiles; fill: the share of the CUs that
+//             rounds of the latter use
+//   edge      tiles that are not full: every shape then checks its bounds
+// Split forms: a launch that leaves CUs idle splits its slabs over waves (256^2, 3
+// planes: 7.0 us against 7.8), with 4 of them where the longer slab costs no padding
+// (48 x 256: 9.2 against 9.6); one that fills them is faster with shallow slabs and no
+// split (512^2, 8 planes: 23.1 against 25.8), and a K that is an odd multiple of 64 has
+// 32 deep slabs alone without checks (320^2: 7.9 against 14.6).  Float: four waves per
+// 32-sided tile unless 64-sided ones fill their rounds (320^2, 8 planes: 15.9 against
+// 19.6 us).
+bool gemm_same_order(int prec, int variant, int M, int N, int K, int planes, bool zpass) {
+  if (prec == QSS_PREC_FP64) return true;
+  const auto up = [](int a, int b) { return (a + b - 1) / b; };
+  const int t32 = up(M, 32) * up(N, 32) * planes, t64 = up(M, 64) * up(N, 64) * planes;
+  const bool edge = M % 32 || N % 32;
+  const double fill = t64 / (256.0 * up(t64, 256));
+  int bk, ks;
+  if (prec == QSS_PREC_MIXED32) {
+    bk = 16;
+    if (M % 64 == 0 && N % 64 == 0) ks = fill > 0.75 ? 2 : 4;
+    else ks = edge && t64 > 150 && (zpass || fill > 0.6) ? 2 : 4;
+  } else {
+    const bool three = prec == QSS_PREC_MIXED_BF16X6;
+    if (edge || K % 64) {
+      bk = 64; ks = 2;
+      if (up(K, 128) * 2 == up(K, 64) && (K % 64 == 0 || (K >= 320 && K % 32 == 0)) && t32 <= 256) {
+        bk = 128; ks = 4;
+      } else if (!edge && t64 > (three ? 256 : 300)) {
+        bk = 32; ks = 1;
+      } else if (edge && !three && t64 > 256) {
+        ks = 1;
+      }
+    } else if (K % 128) {
+      bk = 32; ks = 1;
+    } else if (t32 <= 256) {
+      const bool deep = three || K > 128;
+      bk = deep ? 64 : 32; ks = deep ? 2 : 1;
+    } else if (K >= 384 && t64 <= (three ? 256 : 128)) {
+      bk = 64; ks = 2;
+    } else {
+      bk = !three && K >= 384 && (zpass || fill > 0.8) ? 64 : 32; ks = 1;
+    }
+  }
+  const Variant &v = table(prec).v[variant];
+  return v.bk == bk && v.ks == ks;
+}
 const char *gemm_variant_name(int prec, int v) {
   const Table tb = table(prec);
   return (v >= 0 && v < tb.n) ? tb.v[v].name : "";

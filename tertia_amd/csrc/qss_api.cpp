@@ -2123,7 +2123,10 @@ int qss_autotune(qss_ctx *c, int reps, float *table_ms) {
         float ms = 0.f;
         (void)hipEventElapsedTime(&ms, e0, e1);
         if (table_ms) table_ms[(pass * kGemmMaxBatch + (b - 1)) * nv + v] = ms / reps;
-        if (ms < best) { best = ms; bestv = v; }
+        if (ms < best && gemm_same_order(prec, v, g.M, g.N, g.K, b * c->nw, pass == 1)) {
+          best = ms;
+          bestv = v;
+        }
       }
       c->gemm_var[pass][b] = bestv;
     }
@@ -2197,9 +2200,19 @@ int qss_autotune(qss_ctx *c, int reps, float *table_ms) {
       }
       c->ffv[pass][b] = bestv;
     }
-  // work-groups per tile of the push: one predictor pass (state unchanged)
-  // plus the window combine into scratch planes, per candidate
-  if (rc == QSS_OK && c->tiled && c->np > 0) {
+  // work-groups per tile of the push.  Mixed modes: by the number of tiles, since the
+  // split sets the order of the deposit's sums, whose last bits flip roundings of the
+  // float fields (1e-8 of a field after a sweep); the lines lie where timing put them
+  // (4 up to 169 tiles, 2 from 195 to 512, 1 from 529; 256 tiles 2 in three contexts of
+  // four).  No more parts than a tile has chunks of 256 particles.
+  if (rc == QSS_OK && c->tiled && c->mixed) {
+    const long nt = (long)c->ntj * c->ntk * c->nw, per_tile = c->np_cap / (c->ntj * c->ntk);
+    c->nsplit = nt > 512 ? 1 : nt > 180 ? 2 : 4;
+    while (c->nsplit > 1 && (c->nsplit - 1) * 256 >= per_tile) c->nsplit /= 2;
+  }
+  // FP64: one predictor pass (state unchanged) plus the window combine into scratch
+  // planes, per candidate
+  if (rc == QSS_OK && c->tiled && !c->mixed && c->np > 0) {
     double *const outs[4] = {c->tmp[0], c->tmp[1], c->tmp[2], c->tmp[3]};
     float best = 1e30f;
     int bests = c->nsplit;

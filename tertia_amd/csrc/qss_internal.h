@@ -72,6 +72,9 @@ hipError_t launch_gemm(const GemmArgs &a, hipStream_t s, int prec, int variant,
                        hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 int gemm_num_variants(int prec);
 const char *gemm_variant_name(int prec, int v);
+// the variant sums its products in the order that a tuned launch of this shape uses
+// (FP64: any order, its differences are roundings of 1e-16)
+bool gemm_same_order(int prec, int variant, int M, int N, int K, int planes, bool zpass);
 int gemm_pieces(int prec);   // bf16 pieces per operand element (0: not split)
 // out[b] (npc planes of n bf16) = pieces of in[b] (n doubles), b < nb
 hipError_t launch_split_bf16(const double *const *in, uint16_t *const *out, int nb, long n,
