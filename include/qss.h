@@ -202,7 +202,8 @@ int  qss_copy_c_to_p(qss_ctx *c);
  * `in` and `out` may not alias.                                             */
 int  qss_transform2d(qss_ctx *c, int kind_z, int kind_y, const double *in_dev,
                      double *out_dev, double scale);
-/* Batched form: n transforms in one launch pair. */
+/* Batched form: n transforms in one launch or two.  An output may be another
+ * entry's input: every input is read before any such output is written.     */
 int  qss_transform2d_batched(qss_ctx *c, int n, const int *kind_z,
                              const int *kind_y, const double *const *in_dev,
                              double *const *out_dev, double scale);

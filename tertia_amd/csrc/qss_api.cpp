@@ -307,10 +307,26 @@ int line_rows(qss_ctx *c, int n, const int *ky, const double *const *in, bool on
   return QSS_OK;
 }
 
+// no output lies on an input, other than a plane on its own: then the planes may be
+// transformed one by one in any order
+bool planes_apart(int n, const double *const *in, double *const *out, long len) {
+  const uintptr_t bytes = (uintptr_t)len * sizeof(double);
+  for (int i = 0; i < n; ++i)
+    for (int o = 0; o < n; ++o) {
+      if (i == o && in[i] == out[o]) continue;
+      const uintptr_t x = (uintptr_t)in[i], y = (uintptr_t)out[o];
+      if (x < y + bytes && y < x + bytes) return false;
+    }
+  return true;
+}
+
 int transform_line(qss_ctx *c, int n, const int *kz, const int *ky, const double *const *in,
                    double *const *out, double alpha, const int *resid, const int *push,
                    const double *const *pplane, double beta, bool one_wake) {
-  if (!resid && !push && beta == 0.0 && line_plane_ok(c->line[0], c->line[1])) {
+  // the two passes below read every input before an output is written; the one launch
+  // of small planes does so plane by plane
+  if (!resid && !push && beta == 0.0 && line_plane_ok(c->line[0], c->line[1]) &&
+      planes_apart(n, in, out, c->ncell * (one_wake ? 1 : c->nw))) {
     SmallPlaneArgs a{};
     a.y = c->line[0]; a.z = c->line[1];
     a.nbatch = n; a.nw = one_wake ? 1 : c->nw; a.nc = c->ncell; a.alpha = alpha;
