@@ -103,11 +103,12 @@ def parse():
     ap.add_argument("--gemm-tiles", default="", metavar="Y/Z[/FY/FZ]",
                     help="FP64 transform tile variants per batch size 1..8 for the y and z "
                          "passes, e.g. 11,12,11,13,11,14,0,0/11,12,12,13,11,15,0,2, then "
-                         "optionally those of the fused factored kernels "
-                         "(default: the autotuner's choice)")
+                         "optionally those of the fused factored kernels; runs the GEMM "
+                         "form of the transforms (default: no GEMM where lines run, else "
+                         "the autotuner's choice)")
     ap.add_argument("--transform", default="auto", choices=("auto", "dense", "factored"),
                     help="2-D transform method of the FP64 sweeps (auto: the context's "
-                         "default, factored on grids of at least 256^2)")
+                         "default, line transforms)")
     ap.add_argument("--particle-split", type=int, default=0, choices=(0, 1, 2, 4),
                     help="work-groups per tile of the push (0: the autotuner's choice)")
     ap.add_argument("--library-gemm", action="store_true",
@@ -249,7 +250,8 @@ def timed_run(mode, a):
         if a.gemm_tiles and mode == "fp64":
             # a fixed tile table (y-pass and z-pass variant per batch size 1..8;
             # then optionally those of the fused factored kernels) instead of
-            # the tuned one, e.g. to repeat a run's kernels exactly
+            # the tuned one, and the GEMM form that has these shapes instead of lines
+            m.transform_method = m.transform_method
             parts = [[int(v) for v in part.split(",")] for part in a.gemm_tiles.split("/")]
             c = m.gemm_choice()
             c.update({"y_pass": parts[0], "z_pass": parts[1]})
@@ -684,9 +686,7 @@ def main():
     if "gemm" in base:
         g = base["gemm"]
         factored = base["gemm_tiles"].get("transform_method") == 1
-        # what the library counts for a slice: tens of N log N per node with the
-        # line transforms, 35 x 2N^3 at least with a GEMM
-        if g["flops"] < a.steps * 2.0 * 512 ** 3:
+        if base["gemm_tiles"].get("transform_in_use") == 2:   # line transforms
             gbs = a.steps * 35 * 2 * 512 * 512 * 8 / (g["ms"] * 1e-3) / 1e9
             line["roofline"] = {"bound": "hbm", "achieved": gbs, "peak": 8000.0, "unit": "GB/s",
                                 "frac": gbs / 8000.0,

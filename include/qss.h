@@ -363,16 +363,21 @@ int  qss_unpack_layer_record(qss_ctx *c, const double *src, size_t n);
  * least 256).  Where ny and nz are multiples of 128 (at most 1024) the
  * twiddles run inside the two GEMMs; elsewhere in twiddle kernels between
  * them.  Contexts start FACTORED where the twiddles run inside the GEMMs
- * (measured faster at 256^2, 384^2 and 512^2) and DENSE otherwise.  FP64
- * contexts whose axes allow it run O(N log N) line transforms instead of
- * either GEMM form until a method is set here or a tile shape is forced
- * (qss_set_gemm_variant); qss_transform_method names the GEMM form all the
- * while.  Results agree to rounding.  Setting a method drops a captured
- * graph.                                                                     */
+ * (measured faster at 256^2, 384^2 and 512^2) and DENSE otherwise.
+ * LINES: O(N log N) line transforms instead of either GEMM form, in every FP64
+ * context with a side that has them; such contexts start so.
+ * qss_transform_method names the GEMM form that runs where lines do not;
+ * qss_transform_in_use names what runs: LINES, or that form once it was set
+ * or a tile shape is forced (qss_set_gemm_variant).  Setting LINES returns a
+ * context to what it ran when it was created, and what qss_transform_in_use
+ * returned can be set again.  Results agree to rounding.  Setting a method
+ * drops a captured graph.                                                    */
 #define QSS_TRANSFORM_DENSE    0
 #define QSS_TRANSFORM_FACTORED 1
+#define QSS_TRANSFORM_LINES    2
 int  qss_set_transform_method(qss_ctx *c, int method);
 int  qss_transform_method(const qss_ctx *c);
+int  qss_transform_in_use(const qss_ctx *c);
 /* The FACTORED method's tile shapes (qss_autotune tunes them), 4 blocks of
  * 9 ints, each indexed by batch size 0..8 like qss_gemm_choice: the GEMMs of
  * the twiddle-kernel form (y pass, z pass; FP64 variants), then the fused

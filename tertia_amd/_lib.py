@@ -57,6 +57,7 @@ SIGNATURES = {
     "qss_unpack_layer": (ctypes.c_int, [_vp, _vp, ctypes.c_size_t]),
     "qss_set_transform_method": (ctypes.c_int, [_vp, ctypes.c_int]),
     "qss_transform_method": (ctypes.c_int, [_vp]),
+    "qss_transform_in_use": (ctypes.c_int, [_vp]),
     "qss_fact_choice": (ctypes.c_int, [_vp, _ip]),
     "qss_set_fact_choice": (ctypes.c_int, [_vp, _ip]),
     "qss_transform2d_noalloc": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int,

@@ -261,11 +261,14 @@ double line_flops(const LineAxis &ax, double cells) {
   return cells * (ax.np ? 2.5 * std::log2((double)ax.n) : 2.0 * ax.n);
 }
 
-bool use_lines(const qss_ctx *c) { return c->line_use && c->gemm_force < 0; }
+bool lines_on(const qss_ctx *c) { return !c->line_off && c->gemm_force < 0; }
+bool use_lines(const qss_ctx *c) { return c->line_use && lines_on(c); }
+// some transform of the context is or has a line pass
+bool has_lines(const qss_ctx *c) { return c->line_use || c->line_pass[0] || c->line_pass[1]; }
 // the pass along axis i of a plain transform of n fields is a line transform beside
 // a GEMM along the other
 bool use_line_pass(const qss_ctx *c, int i, int n) {
-  return c->line_pass[i] && c->gemm_force < 0 &&
+  return c->line_pass[i] && lines_on(c) &&
          (c->line[i].n >= kLinePassMin || (i == 1 && n >= kLinePassBatch));
 }
 
@@ -1989,7 +1992,8 @@ int qss_set_particles(qss_ctx *c, int64_t n, const int32_t *cell_j, const int32_
 }
 
 int qss_set_transform_method(qss_ctx *c, int method) {
-  if (!c || (method != QSS_TRANSFORM_DENSE && method != QSS_TRANSFORM_FACTORED)) {
+  if (!c || (method != QSS_TRANSFORM_DENSE && method != QSS_TRANSFORM_FACTORED &&
+             method != QSS_TRANSFORM_LINES)) {
     qss_set_error("unknown transform method");
     return QSS_E_ARG;
   }
@@ -1998,16 +2002,24 @@ int qss_set_transform_method(qss_ctx *c, int method) {
                   std::to_string(kFactMinN));
     return QSS_E_ARG;
   }
+  if (method == QSS_TRANSFORM_LINES && !has_lines(c)) {
+    qss_set_error("line transforms need FP64 and a side that has them");
+    return QSS_E_ARG;
+  }
   graph_free(c);   // a captured graph holds the other method's launches
-  // a GEMM method was asked for
-  c->line_plain = c->line_use = c->line_pass[0] = c->line_pass[1] = false;
-  c->fact_use = method == QSS_TRANSFORM_FACTORED;
+  c->line_off = method != QSS_TRANSFORM_LINES;
+  c->fact_use = method == QSS_TRANSFORM_LINES ? c->ffused_ok : method == QSS_TRANSFORM_FACTORED;
   return QSS_OK;
 }
 
 int qss_transform_method(const qss_ctx *c) {
   if (!c) return QSS_E_ARG;
   return c->fact_use ? QSS_TRANSFORM_FACTORED : QSS_TRANSFORM_DENSE;
+}
+
+int qss_transform_in_use(const qss_ctx *c) {
+  if (!c) return QSS_E_ARG;
+  return has_lines(c) && lines_on(c) ? QSS_TRANSFORM_LINES : qss_transform_method(c);
 }
 
 int qss_gemm_variants(int precision) {

@@ -321,8 +321,9 @@ struct qss_ctx {
   double2 *d_tw[2] = {};
   double *tmp2[kGemmMaxBatch] = {};
   int fact_var[2][kGemmMaxBatch + 1] = {};
-  // line transforms (line.hip), in use until a GEMM method or tile shape is
-  // asked for
+  // line transforms (line.hip): what the axes allow, and whether a GEMM method was
+  // asked for instead
+  bool line_off = false;
   bool line_plain = false, line_use = false;   // transforms by themselves; layer steps
   // the passes of a plain transform (y, z) that are line transforms: a compiled chain
   // or one from kLineLooseMin on; where only one side has that, a compiled one (from

@@ -387,7 +387,8 @@ class Mesh:
         check(self.L.qss_gemm_choice(self.h, arr), "qss_gemm_choice")
         out = {"y_pass": list(arr[1:9]), "z_pass": list(arr[10:18]),
                "particle_split": self.particle_split,
-               "transform_method": self.transform_method}
+               "transform_method": self.transform_method,
+               "transform_in_use": self.transform_in_use}
         fa = (ctypes.c_int * 36)()
         check(self.L.qss_fact_choice(self.h, fa), "qss_fact_choice")
         out["fact_y_pass"] = list(fa[1:9])
@@ -433,12 +434,19 @@ class Mesh:
 
     @property
     def transform_method(self) -> int:
-        """QSS_TRANSFORM_DENSE (0) or QSS_TRANSFORM_FACTORED (1)."""
+        """The GEMM form, QSS_TRANSFORM_DENSE (0) or QSS_TRANSFORM_FACTORED (1); setting
+        QSS_TRANSFORM_LINES (2) returns to line transforms.  To restore a method
+        later, keep `transform_in_use`."""
         return self.L.qss_transform_method(self.h)
 
     @transform_method.setter
     def transform_method(self, method: int) -> None:
         check(self.L.qss_set_transform_method(self.h, int(method)), "qss_set_transform_method")
+
+    @property
+    def transform_in_use(self) -> int:
+        """What the transforms run: QSS_TRANSFORM_LINES (2) or the GEMM form."""
+        return self.L.qss_transform_in_use(self.h)
 
     @staticmethod
     def gemm_variants(precision: int = 0) -> int:
