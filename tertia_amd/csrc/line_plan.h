@@ -51,7 +51,10 @@ inline bool line_big(const LineAxis &ax) {
 // n / 2 above 13, or beyond 512.  Other lengths than the fixed ones take the
 // cheapest chain (cycles of one wave, fitted by hand): per pass an exchange
 // through LDS, per butterfly of a thread its loads, products and DFT; primes from 5
-// on cost their square.
+// on cost their square.  Radices above 8 only where m has no chain without: the row
+// kernels that hold them spill, which costs more than a pass more does (layers of
+// 288 x 288 as 12 12 321 us, as 3 6 8 218; 480 x 480 459, 327; 162 x 162 as 9 9 269, as
+// 3 3 3 3 228; planes of 216 x 216 29.3, 24.3).
 inline bool line_chain(int n, LineAxis *ax) {
   ax->n = n;
   ax->np = 0;
@@ -73,6 +76,7 @@ inline bool line_chain(int n, LineAxis *ax) {
     return 300.0 +
            ((m / r + kLineT - 1) / kLineT) * (40.0 * r + (prime ? 4.0 * r * r : 0.0));
   };
+  int most = 8;   // the largest radix to try
   const std::function<void(int, int, double)> search = [&](int p, int left, double c) {
     if (c >= best) return;
     if (left == 1 && p >= 2) {
@@ -82,7 +86,7 @@ inline bool line_chain(int n, LineAxis *ax) {
       return;
     }
     if (p == kLinePasses) return;
-    for (int r = left == 1 ? 1 : 2; r <= (left == 1 ? 1 : 13); ++r) {
+    for (int r = left == 1 ? 1 : 2; r <= (left == 1 ? 1 : most); ++r) {
       // radix 1: the second pass of a prime m
       if (left % r || m / r > 2 * kLineT || (r == 1 && m > 13)) continue;
       R = (R & ~(15u << 4 * p)) | (unsigned)r << 4 * p;
@@ -91,6 +95,10 @@ inline bool line_chain(int n, LineAxis *ax) {
     }
   };
   search(0, m, 0.0);
+  if (!ax->np) {
+    most = 13;
+    search(0, m, 0.0);
+  }
   return ax->np > 0;
 }
 
