@@ -268,8 +268,15 @@ bool has_lines(const qss_ctx *c) { return c->line_use || c->line_pass[0] || c->l
 // the pass along axis i of a plain transform of n fields is a line transform beside
 // a GEMM along the other
 bool use_line_pass(const qss_ctx *c, int i, int n) {
-  return c->line_pass[i] && lines_on(c) &&
+  return c->line_pass[i] && line_fixed(c->line[i]) && lines_on(c) &&
          (c->line[i].n >= kLinePassMin || (i == 1 && n >= kLinePassBatch));
+}
+// both passes of a plain transform of n fields of nw wakes are line transforms
+bool use_line_plain(const qss_ctx *c, int n, int nw) {
+  if (!use_lines(c) || !c->line_plain) return false;
+  if (!line_big(c->line[0])) return true;
+  const bool full = c->ny % 32 == 0 && c->nz % 32 == 0;   // the GEMMs' tiles
+  return n * nw * c->ncell >= (full || use_line_pass(c, 1, n) ? 2 : 1) * kLineBigNodes;
 }
 
 // transforms along z with the corrector's epilogue; store[b] = 0: the result
@@ -377,7 +384,7 @@ int transform_batch(qss_ctx *c, int n, const int *kz, const int *ky,
     qss_set_error("transform batch size");
     return QSS_E_ARG;
   }
-  if (use_lines(c) && c->line_plain)
+  if (use_line_plain(c, n, one_wake ? 1 : c->nw))
     return transform_line(c, n, kz, ky, in, out, alpha, resid, push, pplane, beta, one_wake);
   if (c->fact_use && !c->npc && !c->mixed)
     return transform_fact(c, n, kz, ky, in, out, alpha, resid, push, pplane, beta, one_wake);

@@ -156,8 +156,16 @@ constexpr int kLineDenseY = 128, kLineDenseZ = 256, kLineLooseMin = 192;
 // eight), 256 35.5 / 30.9 (by 313, four); 96 23.9 / 24.1, 64 21.8 / 22.0, 32 20.5 /
 // 20.7; a chain not compiled, 200 24.0 / 28.0 (by 35, eight)
 constexpr int kLinePassMin = 128;
-// ... or, along z, batches of a Guess or Iterate: 24 layers of a 199 x 64 deck 7.22 ms
-// by GEMMs, 6.88 with its six and eight fields' passes along z as lines; a batch of
+// The rows of a chain with a radix above 8 (a factor of 11 or 13 along y) spill
+// registers and lose to a GEMM pass until the planes are many or large: lines from
+// this many nodes of a call on (planes in us, GEMMs / lines: 198^2 three 28.4 / 29.7,
+// six 33.3 / 30.4; 234^2 three 29.1 / 30.3, six 33.2 / 31.2), twice as many where the
+// GEMMs' tiles are full (352^2 two 27.7 / 32.7, three 34.2 / 33.2; 352 x 64 eight 22.4 /
+// 29.3; 416^2 one 28.0 / 32.9, two 36.3 / 33.7) or a line pass along z would stay beside
+// the GEMM (208 x 128 three 22.4, eight 24.6 / 26.2).  Along z such a chain loses nothing.
+constexpr long kLineBigNodes = 168 * 1024;
+// A line pass beside a GEMM pass also takes, along z, batches of a Guess or Iterate: 24
+// layers of a 199 x 64 deck 7.22 ms by GEMMs, 6.88 with its six and eight fields' passes along z as lines; a batch of
 // eight 20.9 us / 19.7 at 33 x 48 (along y, 48 x 33, 20.8 / 21.4)
 constexpr int kLinePassBatch = 6;
 // transforms along z of nbatch planes: out = alpha T_z in (+ beta out), with
@@ -325,9 +333,9 @@ struct qss_ctx {
   // asked for instead
   bool line_off = false;
   bool line_plain = false, line_use = false;   // transforms by themselves; layer steps
-  // the passes of a plain transform (y, z) that are line transforms: a compiled chain
-  // or one from kLineLooseMin on; where only one side has that, a compiled one (from
-  // kLinePassMin on, along z also for batches from kLinePassBatch on), and the other pass is a GEMM
+  // the passes of a plain transform (y, z) that can be line transforms: a compiled
+  // chain or one from kLineLooseMin on; beside a GEMM pass a compiled one (from
+  // kLinePassMin on, along z also for batches from kLinePassBatch on)
   bool line_pass[2] = {};
   LineAxis line[2];                  // y, z
   double *d_linetw[2] = {};
