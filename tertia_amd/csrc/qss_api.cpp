@@ -1334,16 +1334,12 @@ int qss_create(const qss_params *p, int device, uint32_t history_mask, qss_ctx *
     }
   }
   // line transforms (line.hip)
-  c->line_use = p->precision == QSS_PREC_FP64;
   for (int i = 0; i < 2 && p->precision == QSS_PREC_FP64; ++i) {
     LineAxis &ax = c->line[i];
     const bool fast = line_chain(i == 0 ? c->ny : c->nz, &ax);
     ax.Tc = c->d_T[2 * i];
     ax.Ts = c->d_T[2 * i + 1];
-    if (!fast) {
-      c->line_use = c->line_use && ax.n <= (i == 0 ? kLineDenseY : kLineDenseZ);
-      continue;
-    }
+    if (!fast) continue;
     c->line_pass[i] = line_fixed(ax) || ax.n >= kLineLooseMin;
     std::vector<double> tw;
     line_table(ax, tw);
@@ -1355,6 +1351,7 @@ int qss_create(const qss_params *p, int device, uint32_t history_mask, qss_ctx *
       return fail(QSS_E_HIP);
     }
   }
+  c->line_use = p->precision == QSS_PREC_FP64 && line_dense_ok(c->line[0], c->line[1]);
   c->line_plain = c->line_use && c->line_pass[0] && c->line_pass[1];
   if (!c->line_plain)
     for (int i = 0; i < 2; ++i)

@@ -145,12 +145,22 @@ void fact_fused_twiddles(int n, std::vector<double> &tw);
 // fast form (a chain of passes of small radix) or the dense table applied line
 // by line (np = 0).  Transforms by themselves take lines where both axes are
 // fast and of a compile-time length or at least kLineLooseMin (3 planes of 200 x
-// 312 1.14 times the GEMMs' speed, 4 of 100 x 100 0.90); a layer step's Guess and Iterate, whose row kernel does the work of five
-// launches, also with a dense axis: along y up to 128 (a 121 x 97 sweep 1.07 times
-// the GEMMs' speed, 74 x 122 1.12, 129 x 129 0.86), along z up to 256 (64 x 161
-// 1.17)
+// 312 1.14 times the GEMMs' speed when the line was drawn; since radices above 8 were
+// given up where others do, 180^2 would be 1.16 and 100^2 1.02).
 // ---------------------------------------------------------------------------
-constexpr int kLineDenseY = 128, kLineDenseZ = 256, kLineLooseMin = 192;
+constexpr int kLineLooseMin = 192;
+// A layer step's Guess and Iterate, whose row kernel does the work of five launches,
+// run as lines with a dense axis too: along y up to 128 (a 121 x 97 sweep 1.07 times
+// the GEMMs' speed, 74 x 122 1.12), along z as far as the columns' table, read once per
+// strip, does not outgrow that (us a layer, GEMMs / lines: by 64 and 128 along y 177
+// 258 / 238 and 287 / 271, 193 265 / 273 and 293 / 307; by 350 and 512, whose GEMMs are
+// larger, 255 536 / 503 and 582 / 577; by a dense 121, 129 272 / 267, 145 280 / 280, 161
+// 284 / 292).
+constexpr int kLineDenseY = 128, kLineDenseZ = 256;
+inline bool line_dense_ok(const LineAxis &y, const LineAxis &z) {
+  if (!y.np && y.n > kLineDenseY) return false;
+  return z.np || z.n <= (!y.np ? 144 : y.n < 320 ? 180 : kLineDenseZ);
+}
 // A line pass next to a GEMM pass (one side without a chain), planes in us, GEMM only
 // against this: side 512 31.7 / 24.0 (by 121, one plane) and 37.0 / 27.7 (by 121,
 // eight), 256 35.5 / 30.9 (by 313, four); 96 23.9 / 24.1, 64 21.8 / 22.0, 32 20.5 /

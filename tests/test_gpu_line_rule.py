@@ -44,3 +44,28 @@ def test_rows_of_large_radix(oracle_mod, ny, nz, n, lines):
         assert same != lines
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("ny,nz,lines", [
+    (64, 179, True), (64, 181, False), (100, 255, False), (126, 201, False),   # y a chain
+    (320, 255, True), (121, 143, True), (121, 145, False),                     # a long one; dense
+    (129, 97, False)])
+def test_dense_columns_in_layer_steps(oracle_mod, ny, nz, lines):
+    """Layers of a grid whose z side has no chain: lines on one side of the rule, the
+    GEMMs' bits on the other."""
+    from tertia_amd.mesh import Mesh
+    p = small(ny=ny, nz=nz, nslices=4)
+    m, o = Mesh(p, history=("Ex",)), oracle_mod.Oracle(p, history=("Ex",))
+    try:
+        runs = []
+        for _ in range(2):
+            m.MoveAllSplitLayers()
+            runs.append(np.stack([m.history("Ex", s) for s in range(p.nslices)]))
+            m.transform_method = m.transform_method   # the GEMM form
+        o.sweep()
+        ref = np.stack([o.history("Ex", s) for s in range(p.nslices)])
+        assert np.linalg.norm(runs[0] - ref) <= 1e-10 * np.linalg.norm(ref)
+        assert np.array_equal(*runs) != lines
+    finally:
+        m.close()
+        o.close()
