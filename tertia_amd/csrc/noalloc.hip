@@ -18,7 +18,7 @@
 // hundred entries where the dense ones are n^2 cosines, and the passes a fraction of
 // the dense products' work; beside a side without one, from kLinePassMin on.  Dense
 // against lines, us a call: 512 x 512 54.0 / 16.1,
-// 312 x 200 38.0 / 18.2, 100 x 100 22.0 / 15.9, 66 x 52 17.8 / 16.8, 12 x 10 16.6 /
+// 312 x 200 38.0 / 18.2, 100 x 100 22.0 / 15.9, 66 x 66 19.3 / 17.4, 12 x 10 16.6 /
 // 14.2 (a context, whose tables stand ready, keeps dense products for loose chains
 // below 192); what is left is three launches and two passes over the plane.
 //
@@ -152,6 +152,10 @@ extern "C" int qss_transform2d_noalloc(int ny, int nz, int kind_z, int kind_y,
   }
   double *Ty = base, *Tz = base + kPlane, *mid = base + 2 * kPlane;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // a short y side with a factor of 11 or 13: its rows spill registers and take longer
+  // than the dense pass (22 x 22 13.1 / 16.6 us, 52 x 52 17.2 / 17.9, 26 x 64 15.6 / 17.0;
+  // 66 x 66 19.3 / 17.4)
+  if (y.np && line_big(y) && ny < 56) y.np = 0;
   // one side without a chain: the other one's is worth it from kLinePassMin on
   // (121 x 256 30.3 / 18.9 us, 300 x 97 32.2 / 21.9, 200 x 35 23.3 / 20.4; 64 x 35 16.7
   // / 16.8, 26 x 35 16.5 / 19.8)
