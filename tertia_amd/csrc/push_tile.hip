@@ -136,6 +136,33 @@ __device__ inline const FT *field_of(const TileArgs &a) {
 // kCell: events of a cell that its owner lane sums directly: the bytes of one 8-byte
 // list, and past 8 the longest list sets the pace of its wave.
 
+template <int NQ>
+__device__ inline void add_corners(double yp, double zp, const double *w, double (*s)[NQ]) {
+  const double yc = 1. - yp, zc = 1. - zp;
+  const double c[4] = {yc * zc, yp * zc, yc * zp, yp * zp};
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) s[k][q] = __builtin_fma(c[k], w[q], s[k][q]);
+}
+
+// A cell's corner sums onto the window's nodes, one corner after the other with a barrier
+// between: in one corner's turn no two cells share a node.
+template <int NQ>
+__device__ inline void corner_turns(bool on, int cell, const double (*s)[NQ],
+                                    double (*wacc)[NWIN], bool cic) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (k > 0 && !cic) break;
+    if (on) {
+      const int node = cell + (k & 1) + (k >> 1) * W;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) wacc[q][node] += s[k][q];
+    }
+    __syncthreads();
+  }
+}
+
 // Sums of one cell's events over its four nodes, in the order of the events'
 // indices: the order in which they reached the list does not matter.
 template <int N, int NQ>
@@ -152,22 +179,15 @@ __device__ inline void cell_sums(uint2 bytes, int n, const double *ev_y, const d
     for (int q = 0; q < NQ; ++q) w[q] = ev_w[q][ei];
     // NGP: all of it in corner 0
     const double yp = cic ? ev_y[ei] : 0., zp = cic ? ev_z[ei] : 0.;
-    const double yc = 1. - yp, zc = 1. - zp;
-    const double c[4] = {yc * zc, yp * zc, yc * zp, yp * zp};
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) s[k][q] = __builtin_fma(c[k], w[q], s[k][q]);
+    add_corners<NQ>(yp, zp, w, s);
   }
 }
 
 // A lane sums the events of the window cell it owns in this half (cells 0 .. NT - 1
-// or the rest) over the four corners in registers, each event read once, and the
-// four corners are added to the node sums one after the other, a barrier
-// between: in one corner's turn no two cells share a node.  A chunk's events lie in
-// few neighbouring rows, so with the cells in order some waves have all the work
-// and the others none to issue (dealt to the waves in turn: 34.4 us a push at 512^2
-// against 32.0).
+// or the rest) over the four corners in registers, each event read once.  A chunk's
+// events lie in few neighbouring rows, so with the cells in order some waves have all
+// the work and the others none to issue (dealt to the waves in turn: 34.4 us a push at
+// 512^2 against 32.0).
 // Leaves the counts at zero.
 template <int NQ>
 __device__ inline void deposit_cells(int half, int *cnt, const uint2 *list, const double *ev_y,
@@ -187,16 +207,7 @@ __device__ inline void deposit_cells(int half, int *cnt, const uint2 *list, cons
     if (n <= 4) cell_sums<4, NQ>(bytes, n, ev_y, ev_z, ev_w, cic, s);
     else cell_sums<8, NQ>(bytes, n, ev_y, ev_z, ev_w, cic, s);
   }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (k > 0 && !cic) break;
-    if (n) {
-      const int node = cell + (k & 1) + (k >> 1) * W;
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) wacc[q][node] += s[k][q];
-    }
-    __syncthreads();
-  }
+  corner_turns<NQ>(n > 0, cell, s, wacc, cic);
 }
 
 // The float form's round: the owner lanes put the lists in order, then every node
@@ -272,11 +283,21 @@ __device__ inline void deposit_lists(int *cnt, uint2 *list, const double *ev_y, 
 }
 
 // A round with more than kCell events in some cell: the events sorted by cell and
-// index, every node summing the runs of its four corner cells.
-template <int NQ>
+// index.  BY_CELL (the double form): the owner lane sums its cell's run as
+// deposit_cells does its list; else every node sums the runs of its four corner cells,
+// event by event, in the order that deposit_lists keeps.  ev: y, z and the NQ weights by
+// rows; the sorted events take the same memory in pairs, (y, z), (w0, w1), which are
+// read at once.  halves: bit h set where half h of the cells has events.
+// Bound by the chain of a lane's events (their reads' latency; with the chip full, the
+// reads themselves), so the reads are paired, spread over the banks (run_slot) and two
+// events in flight.  A layer's three pushes of 512^2, us: 9 per cell 387 with every chunk
+// sorted, 395 with lists tried first and single reads, 333 like this; 16 811, 889, 612; 25
+// 1318, 1430, 1057.  By nodes (float) 9 354, 362, 363; 16 771, 846, 703; 25 1233, 1369, 1279.
+template <int NQ, bool BY_CELL>
 __device__ inline void deposit_sorted(int cellw, int *keys, int *sorted, short *cstart,
-                                            short *cend, double *ev_y, double *ev_z,
-                                            double (*ev_w)[NT], double (*wacc)[NWIN], bool cic) {
+                                      short *cend, double (*ev)[NT], double (*wacc)[NWIN],
+                                      bool cic, int halves) {
+  typedef double pair __attribute__((ext_vector_type(2)));
   const int t = thread_index();
   for (int i = t; i < NWIN; i += NT) { cstart[i] = 0; cend[i] = 0; }
   const int sk = sort256(cellw < 0 ? kInvalid : cellw << 8 | t, keys);
@@ -284,20 +305,20 @@ __device__ inline void deposit_sorted(int cellw, int *keys, int *sorted, short *
   // the event at sorted position t, moved there in place: gathered before the
   // barrier, stored after it, so the node sums below read events without the
   // sorted[] indirection
-  double gy = 0, gz = 0, gw[NQ];
+  double g[2 + NQ];
   if (sk != kInvalid) {
     const int e = sk & 255;
-    gy = ev_y[e];
-    gz = ev_z[e];
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) gw[q] = ev_w[q][e];
+    for (int q = 0; q < 2 + NQ; ++q) g[q] = ev[q][e];
   }
+  pair *const yz = reinterpret_cast<pair *>(ev[0]), *const w01 = reinterpret_cast<pair *>(ev[2]);
   __syncthreads();
   if (sk != kInvalid) {
-    ev_y[t] = gy;
-    ev_z[t] = gz;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) ev_w[q][t] = gw[q];
+    const int at = qss_tile::run_slot(t);
+    yz[at] = pair{g[0], g[1]};
+    w01[at] = pair{g[2], g[3]};
+    if constexpr (NQ == 4) reinterpret_cast<pair *>(ev[4])[at] = pair{g[4], g[5]};
+    else ev[4][at] = g[4];
     const int c = sk >> 8;
     const int prev = t > 0 ? sorted[t - 1] : kInvalid;
     const int next = t + 1 < NT ? sorted[t + 1] : kInvalid;
@@ -305,6 +326,35 @@ __device__ inline void deposit_sorted(int cellw, int *keys, int *sorted, short *
     if (next == kInvalid || (next >> 8) != c) cend[c] = (short)(t + 1);
   }
   __syncthreads();
+  const auto event = [&](int e, double &y, double &z, double *w) {
+    const int at = qss_tile::run_slot(e);
+    const pair p = yz[at], a = w01[at];
+    y = p.x; z = p.y;
+    w[0] = a.x; w[1] = a.y;
+    if constexpr (NQ == 4) {
+      const pair b = reinterpret_cast<const pair *>(ev[4])[at];
+      w[2] = b.x; w[3] = b.y;
+    } else {
+      w[2] = ev[4][at];
+    }
+  };
+  if constexpr (BY_CELL) {
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+      if (!(halves >> half & 1)) continue;
+      const int cell = t + NT * half;
+      const int e0 = cell < NWIN ? cstart[cell] : 0, e1 = cell < NWIN ? cend[cell] : 0;
+      double s[4][NQ] = {};
+#pragma unroll 2
+      for (int e = e0; e < e1; ++e) {
+        double y, z, w[4];
+        event(e, y, z, w);
+        add_corners<NQ>(cic ? y : 0., cic ? z : 0., w, s);   // NGP: all of it in corner 0
+      }
+      corner_turns<NQ>(e1 > e0, cell, s, wacc, cic);
+    }
+    return;
+  }
   for (int n = t; n < NWIN; n += NT) {
     double acc[NQ];
 #pragma unroll
@@ -318,17 +368,14 @@ __device__ inline void deposit_sorted(int cellw, int *keys, int *sorted, short *
       if (cj < 0 || ck < 0) continue;
       const int cw = ck * W + cj;
       const int e1 = cend[cw];
+#pragma unroll 2
       for (int e = cstart[cw]; e < e1; ++e) {
-        if (cic) {
-          const double ayp = ev_y[e], ayc = 1. - ayp, azp = ev_z[e], azc = 1. - azp;
-          const double wy = (cn & 1) ? ayp : ayc;
-          const double wz = (cn >> 1) ? azp : azc;
+        double y, z, w[4];
+        event(e, y, z, w);
+        const double wy = (cn & 1) ? y : 1. - y;
+        const double wz = (cn >> 1) ? z : 1. - z;
 #pragma unroll
-          for (int q = 0; q < NQ; ++q) acc[q] += ev_w[q][e] * wy * wz;
-        } else {
-#pragma unroll
-          for (int q = 0; q < NQ; ++q) acc[q] += ev_w[q][e];
-        }
+        for (int q = 0; q < NQ; ++q) acc[q] += cic ? w[q] * wy * wz : w[q];
       }
     }
 #pragma unroll
@@ -370,7 +417,9 @@ void k_push_tile(TileArgs a0) {
   // cycles per wave and chunk, a third of the LDS time)
   __shared__ pair_t<FT> Fw[3][NF];
   constexpr int NQ = RHO ? 4 : 3;
-  __shared__ double ev_y[NT], ev_z[NT], ev_w[NQ][NT];
+  __shared__ __attribute__((aligned(16))) double ev[2 + NQ][NT];   // y, z, weights
+  double *const ev_y = ev[0], *const ev_z = ev[1];
+  double(*const ev_w)[NT] = ev + 2;
   __shared__ double wacc[NQ][NWIN];   // the window's node sums
   // the round's events of each cell, or the sort's arrays in a crowded round
   __shared__ union {
@@ -602,8 +651,8 @@ void k_push_tile(TileArgs a0) {
       if (t < FL_N) flag_sh[par][t] = 0;   // last read a barrier ago
       if (crowded) {
         __syncthreads();   // the lists give way to the sort
-        deposit_sorted<NQ>(cellw, sh.sort.keys, sh.sort.sorted, sh.sort.cstart, sh.sort.cend, ev_y,
-                           ev_z, ev_w, wacc, cic);
+        deposit_sorted<NQ, sizeof(R) == 8>(cellw, sh.sort.keys, sh.sort.sorted, sh.sort.cstart,
+                                           sh.sort.cend, ev, wacc, cic, half0 | half1 << 1);
         __syncthreads();
         for (int i = t; i < NWIN; i += NT) sh.cell.cnt[i] = 0;
         __syncthreads();

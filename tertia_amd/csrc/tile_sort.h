@@ -84,6 +84,11 @@ __device__ inline int sort256(int key, int *sh) {
   return bitonic_sort<256>(key, sh, thread_index());
 }
 
+// Where the event at sorted position i lies.  Neighbouring lanes walk the runs of
+// neighbouring cells, and runs of 16 events put them 16 apart, on two of the banks:
+// with the row of 16 mixed into the place they are on different ones.
+__device__ inline int run_slot(int i) { return i ^ i >> 4; }
+
 // Events of a cell that one lane sums: the bytes of one 8-byte list (indices of the
 // round's 256 events), put in the order of the indices by networks of 4 or 8.
 constexpr int kCell = 8;
