@@ -287,16 +287,18 @@ __device__ inline void deposit_lists(int *cnt, uint2 *list, const double *ev_y, 
 // deposit_cells does its list; else every node sums the runs of its four corner cells,
 // event by event, in the order that deposit_lists keeps.  ev: y, z and the NQ weights by
 // rows; the sorted events take the same memory in pairs, (y, z), (w0, w1), which are
-// read at once.  halves: bit h set where half h of the cells has events.
+// read at once.  halves: bit h set where half h of the cells has events.  *still is set
+// where a cell is crowded: the next round is then sorted without trying the lists (a
+// per cent of a push).  Both ways give a node the same sums, bit by bit.
 // Bound by the chain of a lane's events (their reads' latency; with the chip full, the
 // reads themselves), so the reads are paired, spread over the banks (run_slot) and two
 // events in flight.  A layer's three pushes of 512^2, us: 9 per cell 387 with every chunk
-// sorted, 395 with lists tried first and single reads, 333 like this; 16 811, 889, 612; 25
-// 1318, 1430, 1057.  By nodes (float) 9 354, 362, 363; 16 771, 846, 703; 25 1233, 1369, 1279.
+// sorted, 395 with lists tried first and single reads, 333 like this; 16 811, 889, 605; 25
+// 1318, 1430, 1040.  By nodes (float) 9 357, 362, 365; 16 772, 846, 708; 25 1239, 1369, 1298.
 template <int NQ, bool BY_CELL>
 __device__ inline void deposit_sorted(int cellw, int *keys, int *sorted, short *cstart,
                                       short *cend, double (*ev)[NT], double (*wacc)[NWIN],
-                                      bool cic, int halves) {
+                                      bool cic, int halves, int *still) {
   typedef double pair __attribute__((ext_vector_type(2)));
   const int t = thread_index();
   for (int i = t; i < NWIN; i += NT) { cstart[i] = 0; cend[i] = 0; }
@@ -324,6 +326,7 @@ __device__ inline void deposit_sorted(int cellw, int *keys, int *sorted, short *
     const int next = t + 1 < NT ? sorted[t + 1] : kInvalid;
     if (t == 0 || (prev >> 8) != c) cstart[c] = (short)t;
     if (next == kInvalid || (next >> 8) != c) cend[c] = (short)(t + 1);
+    if (t + kCell < NT && sorted[t + kCell] >> 8 == c) *still = 1;   // more than kCell of them
   }
   __syncthreads();
   const auto event = [&](int e, double &y, double &z, double *w) {
@@ -477,6 +480,7 @@ void k_push_tile(TileArgs a0) {
   if (t < 9) dir_total[t] = 0;
   if (t < 2 * FL_N) flag_sh[t / FL_N][t % FL_N] = 0;
   int par = 0;
+  int sorting = 0;   // the round before was crowded
   for (int i = t; i < NWIN; i += NT) {
     sh.cell.cnt[i] = 0;
 #pragma unroll
@@ -634,9 +638,11 @@ void k_push_tile(TileArgs a0) {
           ev_w[1][t] = (double)(djy * part_step);
           ev_w[2][t] = (double)(djz * part_step);
           if constexpr (RHO) ev_w[3][t] = (double)(drho * part_step);
-          const int r = atomicAdd(&sh.cell.cnt[cellw], 1);
-          if (r < kCell) reinterpret_cast<uint8_t *>(&sh.cell.list[cellw])[r] = (uint8_t)t;
-          else flag_sh[par][FL_CROWDED] = 1;
+          if (!sorting) {
+            const int r = atomicAdd(&sh.cell.cnt[cellw], 1);
+            if (r < kCell) reinterpret_cast<uint8_t *>(&sh.cell.list[cellw])[r] = (uint8_t)t;
+            else flag_sh[par][FL_CROWDED] = 1;
+          }
           flag_sh[par][cellw < NT ? FL_HALF0 : FL_HALF1] = 1;
         } else {
           status |= (ST_FAR);
@@ -645,17 +651,22 @@ void k_push_tile(TileArgs a0) {
       if (active && partdx > 0.) flag_sh[par][FL_MORE] = 1;
       __syncthreads();
       const int *fl = flag_sh[par];
-      const bool more = fl[FL_MORE], crowded = fl[FL_CROWDED];
+      const bool more = fl[FL_MORE], crowded = sorting || fl[FL_CROWDED];
       const bool half0 = fl[FL_HALF0], half1 = fl[FL_HALF1];
       par ^= 1;
       if (t < FL_N) flag_sh[par][t] = 0;   // last read a barrier ago
       if (crowded) {
-        __syncthreads();   // the lists give way to the sort
+        if (!sorting) __syncthreads();   // the lists give way to the sort
         deposit_sorted<NQ, sizeof(R) == 8>(cellw, sh.sort.keys, sh.sort.sorted, sh.sort.cstart,
-                                           sh.sort.cend, ev, wacc, cic, half0 | half1 << 1);
+                                           sh.sort.cend, ev, wacc, cic, half0 | half1 << 1,
+                                           &flag_sh[par][FL_CROWDED]);
         __syncthreads();
-        for (int i = t; i < NWIN; i += NT) sh.cell.cnt[i] = 0;
-        __syncthreads();
+        // crowded still: the next round is sorted without trying the lists
+        sorting = __builtin_amdgcn_readfirstlane(flag_sh[par][FL_CROWDED]);
+        if (!sorting) {
+          for (int i = t; i < NWIN; i += NT) sh.cell.cnt[i] = 0;
+          __syncthreads();
+        }
       } else if constexpr (sizeof(R) == 4) {
         deposit_lists<NQ>(sh.cell.cnt, sh.cell.list, ev_y, ev_z, ev_w, wacc, cic);
       } else {
