@@ -2232,15 +2232,20 @@ int qss_autotune(qss_ctx *c, int reps, float *table_ms) {
       }
       c->ffv[pass][b] = bestv;
     }
-  // work-groups per tile of the push.  Mixed modes: by the number of tiles, since the
-  // split sets the order of the deposit's sums, whose last bits flip roundings of the
-  // float fields (1e-8 of a field after a sweep); the lines lie where timing put them
-  // (4 up to 169 tiles, 2 from 195 to 512, 1 from 529; 256 tiles 2 in three contexts of
-  // four).  No more parts than a tile has chunks of 256 particles.
+  // work-groups per tile of the push.  Mixed modes: by the number of tiles and of a
+  // tile's chunks of 256 particles, since the split sets the order of the deposit's sums,
+  // whose last bits flip roundings of the float fields (1e-8 of a field after a sweep).
+  // The lines lie where timing put them: with four chunks (4 particles per cell) 4 parts
+  // up to 169 tiles, 2 from 195 to 512 (256 tiles: 2 in three contexts of four), 1 from 529;
+  // longer tiles are worth more parts (a layer's pushes of 256 tiles in us, 2 parts / 4: 16
+  // per cell 313 / 239; 400 tiles: 8 per cell 165 / 162, 16 428 / 398).
   if (rc == QSS_OK && c->tiled && c->mixed) {
-    const long nt = (long)c->ntj * c->ntk * c->nw, per_tile = c->np_cap / (c->ntj * c->ntk);
-    c->nsplit = nt > 512 ? 1 : nt > 180 ? 2 : 4;
-    while (c->nsplit > 1 && (c->nsplit - 1) * 256 >= per_tile) c->nsplit /= 2;
+    const long tiles = (long)c->ntj * c->ntk, nt = tiles * c->nw;
+    const long chunks = (c->np_cap / tiles + 255) / 256;
+    c->nsplit = nt <= 180 ? 4 : nt <= 512 ? 2 : 1;
+    if (nt > 180 && nt < 1024 && chunks > 4)
+      c->nsplit = nt <= 300 || chunks >= 16 ? 4 : 2;
+    while (c->nsplit > 1 && c->nsplit - 1 >= chunks) c->nsplit /= 2;
   }
   // FP64: one predictor pass (state unchanged) plus the window combine into scratch
   // planes, per candidate
