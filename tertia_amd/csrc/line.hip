@@ -6,7 +6,7 @@
 //   w_k = 2 V_k e^{-i pi k/N},  y_2k = Re w_k,  y_{N-1-2k} = -Im w_k
 // (a DST-IV is the DCT-IV of the reversed line with its odd outputs negated:
 // swap the two inputs, flip the sign of Im).  The DFT is a Stockham chain of
-// passes of radix R_0, R_1, ... (1 to 13, at most 8 where m allows): pass p
+// two to four passes of radix R_0, R_1, ... (1 to 13, at most 8 where m allows): pass p
 // takes elements b + r m/R_p, multiplies them by a table T_p, transforms R_p
 // points in registers and leaves them in the order of the next pass, so there is
 // no bit reversal.  The outer twiddles cost nothing of their own: with
@@ -107,15 +107,15 @@ struct Loose {
   }
 
 // pass tables T_1, T_2, ...: fetched early with the other loads, put into LDS
-// once the first pass has its inputs
+// once the first pass has its inputs.  m is at most the work-group's threads, so a
+// thread holds an entry per table.
 template <class C>
 struct Tables {
-  double x0, y0, x1, y1, x2, y2, x3, y3;
+  double x0, y0, x1, y1, x2, y2;
   __device__ explicit Tables(const LineAxis &ax) {
     fetch(ax, 0, x0, y0);
     fetch(ax, 1, x1, y1);
     fetch(ax, 2, x2, y2);
-    fetch(ax, 3, x3, y3);
   }
   static __device__ void fetch(const LineAxis &ax, int q, double &x, double &y) {
     const int i = threadIdx.x + q * blockDim.x;
@@ -132,10 +132,9 @@ struct Tables {
     put(ax, tw, 0, x0, y0);
     put(ax, tw, 1, x1, y1);
     put(ax, tw, 2, x2, y2);
-    put(ax, tw, 3, x3, y3);
   }
 };
-static_assert(kLinePasses == 5, "Tables holds four entries per thread");
+static_assert(kLinePasses == 4 && kPer == 2, "Tables holds three entries per thread");
 
 // exchange slot of element i of a line: columns lie side by side; a row has a
 // free slot after every eight, which keeps the first pass's writes (R consecutive

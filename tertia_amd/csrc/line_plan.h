@@ -13,7 +13,7 @@
 #define QSS_LP
 #endif
 
-constexpr int kLinePasses = 5;   // at most
+constexpr int kLinePasses = 4;   // at most
 constexpr int kLineT = 32;       // threads per line at most; a pass has at most two
                                  // butterflies per thread
 

@@ -89,11 +89,6 @@ __device__ inline void cell_jk(int32_t c, int ny, uint64_t magic, int &j, int &k
   j = c - k * ny;
 }
 
-__device__ inline int wrapi(int a, int n) {
-  a %= n;
-  return a < 0 ? a + n : a;
-}
-
 // the arguments of wake w of a batch: every per-wake array is stored
 // wake-major with a fixed stride
 __host__ __device__ inline TileArgs wake_view(const TileArgs &a0, int w) {
@@ -397,14 +392,16 @@ __device__ inline void deposit_sorted(int cellw, int *keys, int *sorted, short *
 // chunks p, p + nsplit, ...): each part writes its own window, direction
 // counts and ranks, and the combine / reorder kernels visit the parts in
 // order, so results are a pure function of the input and nsplit.
-// 128 VGPRs and 40 KB of LDS at most (RHO: 46 KB): four waves per SIMD, so all the
-// tiles of a 512^2 grid (4 work-groups per CU) are resident at once.  The bound is
+// A layer step's forms (no RHO) hold at most 128 VGPRs and 40 KB of LDS: four waves per
+// SIMD, so all the tiles of a 512^2 grid (4 work-groups per CU) are resident at once;
+// with the density 132 VGPRs (FULL: 144) and 46 KB, three.  The bound is
 // instruction issue and latency, not memory: at 512^2 and 4 per cell 58 MB in and
 // 15 MB out (full: 61 MB) in 31.8 us (full: 38.0), half of the wave cycles waiting at
 // barriers and for LDS.  What spilled registers here cost most: with uniform FP64
 // products made on the host, the sort's lane masks not kept over the loop and
-// machine LICM off (it keeps FP64 literals in registers) nothing spills: 37 us on
-// average of a step's three pushes at that point, against 42.6 with 104 scalar registers spilled.
+// machine LICM off (it keeps FP64 literals in registers) no vector register spills and
+// only the FULL forms keep scalar ones in vector lanes (30, float 12): 37 us on average
+// of a step's three pushes at that point, against 42.6 with 104 scalar registers spilled.
 // FULL: the pushed particles are staged for the reorder.
 // RHO = false: the deposit sums Jx, Jy, Jz only and the windows' density
 // component stays 0 (inside a layer step nothing reads the deposited density:
@@ -982,7 +979,7 @@ __global__ void k_uniform_tile_start(int32_t *ts, int nt, int nw, int per_tile) 
 
 inline dim3 grid1(long n) { return dim3((unsigned)((n + NT - 1) / NT)); }
 
-TileArgs make_args(qss_ctx *c, int full) {
+TileArgs make_args(qss_ctx *c) {
   TileArgs a;
   const int b = c->cur;
   a.y = c->py_[b]; a.z = c->pz_[b]; a.px = c->ppx[b]; a.py = c->ppy[b]; a.pz = c->ppz[b];
@@ -1026,9 +1023,9 @@ hipError_t launch_push_tile(qss_ctx *c, int full, bool rho, hipEvent_t ev0, hipE
   auto fn = c->mixed ? (full ? pick(0.0f, yes) : pick(0.0f, no))
                      : (full ? pick(0.0, yes) : pick(0.0, no));
   if (ev0 || ev1)
-    hipExtLaunchKernelGGL(fn, grid, block, 0, c->stream, ev0, ev1, 0, make_args(c, full));
+    hipExtLaunchKernelGGL(fn, grid, block, 0, c->stream, ev0, ev1, 0, make_args(c));
   else
-    hipLaunchKernelGGL(fn, grid, block, 0, c->stream, make_args(c, full));
+    hipLaunchKernelGGL(fn, grid, block, 0, c->stream, make_args(c));
   return hipGetLastError();
 }
 
@@ -1055,7 +1052,7 @@ hipError_t launch_combine(qss_ctx *c, bool rho, double *const *out, bool scan) {
 
 hipError_t launch_tile_reorder(qss_ctx *c) {
   const int nb = c->cur ^ 1;
-  hipLaunchKernelGGL(k_permute, grid1(c->np * c->nw), dim3(NT), 0, c->stream, make_args(c, 1),
+  hipLaunchKernelGGL(k_permute, grid1(c->np * c->nw), dim3(NT), 0, c->stream, make_args(c),
                      c->goff, c->np, c->nw, c->py_[nb], c->pz_[nb], c->ppx[nb], c->ppy[nb],
                      c->ppz[nb], c->pcell[nb], c->pid[nb]);
   return hipGetLastError();
