@@ -56,7 +56,7 @@ extern "C" {
  * FP64, deposits are summed in FP64, and the spectral state, the transform
  * operands/results in HBM and the corrector residual stay FP64.  Mixed modes
  * need ny, nz multiples of 16 and fix_subcycle = 0 (the tiled particle path). */
-#define QSS_PREC_FP64         0   /* FP64 push, FP64 MFMA transforms          */
+#define QSS_PREC_FP64         0   /* FP64 push and transforms                  */
 #define QSS_PREC_MIXED32      1   /* transforms on FP32 MFMA (fp32 operands)  */
 #define QSS_PREC_MIXED_BF16X3 2   /* transforms on BF16 MFMA, operands split
                                      into 2 bf16 pieces, 3 products          */
@@ -210,8 +210,9 @@ int  qss_transform2d_batched(qss_ctx *c, int n, const int *kind_z,
 
 /* ---- transform tile shapes --------------------------------------------- */
 /* The reference plans its transforms with FFTW_ESTIMATE
- * (movefieldshydrolinlayersplit.cpp:389-427).  Here the transform is a
- * batched MFMA GEMM compiled for several tile shapes; qss_autotune times
+ * (movefieldshydrolinlayersplit.cpp:389-427).  Here the GEMM forms of the
+ * transform (all modes but FP64 where lines run, see qss_transform_in_use)
+ * are compiled for several tile shapes; qss_autotune times
  * every shape on this context's buffers for every launch shape the sweep
  * uses (1..8 fields, both passes, the 6- and 8-field inverse passes with
  * their corrector epilogue) and keeps the fastest.  It also picks the
@@ -393,7 +394,7 @@ int  qss_set_fact_choice(qss_ctx *c, const int *chosen);
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): qss_transform2d without a context.  out = scale *
  * T_kind_z . in . T_kind_y for one Ny x Nz plane (y fastest) in device
- * memory, FP64 MFMA, enqueued on `stream` (a hipStream_t of the current
+ * memory, in FP64, enqueued on `stream` (a hipStream_t of the current
  * device; NULL = its null stream): no allocation and no synchronisation.
  * The transform tables and the intermediate plane live in a fixed per-device
  * scratch array of 3 x 512 x 512 doubles (6 MiB, held by each device the

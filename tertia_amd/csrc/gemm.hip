@@ -785,7 +785,8 @@ bool gemm_same_order(int prec, int variant, int M, int N, int K, int planes, boo
   int bk, ks;
   if (prec == QSS_PREC_MIXED32) {
     bk = 16;
-    if (M % 64 == 0 && N % 64 == 0) ks = fill > 0.75 || (fill == 0.75 && zpass && t64 > 256) ? 2 : 4;
+    if (M % 64 == 0 && N % 64 == 0)
+      ks = fill > 0.75 || (fill == 0.75 && zpass && t64 > 256) ? 2 : 4;
     else ks = edge && t64 > 150 && (zpass || fill > 0.6) ? 2 : 4;
   } else {
     const bool three = prec == QSS_PREC_MIXED_BF16X6;

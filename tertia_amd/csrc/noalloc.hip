@@ -17,9 +17,9 @@
 // goes through the line transforms (line.hip): a chain's tables are a few
 // hundred entries where the dense ones are n^2 cosines, and the passes a fraction of
 // the dense products' work; beside a side without one, from kLinePassMin on.  Dense
-// against lines, us a call: 512 x 512 54.0 / 16.1,
-// 312 x 200 38.0 / 18.2, 100 x 100 22.0 / 15.9, 66 x 66 19.3 / 17.4, 12 x 10 16.6 /
-// 14.2 (a context, whose tables stand ready, keeps dense products for loose chains
+// against lines, us a call: 512 x 512 54.5 / 16.5, 312 x 200 38.5 / 15.7, 240 x 240 35.9 /
+// 15.5, 100 x 100 22.4 / 14.3, 66 x 66 19.0 / 17.0, 12 x 10 14.3 / 12.3 (a context,
+// whose tables stand ready, keeps dense products for loose chains
 // below 192); what is left is three launches and two passes over the plane.
 //
 // The array's name is not a device address in host code: its per-device

@@ -150,12 +150,13 @@ void fact_fused_twiddles(int n, std::vector<double> &tw);
 // ---------------------------------------------------------------------------
 constexpr int kLineLooseMin = 192;
 // A layer step's Guess and Iterate, whose row kernel does the work of five launches,
-// run as lines with a dense axis too: along y up to 128 (a 121 x 97 sweep 1.07 times
-// the GEMMs' speed, 74 x 122 1.12), along z as far as the columns' table, read once per
-// strip, does not outgrow that (us a layer, GEMMs / lines: by 64 and 128 along y 177
-// 258 / 238 and 287 / 271, 193 265 / 273 and 293 / 307; by 350 and 512, whose GEMMs are
-// larger, 255 536 / 503 and 582 / 577; by a dense 121, 129 272 / 267, 145 280 / 280, 161
-// 284 / 292).
+// run as lines with a dense axis too (us a layer, GEMMs / lines).  Along y up to 128: 127
+// by 64, 128 and 312 258 / 206, 285 / 219 and 375 / 358; 129 246 / 218, 259 / 239 and 361 /
+// 389, 199 263 / 287, 276 / 313 and 424 / 550 (between, by a z side of few passes lines
+// would still gain).  Along z as far as the columns' table, read once per strip, does
+// not outgrow that: by 64 and 128 along y 177 258 / 238 and 287 / 271, 193 265 / 273 and
+// 293 / 307; by 350 and 512, whose GEMMs are larger, 255 536 / 503 and 582 / 577; by a
+// dense 121, 129 272 / 267, 145 280 / 280, 161 284 / 292.
 constexpr int kLineDenseY = 128, kLineDenseZ = 256;
 inline bool line_dense_ok(const LineAxis &y, const LineAxis &z) {
   if (!y.np && y.n > kLineDenseY) return false;
@@ -175,8 +176,8 @@ constexpr int kLinePassMin = 128;
 // the GEMM (208 x 128 three 22.4, eight 24.6 / 26.2).  Along z such a chain loses nothing.
 constexpr long kLineBigNodes = 168 * 1024;
 // A line pass beside a GEMM pass also takes, along z, batches of a Guess or Iterate: 24
-// layers of a 199 x 64 deck 7.22 ms by GEMMs, 6.88 with its six and eight fields' passes along z as lines; a batch of
-// eight 20.9 us / 19.7 at 33 x 48 (along y, 48 x 33, 20.8 / 21.4)
+// layers of a 199 x 64 deck 7.22 ms by GEMMs, 6.88 with its six and eight fields' passes
+// along z as lines; a batch of eight 20.9 us / 19.7 at 33 x 48 (along y, 48 x 33, 20.8 / 21.4)
 constexpr int kLinePassBatch = 6;
 // transforms along z of nbatch planes: out = alpha T_z in (+ beta out), with
 // the corrector epilogue
