@@ -762,17 +762,20 @@ int gemm_num_variants(int prec) { return table(prec).n; }
 // same bits, others differ in the last bits of a float, 1e-8 of a field after a
 // sweep.  Which of two shapes is the faster often turns on a per cent that changes
 // from one timing to the next (y pass of three 512^2 planes, split in three: 64 deep
-// by two waves 14.3 us, 32 deep 14.3 us, 17 and 11 of 28 contexts), so the tuner picks
-// the shape and this rule the order: what a tuned sweep returns does not depend on a
-// clock.  The rule is the order that was fastest most often on 95 grids of 48 to 512
-// (sides multiples of 16; passes of 2, 3, 6 and 8 planes), by
+// by two waves 14.3 us, 32 deep 14.3 us, the first in 17 of 28 contexts on an idle card
+// and in 5 of 36 between sweeps), so the tuner picks the shape and this rule the order:
+// what a tuned sweep returns does not depend on a clock.  The rule is the order that
+// was fastest most often between sweeps on 95 grids of 48 to 512 (sides multiples of 16;
+// passes of 2, 3, 6 and 8 planes), by
 //   t32, t64  work-groups of 32- and 64-sided tiles; fill: the share of the CUs that
 //             rounds of the latter use
 //   edge      tiles that are not full: every shape then checks its bounds
 // Split forms: a launch that leaves CUs idle splits its slabs over waves (256^2, 3
 // planes: 7.0 us against 7.8), with 4 of them where the longer slab costs no padding
 // (48 x 256: 9.2 against 9.6); one that fills them is faster with shallow slabs and no
-// split (512^2, 8 planes: 23.1 against 25.8), and a K that is an odd multiple of 64 has
+// split (512^2, 8 planes: 23.1 against 25.8), unless K is long enough for 64-sided tiles of
+// one round (512 x 256, y pass of 8: 14.4 against 14.8) or the corrector's epilogue leaves
+// time (256^2, z pass of 6: 11.1 against 11.2); and a K that is an odd multiple of 64 has
 // 32 deep slabs alone without checks (320^2: 7.9 against 14.6).  Float: four waves per
 // 32-sided tile unless 64-sided ones fill their rounds (320^2, 8 planes: 15.9 against
 // 19.6 us).
@@ -801,10 +804,10 @@ bool gemm_same_order(int prec, int variant, int M, int N, int K, int planes, boo
       }
     } else if (K % 128) {
       bk = 32; ks = 1;
-    } else if (t32 <= 256) {
-      const bool deep = three || K > 128;
-      bk = deep ? 64 : 32; ks = deep ? 2 : 1;
-    } else if (K >= 384 && t64 <= (three ? 256 : 128)) {
+    } else if (t32 <= 256 || (zpass && planes >= 6 && K >= 256 &&
+                              up(M, 64) * up(N, 32) * planes <= 256)) {
+      bk = 64; ks = 2;
+    } else if (K >= 384 && (t64 <= 128 || (three && t64 <= 256 && (zpass || fill > 0.8)))) {
       bk = 64; ks = 2;
     } else {
       bk = !three && K >= 384 && (zpass || fill > 0.8) ? 64 : 32; ks = 1;
